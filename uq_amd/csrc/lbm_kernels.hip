@@ -34,10 +34,10 @@
 
 #include "lbm_device.hpp"
 #include "lbm_launch.hpp"
+#include "lbm_stencil.hpp"
 
 namespace uqlbm {
 
-constexpr int kH = 3;                          // stencil halo (WENO5 reach)
 constexpr int kNT = 256;                       // threads of the pointwise blocks
 constexpr int kNDF = 24;                       // dF planes: f and h of directions 1..12
 
@@ -50,42 +50,9 @@ enum : unsigned {
   kMetaClampY = 32u,
 };
 
-__constant__ int c_lat_x[13] = {0, 1, 0, -1, 0, 1, -1, -1, 1, 2, 0, -2, 0};
-__constant__ int c_lat_y[13] = {0, 0, 1, 0, -1, 1, 1, -1, -1, 0, 2, 0, -2};
-__constant__ int c_mir_ns[13] = {0, 1, 4, 3, 2, 8, 7, 6, 5, 9, 12, 11, 10};
-__constant__ int c_mir_ew[13] = {0, 3, 2, 1, 4, 6, 5, 8, 7, 11, 10, 9, 12};
-
 template <typename T>
 __device__ __forceinline__ T* plane(void* base, long long plane_elems, int k) {
   return reinterpret_cast<T*>(base) + plane_elems * (long long)k;
-}
-
-// Reference index() along one axis (cpuLBM.cpp:1033-1113) for one position,
-// then a clamp into the grid for positions no stencil reaches.
-__device__ __forceinline__ int map_axis(int X, int n, int periodic, int mir_lo, int mir_hi, unsigned& mir,
-                                        unsigned& clamped) {
-  mir = 0;
-  clamped = 0;
-  if (X < 0) {
-    if (periodic) X += n;
-    else if (mir_lo) { X = -X - 1; mir = 1; }
-    else { X = 0; clamped = 1; }
-  } else if (X > n - 1) {
-    if (periodic) X -= n;
-    else if (mir_hi) { X = 2 * n - X - 1; mir = 1; }
-    else { X = n - 1; clamped = 1; }
-  }
-  return X < 0 ? 0 : (X > n - 1 ? n - 1 : X);
-}
-
-// Grid-stride tile loop with an XCD-aware order: gfx950 hands consecutive
-// workgroups to its 8 XCDs in turn, so block b is renumbered so that each
-// XCD walks a contiguous run of tiles (neighbouring tiles share halos and
-// that XCD's L2).
-__device__ __forceinline__ int first_tile() {
-  const int G = gridDim.x, b = blockIdx.x;
-  if (G % 8 != 0) return b;
-  return (b % 8) * (G / 8) + b / 8;
 }
 
 template <int... Is>
@@ -96,14 +63,6 @@ template <int... Is>
 struct MakeSeq<0, Is...> {
   using type = Seq<Is...>;
 };
-
-// `step` counts the steps of the current launch sequence from 1; the global
-// step index of an instance is in.step_base + step. A failure flagged during
-// step s freezes the instance for steps > s only, so this test gives the
-// same answer to every thread of a launch.
-__device__ __forceinline__ bool frozen_by_failure(const InstDev& in, int step) {
-  return *in.fail < in.step_base + step;
-}
 
 __device__ __forceinline__ void flag_failure(const InstDev& in, int step, double rho, double sumfeq, double tol) {
   // reference check |sum feq - rho| > 1e-6 (cpuLBM.cpp:825-843); a
@@ -119,23 +78,6 @@ __device__ __forceinline__ void flag_failure(const InstDev& in, int step, double
 template <typename TE>
 __device__ __forceinline__ double eq_check_tol(double sum_abs) {
   return std::is_same<TE, double>::value ? 1e-6 : 1e-6 + 16.0 * 5.96e-8 * sum_abs;
-}
-
-// Global-memory pointers: loads and stores through them are global, not
-// flat, operations (the pointers read out of the instance table are
-// generic), so they count on the vector-memory counter only: a flat access
-// also counts on the LDS/scalar counter, and every wait for a scalar load
-// then waits for it too.
-template <typename T>
-using gptr = __attribute__((address_space(1))) T*;
-
-template <typename T>
-__device__ __forceinline__ gptr<T> as_global(T* p) {
-  return (gptr<T>)p;
-}
-template <typename T>
-__device__ __forceinline__ gptr<T> as_global(gptr<T> p) {
-  return p;
 }
 
 // ---------------------------------------------------------------------------
@@ -348,16 +290,6 @@ __device__ __forceinline__ PointCell point_cell(const InstDev& in, const TileRef
   c.active = x < in.nx && y < in.ny;
   c.o = c.active ? (long long)y * in.pitch + x : 0;
   return c;
-}
-
-// Whether the pointwise kernel instantiated for equilibrium type TE takes
-// instance `in`: FP32 storage picks the equilibrium precision per instance
-// (InstDev::eq32), and a launch group with both kinds launches each
-// pointwise kernel once per kind.
-template <typename TS, typename TE>
-__device__ __forceinline__ bool eq_kernel_for(const InstDev& in) {
-  if constexpr (sizeof(TS) == 4) return (in.eq32 != 0) == (sizeof(TE) == 4);
-  else return true;
 }
 
 // ---------------------------------------------------------------------------
@@ -849,8 +781,6 @@ struct FluxStage {
 
 typedef __attribute__((address_space(1))) void global_void;
 typedef __attribute__((address_space(3))) void lds_void;
-constexpr int kWaitVmem = 0x0F70;  // s_waitcnt vmcnt(0): this wave's loads (also those into LDS) done
-
 // Issue the loads of direction I's f, h over the region into B, without
 // waiting for them: each wave takes every (NT/64)-th group of CH positions;
 // the first LPP/2 lanes of a position load the f value of the
@@ -952,36 +882,6 @@ __device__ __forceinline__ void store_slots(StageBuf<Sh, TS>& B, const SlotVals<
     const int kind = L.meta[j] >> 8;
     if (kind == 3 || (kind == 1 && !ex) || (kind == 2 && !ey)) continue;
     B.v[L.lds[j]] = FH<TS>{V.f[j], V.h[j]};
-  }
-}
-
-// Reference stencil solid handling along one line (cpuLBM.cpp:1242-1322):
-// the first solid/fluid transition's solid point becomes 2 V(m1) - V(m2) of
-// the two nearest fluid points, and the point beyond it the same value. The
-// addressing equivalence with the reference is checked on the host per
-// geometry (lbm_runtime.hip, validate_geometry).
-// (The transition is located in the unrolled loop and the line updated in
-// the same unrolled iteration, so every index is a constant and the stencil
-// stays in registers.)
-template <int L, typename TC>
-__device__ __forceinline__ void extrapolate(const int* sld, const TC* V, TC* S) {
-#pragma clang fp contract(off)
-  bool found = false;
-#pragma unroll
-  for (int j = 0; j < L - 1; j++) {
-    const int d = sld[j] - sld[j + 1];
-    if (!found && d != 0) {
-      found = true;
-      if (d > 0) {  // solid point j, fluid beyond it at j+1, j+2
-        const TC e = TC(2) * V[j + 1 < L ? j + 1 : L - 1] - V[j + 2 < L ? j + 2 : L - 1];
-        S[j] = e;
-        if (j - 1 >= 0) S[j - 1] = e;
-      } else {      // solid point j+1, fluid before it at j, j-1
-        const TC e = TC(2) * V[j] - V[j - 1 >= 0 ? j - 1 : 0];
-        S[j + 1] = e;
-        if (j + 2 < L) S[j + 2] = e;
-      }
-    }
   }
 }
 
@@ -1107,69 +1007,6 @@ __device__ __forceinline__ void face_flux(const FH<TC>* V, const Region<Sh>& R, 
 // cell thick or near a mirror edge): there each own cell's net flux is
 // formed from global memory, face by face, as the reference forms it.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ int ref_index(const InstDev& in, int i, int pm, int d, int& mir) {
-  unsigned m, cl;
-  int r;
-  if (d == 0)
-    r = map_axis(i + pm, in.nx, in.flags & kPeriodicX, in.flags & kMirrorW, in.flags & kMirrorE, m, cl);
-  else
-    r = map_axis(i + pm, in.ny, in.flags & kPeriodicY, in.flags & kMirrorS, in.flags & kMirrorN, m, cl);
-  mir = (int)m;
-  return r;
-}
-
-// Value of plane k at offset o in FP64 (FP32 storage: deviation + reference).
-template <typename TS>
-__device__ __forceinline__ double full_val(const InstDev& in, const TS* src, int k, long long o) {
-  if constexpr (sizeof(TS) == 4) return double(src[in.plane * k + o]) + in.ref[k];
-  else return double(src[in.plane * k + o]);
-}
-
-// Face flux of distribution k0 + i (k0 = 0: f, kQ: h) out of fluid cell
-// (x, y) along `axis`, with the reference's physical addressing: the
-// stencil line through the mapped neighbours (direction remapped at a
-// mirror), its first solid run extrapolated from the two nearest fluid
-// points of the line in direction i; val(k, o) gives the FP64 value of
-// plane k at offset o.
-template <typename TC, typename Val>
-__device__ TC ref_line_flux(const InstDev& in, const Val& val, int k0, int x, int y, int i, int axis) {
-  const int e = axis == 0 ? c_lat_x[i] : c_lat_y[i];
-  const int s = e > 0 ? 1 : (e < 0 ? -1 : 0);
-  if (s == 0) return TC(0);
-  const int L = in.flux_method == 1 ? 5 : 3;
-  const int low = (L - 1) / 2;
-  const int start = (axis == 0 ? x : y) - s * low;
-  TC V[5];
-  int sld[5], any = 0;
-  for (int j = 0; j < L; j++) {
-    int mir;
-    const int p = ref_index(in, start, s * j, axis, mir);
-    const int d = mir ? (axis == 0 ? c_mir_ew[i] : c_mir_ns[i]) : i;
-    const long long o = axis == 0 ? (long long)y * in.pitch + p : (long long)p * in.pitch + x;
-    V[j] = TC(val(k0 + d, o));
-    sld[j] = in.ctype[o] == 2;
-    any |= sld[j];
-  }
-  if (any) {
-    int diff = 0, jj = 0, pos = 0, mir;
-    for (int j = 0; j < L - 1; j++) {
-      diff = sld[j] - sld[j + 1];
-      if (diff > 0) { jj = j; pos = ref_index(in, start, s * j, axis, mir); break; }
-      if (diff < 0) { jj = j + 1; pos = ref_index(in, start, s * (j + 1), axis, mir); break; }
-    }
-    const int m1 = ref_index(in, pos, s * diff, axis, mir);
-    const int m2 = ref_index(in, pos, s * 2 * diff, axis, mir);
-    const long long o1 = axis == 0 ? (long long)y * in.pitch + m1 : (long long)m1 * in.pitch + x;
-    const long long o2 = axis == 0 ? (long long)y * in.pitch + m2 : (long long)m2 * in.pitch + x;
-    V[jj] = TC(2) * TC(val(k0 + i, o1)) - TC(val(k0 + i, o2));
-    const int nx = jj - diff;
-    if (nx >= 0 && nx < L) V[nx] = V[jj];
-  }
-  const TC v = TC(double(e > 0 ? e : -e) * in.c);
-  if (L == 5) return weno5(v, V[0], V[1], V[2], V[3], V[4]);
-  return nnd(v, V[0], V[1], V[2]);
-}
-
 // Face fluxes (f, h) of direction i out of cell (x, y) along `axis`: the
 // wall closure alpha |e| f at a wall owner, else the reference line.
 template <typename Val>
@@ -1607,8 +1444,6 @@ __global__ __launch_bounds__(Sh::NT) __attribute__((amdgpu_waves_per_eu(6))) voi
   flux_tiles<double, double, MODE, MOM>(insts, tiles, ntiles, par, *stepp, R, S, VA, VB);
 }
 
-#include "lbm_strip.hpp"
-
 // The flux kernel of a storage/compute type pair and tile shape.
 template <typename TS, typename TC, int MODE, bool MOM, typename Sh>
 struct FluxKernel {
@@ -1618,55 +1453,6 @@ template <int MODE, bool MOM, typename Sh>
 struct FluxKernel<double, double, MODE, MOM, Sh> {
   static constexpr auto fn = &k_flux64<MODE, MOM, Sh>;
 };
-
-// ---------------------------------------------------------------------------
-// k_alpha: wall closure factor of each wall cell with a non-solid axis
-// neighbour, from the neighbours' face fluxes of `which` (0: f2 or f1,
-// 1: f3, 2: the current state),
-// following the reference's physical stencil addressing (cpuLBM.cpp:1171-1326,
-// 1502-1590).
-// ---------------------------------------------------------------------------
-__constant__ int c_wall_dx[4] = {-1, 1, 0, 0};
-__constant__ int c_wall_dy[4] = {0, 0, -1, 1};
-__constant__ int c_wall_in[4][4] = {{1, 5, 8, 9}, {3, 6, 7, 11}, {2, 5, 6, 10}, {4, 7, 8, 12}};
-__constant__ int c_wall_out[4][4] = {{3, 6, 7, 11}, {1, 5, 8, 9}, {4, 8, 7, 12}, {2, 6, 5, 10}};
-
-template <typename TS, typename TC>
-__global__ void k_alpha(const InstDev* insts, const WallRef* walls, int nwalls, int which, int par,
-                        const int* stepp) {
-  const int step = *stepp;
-  const int w = blockIdx.x * blockDim.x + threadIdx.x;
-  if (w >= nwalls) return;
-  const WallRef wr = walls[w];
-  const InstDev& in = insts[wr.inst];
-  if (frozen_by_failure(in, step)) return;
-  const void* srcv = which == 0 ? in.f2 : (which == 1 ? in.f3 : in.state[in.parity0 ^ par]);
-  const TS* src = reinterpret_cast<const TS*>(srcv);
-  const auto fv = [&](int k, long long o) { return full_val(in, src, k, o); };
-  const long long ow = (long long)wr.y * in.pitch + wr.x;
-  double in_f = 0, out_f = 0;
-  for (int j = 0; j < 4; j++) {
-    int mx, my;
-    const int xn = ref_index(in, wr.x, c_wall_dx[j], 0, my);
-    const int yn = ref_index(in, wr.y, c_wall_dy[j], 1, mx);
-    const long long on = (long long)yn * in.pitch + xn;
-    if (in.ctype[on] >= 2) continue;
-    const int axis = j < 2 ? 0 : 1;
-    // the wall cell's own spacing: its axis neighbours share its row (x
-    // faces) or column (y faces), so the face-length weights of a
-    // non-uniform grid reduce to it
-    const double dd = axis == 0 ? (in.dxs ? in.dxs[wr.x] : in.dx) : (in.dys ? in.dys[wr.y] : in.dy);
-    for (int k = 0; k < 4; k++) {
-      const int i = c_wall_in[j][k], io = c_wall_out[j][k];
-      const double F = double(ref_line_flux<TC>(in, fv, 0, xn, yn, i, axis));
-      in_f += F / dd;
-      const double vv = fabs(double(axis == 0 ? c_lat_x[io] : c_lat_y[io]) * in.c);
-      const double fw = full_val(in, src, io, ow);
-      out_f += fw * vv / dd;
-    }
-  }
-  in.alpha[ow] = in_f / out_f;
-}
 
 // ---------------------------------------------------------------------------
 // Initialisation (reference initialiseFunctions, cpuLBM.cpp:846-875) and
@@ -1937,20 +1723,6 @@ void flux_tile_dims(int shape, int* w, int* h) {
 int tile_halo() { return kH; }
 int dflux_planes() { return kNDF; }
 
-static int grid_for(const void* kernel, int threads, int max_per = 0) {
-  int dev = 0, cus = 256, per = 4;
-  (void)hipGetDevice(&dev);
-  hipDeviceProp_t prop;
-  if (hipGetDeviceProperties(&prop, dev) == hipSuccess) cus = prop.multiProcessorCount;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, threads, 0) != hipSuccess || per < 1) per = 1;
-  if (max_per > 0 && per > max_per) per = max_per;
-  long long g = (long long)cus * per;
-  g -= g % 8;
-  return (int)(g < 8 ? 8 : g);
-}
-
-static int blocks_for(int ntiles, int g) { return ntiles <= g ? ntiles : g; }
-
 // Persistent grid sizes of every step kernel of one storage/compute type and
 // flux tile shape, computed once (before any stream capture).
 // Compute type of the pointwise stage kernels and the wall closure: FP64
@@ -1964,7 +1736,6 @@ static int blocks_for(int ntiles, int g) { return ntiles <= g ? ntiles : g; }
 // scheme's unstable mode about as strongly as FP32 states do and the run
 // ends earlier.
 using TP = double;
-using TW = double;
 
 // The stage-3 flux kernel also sums the moments of dF(f3) for the FP64
 // moment planes of FP32 storage.
@@ -2010,42 +1781,6 @@ static void launch_phys(const StepLaunch& L, hipStream_t s, int par) {
                                                                                   L.step_ctr);
 }
 
-// Compute type of the strip kernels: FP64 for FP64 storage; for FP32
-// storage the precision of the instance's equilibria (FP32 for instances
-// near their reference equilibrium, FP64 for the others: on the 4096^2
-// Riemann deck FP32 stencil arithmetic on strips ended the mixed run at
-// step 1939, FP64 arithmetic completes the 2000 steps), each kind of
-// instance taken by its own launch over the same item list.
-template <typename TS, typename TC, int MODE>
-struct StripGrids {
-  int fast = 0, solid = 0;
-  static const StripGrids& get() {
-    static const StripGrids g = [] {
-      StripGrids r;
-      // FP64 arithmetic: three 4-wave blocks per CU (three waves per SIMD)
-      // even where the registers would allow four, which run slower (4096^2
-      // Riemann stage-2 flux 2.09 ms at four waves, 1.67 ms at three)
-      const int per = sizeof(TC) == 8 ? 3 : 0;
-      r.fast = grid_for((const void*)k_strip<TS, TC, MODE, false>, 256, per);
-      r.solid = grid_for((const void*)k_strip<TS, TC, MODE, true>, 256, per);
-      return r;
-    }();
-    return g;
-  }
-};
-
-template <typename TS, typename TC, int MODE>
-static void launch_strips(const StepLaunch& L, hipStream_t s, int par) {
-  const StripGrids<TS, TC, MODE>& g = StripGrids<TS, TC, MODE>::get();
-  const int nf = L.nstrips_fast, ns = L.nstrips - L.nstrips_fast;
-  if (nf > 0)
-    k_strip<TS, TC, MODE, false><<<blocks_for((nf + 3) / 4, g.fast), 256, 0, s>>>(L.insts, L.strips, nf, par,
-                                                                                  L.step_ctr);
-  if (ns > 0)
-    k_strip<TS, TC, MODE, true><<<blocks_for((ns + 3) / 4, g.solid), 256, 0, s>>>(L.insts, L.strips + nf, ns, par,
-                                                                                  L.step_ctr);
-}
-
 // One flux stage of MODE: the strip kernels for the instances on strips and
 // the tile kernel for the others (every instance for the moment-summing
 // stage-3 flux of FP32 storage, which has no strip form), then the
@@ -2055,14 +1790,7 @@ static void launch_flux(const StepLaunch& L, hipStream_t s, int par, int grid_ti
   const int* step = L.step_ctr;
   bool tiles = true;
   if constexpr (!MOM) {
-    if (L.nstrips > 0) {
-      if constexpr (sizeof(TS) == 4) {
-        if (L.eq_kinds & 2) launch_strips<TS, float, MODE>(L, s, par);
-        if (L.eq_kinds & 1) launch_strips<TS, double, MODE>(L, s, par);
-      } else {
-        launch_strips<TS, double, MODE>(L, s, par);
-      }
-    }
+    if (L.nstrips > 0) launch_strips<TS, MODE>(L, s, par);
     tiles = L.tiles_rest > 0;
   }
   if (tiles)
@@ -2078,14 +1806,7 @@ static void prepare_shapes() {
   (void)StepGrids<TS, TC, Shape2>::get();
   (void)StepGrids<TS, TC, Shape3>::get();
   (void)StepGrids<TS, TC, Shape4>::get();
-  (void)StripGrids<TS, double, 0>::get();
-  (void)StripGrids<TS, double, 2>::get();
-  if constexpr (sizeof(TS) == 8) {
-    (void)StripGrids<TS, double, 1>::get();
-  } else {
-    (void)StripGrids<TS, float, 0>::get();
-    (void)StripGrids<TS, float, 2>::get();
-  }
+  prepare_strips<TS>();
 }
 
 void prepare_launch(int fp64) {
@@ -2110,7 +1831,6 @@ static void launch_rk3(const StepLaunch& L, hipStream_t s, int par, KernelTimer*
   const int* step = L.step_ctr;
   const StepGrids<TS, TC, Sh>& G = StepGrids<TS, TC, Sh>::get();
   const int g1 = G.flux0, g3 = G.flux3;
-  const int wb = (L.nwalls + 255) / 256;
   if (tm) tm->begin(0, s);
   per_eq_kind<TS>(L, [&](auto te, int k) {
     k_s12<TS, TP, decltype(te)><<<blocks_for(L.nptiles, G.s12[k]), kNT, 0, s>>>(L.insts, L.ptiles, L.nptiles, par,
@@ -2119,7 +1839,7 @@ static void launch_rk3(const StepLaunch& L, hipStream_t s, int par, KernelTimer*
   if (tm) tm->end(0, s);
   if (L.nwalls) {
     if (tm) tm->begin(1, s);
-    k_alpha<TS, TW><<<wb, 256, 0, s>>>(L.insts, L.walls, L.nwalls, 0, par, step);
+    launch_alpha<TS>(L, s, 0, par);
     if (tm) tm->end(1, s);
   }
   if (tm) tm->begin(2, s);
@@ -2133,7 +1853,7 @@ static void launch_rk3(const StepLaunch& L, hipStream_t s, int par, KernelTimer*
   if (tm) tm->end(3, s);
   if (L.nwalls) {
     if (tm) tm->begin(1, s);
-    k_alpha<TS, TW><<<wb, 256, 0, s>>>(L.insts, L.walls, L.nwalls, 1, par, step);
+    launch_alpha<TS>(L, s, 1, par);
     if (tm) tm->end(1, s);
   }
   if (tm) tm->begin(4, s);
@@ -2149,7 +1869,6 @@ static void launch_one_stage(const StepLaunch& L, hipStream_t s, int par, Kernel
   const StepGrids<TS, TC, Sh>& G = StepGrids<TS, TC, Sh>::get();
   const int g1 = FM == 0 ? G.flux0 : G.fluxe;
   const int* g2 = METHOD == 0 ? G.fin0 : (METHOD == 2 ? G.fin2 : G.fin3);
-  const int wb = (L.nwalls + 255) / 256;
   if constexpr (METHOD == 0) {
     if (tm) tm->begin(0, s);
     per_eq_kind<TS>(L, [&](auto te, int k) {
@@ -2160,7 +1879,7 @@ static void launch_one_stage(const StepLaunch& L, hipStream_t s, int par, Kernel
   }
   if (L.nwalls) {
     if (tm) tm->begin(1, s);
-    k_alpha<TS, TW><<<wb, 256, 0, s>>>(L.insts, L.walls, L.nwalls, METHOD == 0 ? 0 : 2, par, step);
+    launch_alpha<TS>(L, s, METHOD == 0 ? 0 : 2, par);
     if (tm) tm->end(1, s);
   }
   if (tm) tm->begin(2, s);

@@ -120,6 +120,16 @@ constexpr int kPointW = 64, kPointH = 4;  // pointwise tile: 64 x 4 cells, 256 t
 template <typename TS, typename TC>
 void launch_step(const StepLaunch& L, hipStream_t s, int par, KernelTimer* tm);
 
+// The strip flux kernels of one flux stage (MODE 0, 1, 2 of k_strip) and the
+// wall closure of the distributions `which` (0: f2 or f1, 1: f3, 2: the
+// current state).
+template <typename TS, int MODE>
+void launch_strips(const StepLaunch& L, hipStream_t s, int par);
+template <typename TS>
+void launch_alpha(const StepLaunch& L, hipStream_t s, int which, int par);
+template <typename TS>
+void prepare_strips();
+
 // Computes the persistent grid sizes of the step kernels (call before a
 // stream capture).
 void prepare_launch(int fp64);

@@ -1,0 +1,131 @@
+// lbm_strip.hip — strip flux kernels (lbm_strip.hpp) and the wall closure
+// kernel of the D2Q13 thermal FD-LBM, with their launchers.
+#include "lbm_stencil.hpp"
+
+namespace uqlbm {
+
+#include "lbm_strip.hpp"
+
+// ---------------------------------------------------------------------------
+// k_alpha: wall closure factor of each wall cell with a non-solid axis
+// neighbour, from the neighbours' face fluxes of `which` (0: f2 or f1,
+// 1: f3, 2: the current state),
+// following the reference's physical stencil addressing (cpuLBM.cpp:1171-1326,
+// 1502-1590).
+// ---------------------------------------------------------------------------
+static __constant__ int c_wall_dx[4] = {-1, 1, 0, 0};
+static __constant__ int c_wall_dy[4] = {0, 0, -1, 1};
+static __constant__ int c_wall_in[4][4] = {{1, 5, 8, 9}, {3, 6, 7, 11}, {2, 5, 6, 10}, {4, 7, 8, 12}};
+static __constant__ int c_wall_out[4][4] = {{3, 6, 7, 11}, {1, 5, 8, 9}, {4, 8, 7, 12}, {2, 6, 5, 10}};
+
+template <typename TS, typename TC>
+__global__ void k_alpha(const InstDev* insts, const WallRef* walls, int nwalls, int which, int par,
+                        const int* stepp) {
+  const int step = *stepp;
+  const int w = blockIdx.x * blockDim.x + threadIdx.x;
+  if (w >= nwalls) return;
+  const WallRef wr = walls[w];
+  const InstDev& in = insts[wr.inst];
+  if (frozen_by_failure(in, step)) return;
+  const void* srcv = which == 0 ? in.f2 : (which == 1 ? in.f3 : in.state[in.parity0 ^ par]);
+  const TS* src = reinterpret_cast<const TS*>(srcv);
+  const auto fv = [&](int k, long long o) { return full_val(in, src, k, o); };
+  const long long ow = (long long)wr.y * in.pitch + wr.x;
+  double in_f = 0, out_f = 0;
+  for (int j = 0; j < 4; j++) {
+    int mx, my;
+    const int xn = ref_index(in, wr.x, c_wall_dx[j], 0, my);
+    const int yn = ref_index(in, wr.y, c_wall_dy[j], 1, mx);
+    const long long on = (long long)yn * in.pitch + xn;
+    if (in.ctype[on] >= 2) continue;
+    const int axis = j < 2 ? 0 : 1;
+    // the wall cell's own spacing: its axis neighbours share its row (x
+    // faces) or column (y faces), so the face-length weights of a
+    // non-uniform grid reduce to it
+    const double dd = axis == 0 ? (in.dxs ? in.dxs[wr.x] : in.dx) : (in.dys ? in.dys[wr.y] : in.dy);
+    for (int k = 0; k < 4; k++) {
+      const int i = c_wall_in[j][k], io = c_wall_out[j][k];
+      const double F = double(ref_line_flux<TC>(in, fv, 0, xn, yn, i, axis));
+      in_f += F / dd;
+      const double vv = fabs(double(axis == 0 ? c_lat_x[io] : c_lat_y[io]) * in.c);
+      const double fw = full_val(in, src, io, ow);
+      out_f += fw * vv / dd;
+    }
+  }
+  in.alpha[ow] = in_f / out_f;
+}
+
+template <typename TS>
+void launch_alpha(const StepLaunch& L, hipStream_t s, int which, int par) {
+  k_alpha<TS, double><<<(L.nwalls + 255) / 256, 256, 0, s>>>(L.insts, L.walls, L.nwalls, which, par, L.step_ctr);
+}
+
+// Compute type of the strip kernels: FP64 for FP64 storage; for FP32
+// storage the precision of the instance's equilibria (FP32 for instances
+// near their reference equilibrium, FP64 for the others: on the 4096^2
+// Riemann deck FP32 stencil arithmetic on strips ended the mixed run at
+// step 1939, FP64 arithmetic completes the 2000 steps), each kind of
+// instance taken by its own launch over the same item list.
+template <typename TS, typename TC, int MODE>
+struct StripGrids {
+  int fast = 0, solid = 0;
+  static const StripGrids& get() {
+    static const StripGrids g = [] {
+      StripGrids r;
+      // FP64 arithmetic: three 4-wave blocks per CU (three waves per SIMD)
+      // even where the registers would allow four, which run slower (4096^2
+      // Riemann stage-2 flux 2.09 ms at four waves, 1.67 ms at three)
+      const int per = sizeof(TC) == 8 ? 3 : 0;
+      r.fast = grid_for((const void*)k_strip<TS, TC, MODE, false>, 256, per);
+      r.solid = grid_for((const void*)k_strip<TS, TC, MODE, true>, 256, per);
+      return r;
+    }();
+    return g;
+  }
+};
+
+template <typename TS, typename TC, int MODE>
+static void launch_strips_as(const StepLaunch& L, hipStream_t s, int par) {
+  const StripGrids<TS, TC, MODE>& g = StripGrids<TS, TC, MODE>::get();
+  const int nf = L.nstrips_fast, ns = L.nstrips - L.nstrips_fast;
+  if (nf > 0)
+    k_strip<TS, TC, MODE, false><<<blocks_for((nf + 3) / 4, g.fast), 256, 0, s>>>(L.insts, L.strips, nf, par,
+                                                                                  L.step_ctr);
+  if (ns > 0)
+    k_strip<TS, TC, MODE, true><<<blocks_for((ns + 3) / 4, g.solid), 256, 0, s>>>(L.insts, L.strips + nf, ns, par,
+                                                                                  L.step_ctr);
+}
+
+template <typename TS, int MODE>
+void launch_strips(const StepLaunch& L, hipStream_t s, int par) {
+  if constexpr (sizeof(TS) == 4) {
+    if (L.eq_kinds & 2) launch_strips_as<TS, float, MODE>(L, s, par);
+    if (L.eq_kinds & 1) launch_strips_as<TS, double, MODE>(L, s, par);
+  } else {
+    launch_strips_as<TS, double, MODE>(L, s, par);
+  }
+}
+
+template <typename TS>
+void prepare_strips() {
+  (void)StripGrids<TS, double, 0>::get();
+  (void)StripGrids<TS, double, 2>::get();
+  if constexpr (sizeof(TS) == 8) {
+    (void)StripGrids<TS, double, 1>::get();
+  } else {
+    (void)StripGrids<TS, float, 0>::get();
+    (void)StripGrids<TS, float, 2>::get();
+  }
+}
+
+template void launch_alpha<double>(const StepLaunch&, hipStream_t, int, int);
+template void launch_alpha<float>(const StepLaunch&, hipStream_t, int, int);
+template void launch_strips<double, 0>(const StepLaunch&, hipStream_t, int);
+template void launch_strips<double, 1>(const StepLaunch&, hipStream_t, int);
+template void launch_strips<double, 2>(const StepLaunch&, hipStream_t, int);
+template void launch_strips<float, 0>(const StepLaunch&, hipStream_t, int);
+template void launch_strips<float, 2>(const StepLaunch&, hipStream_t, int);
+template void prepare_strips<double>();
+template void prepare_strips<float>();
+
+}  // namespace uqlbm

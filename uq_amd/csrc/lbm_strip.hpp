@@ -1,5 +1,5 @@
 // lbm_strip.hpp — strip flux kernels (k_strip) of the D2Q13 thermal FD-LBM,
-// included by lbm_kernels.hip after the face reconstructions.
+// included by lbm_strip.hip after the face reconstructions.
 //
 // The net fluxes of MODE 0, 1 and 2 without moment sums (every flux stage
 // except the stage-3 flux of FP32 storage) for the instances whose cells all
