@@ -136,16 +136,16 @@ __device__ __forceinline__ double full_val(const InstDev& in, const TS* src, int
 // mirror), its first solid run extrapolated from the two nearest fluid
 // points of the line in direction i; val(k, o) gives the FP64 value of
 // plane k at offset o.
-template <typename TC, typename Val>
-__device__ TC ref_line_flux(const InstDev& in, const Val& val, int k0, int x, int y, int i, int axis) {
-  const int e = axis == 0 ? c_lat_x[i] : c_lat_y[i];
-  const int s = e > 0 ? 1 : (e < 0 ? -1 : 0);
-  if (s == 0) return TC(0);
-  const int L = in.flux_method == 1 ? 5 : 3;
-  const int low = (L - 1) / 2;
+// (The loops are unrolled over the L points, so a line's loads go out
+// together and every array index is a constant.)
+template <int L, typename TC, typename Val>
+__device__ TC ref_line(const InstDev& in, const Val& val, int k0, int x, int y, int i, int axis, int e) {
+  const int s = e > 0 ? 1 : -1;
+  constexpr int low = (L - 1) / 2;
   const int start = (axis == 0 ? x : y) - s * low;
-  TC V[5];
-  int sld[5], any = 0;
+  TC V[L];
+  int sld[L], any = 0;
+#pragma unroll
   for (int j = 0; j < L; j++) {
     int mir;
     const int p = ref_index(in, start, s * j, axis, mir);
@@ -157,22 +157,36 @@ __device__ TC ref_line_flux(const InstDev& in, const Val& val, int k0, int x, in
   }
   if (any) {
     int diff = 0, jj = 0, pos = 0, mir;
+#pragma unroll
     for (int j = 0; j < L - 1; j++) {
-      diff = sld[j] - sld[j + 1];
-      if (diff > 0) { jj = j; pos = ref_index(in, start, s * j, axis, mir); break; }
-      if (diff < 0) { jj = j + 1; pos = ref_index(in, start, s * (j + 1), axis, mir); break; }
+      const int d = sld[j] - sld[j + 1];
+      if (diff == 0 && d != 0) {
+        diff = d;
+        jj = d > 0 ? j : j + 1;
+        pos = ref_index(in, start, s * jj, axis, mir);
+      }
     }
     const int m1 = ref_index(in, pos, s * diff, axis, mir);
     const int m2 = ref_index(in, pos, s * 2 * diff, axis, mir);
     const long long o1 = axis == 0 ? (long long)y * in.pitch + m1 : (long long)m1 * in.pitch + x;
     const long long o2 = axis == 0 ? (long long)y * in.pitch + m2 : (long long)m2 * in.pitch + x;
-    V[jj] = TC(2) * TC(val(k0 + i, o1)) - TC(val(k0 + i, o2));
+    const TC ex = TC(2) * TC(val(k0 + i, o1)) - TC(val(k0 + i, o2));
     const int nx = jj - diff;
-    if (nx >= 0 && nx < L) V[nx] = V[jj];
+#pragma unroll
+    for (int j = 0; j < L; j++)
+      if (j == jj || j == nx) V[j] = ex;
   }
   const TC v = TC(double(e > 0 ? e : -e) * in.c);
-  if (L == 5) return weno5(v, V[0], V[1], V[2], V[3], V[4]);
-  return nnd(v, V[0], V[1], V[2]);
+  if constexpr (L == 5) return weno5(v, V[0], V[1], V[2], V[3], V[4]);
+  else return nnd(v, V[0], V[1], V[2]);
+}
+
+template <typename TC, typename Val>
+__device__ __forceinline__ TC ref_line_flux(const InstDev& in, const Val& val, int k0, int x, int y, int i, int axis) {
+  const int e = axis == 0 ? c_lat_x[i] : c_lat_y[i];
+  if (e == 0) return TC(0);
+  return in.flux_method == 1 ? ref_line<5, TC>(in, val, k0, x, y, i, axis, e)
+                             : ref_line<3, TC>(in, val, k0, x, y, i, axis, e);
 }
 
 static int grid_for(const void* kernel, int threads, int max_per = 0) {
