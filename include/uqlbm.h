@@ -276,17 +276,16 @@ int lbm_set_graphs(int32_t enable);
 
 /*
  * Flux stages of instances whose cells all take the logical stencil
- * addressing can run on the strip kernels (one wavefront per 58-column,
- * 32-row strip, marched row by row) instead of the flux tile kernels, except
- * the moment-summing stage-3 flux of LBM_PREC_MIXED. mode 0: every flux
- * stage on the tile kernels; 1 (default): strips for launch groups with at
- * least 2048 strip items (enough to fill the GPU; e.g. a 4096^2 instance or
- * the 256-member ensemble), tiles for smaller groups; 2: strips wherever an
- * instance can take them. Results are bitwise equal either way (FP64, and
- * LBM_PREC_MIXED instances near their reference equilibrium; mixed
- * instances far from it compute their strip stencils in FP64, the tile
- * kernels in FP32). Applies to step calls made afterwards; LBM_ERR_ARG for
- * another mode. No counterpart in the reference.
+ * addressing run on the strip kernels (one wavefront per direction of a
+ * 58-column strip of 2 to 32 rows, marched row by row) instead of the flux
+ * tile kernels, except the moment-summing stage-3 flux of LBM_PREC_MIXED.
+ * mode 0: every flux stage on the tile kernels; 1 (default) and 2: strips
+ * wherever an instance can take them. Results are bitwise equal either way,
+ * except LBM_PREC_MIXED instances far from their reference equilibrium: they
+ * compute their strip stencils in FP64 in mode 2 and, in mode 1, in step
+ * calls of at least 2048 32-row strips (a 4096^2 instance), elsewhere in FP32
+ * as the tile kernels do. Applies to step calls made afterwards; LBM_ERR_ARG
+ * for another mode. No counterpart in the reference.
  */
 int lbm_set_strips(int32_t mode);
 

@@ -108,14 +108,14 @@ constexpr int kResHist = 20;  // residual history slots per tracked instance
 template <typename TS>
 constexpr bool kStage3G = sizeof(TS) == 4;
 
-// One tile of one instance: the unit of work of a block.
 // Strip work items of the strip flux kernels (TileRef with tx = strip index,
-// ty = first row, flags = kTileSolid | kStripDesc | row count << 8):
-// kStripW own columns (with a 3-column halo on each side, 64 lanes) by up to
-// kStripH rows; kStripDesc: the item takes its rows from the last to the
-// first.
-constexpr int kStripW = 58, kStripH = 32;
+// ty = first row, flags = kTileSolid | kStripDesc | row count <<
+// kStripRowsBit): kStripW own columns (with a 3-column halo on each side, 64
+// lanes) by some rows; kStripDesc: the item takes its rows from the last to
+// the first.
+constexpr int kStripW = 58, kStripRowsBit = 8;
 
+// One tile of one instance: the unit of work of a block.
 struct TileRef {
   int inst;
   int tx, ty;

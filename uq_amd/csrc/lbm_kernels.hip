@@ -1806,7 +1806,6 @@ static void prepare_shapes() {
   (void)StepGrids<TS, TC, Shape2>::get();
   (void)StepGrids<TS, TC, Shape3>::get();
   (void)StepGrids<TS, TC, Shape4>::get();
-  prepare_strips<TS>();
 }
 
 void prepare_launch(int fp64) {

@@ -570,33 +570,59 @@ static std::vector<TileRef> build_flux_tiles(const Solver& s, int shape) {
   return tiles;
 }
 
-// Strip work items of an instance whose cells all take the logical stencil
-// addressing (none otherwise). Strip sx covers columns 58 sx .. 58 sx + 57;
-// its rows are grouped into items of at most 32 rows. A row is solid when
-// the region its cells' stencils read (the strip's 64 columns x0 - 3 ..
-// x0 + 60 by rows y - 3 .. y + 3, each position mapped as the kernels map
-// it: periodic, mirrored or clamped) holds a solid cell; consecutive rows
-// of the same kind form an item, so that only the rows near a solid take
-// the solid path. TileRef: tx = strip index, ty = first row,
-// flags = kTileSolid (solid rows) | kStripDesc (every second item of a
-// column) | row count << 8.
-static void build_strips(const Solver& s, std::vector<TileRef>& fast, std::vector<TileRef>& solid) {
-  fast.clear();
-  solid.clear();
+// Strip work items of up to `rows` rows of an instance (instance index
+// `inst`), appended to out. Consecutive rows of the same kind (solid or not)
+// form an item, so that only the rows near a solid take the solid path.
+// TileRef: tx = strip index, ty = first row, flags = kTileSolid (solid rows)
+// | kStripDesc (every second item of a column) | row count << kStripRowsBit.
+static void strip_items(const Solver& s, int rows, int inst, std::vector<TileRef>& out) {
+  const size_t first = out.size();
+  for (int sx = 0; sx < s.strip_cols; sx++) {
+    const char* solid = s.strip_solid.data() + (size_t)sx * s.ny;
+    // the items of a strip column alternate between ascending and
+    // descending row order (kStripDesc), so that neighbours one above the
+    // other read the rows they share at about the same time
+    for (int y = 0, k = 0; y < s.ny; k++) {
+      int n = 1;
+      while (y + n < s.ny && n < rows && solid[y + n] == solid[y]) n++;
+      out.push_back(TileRef{inst, sx, y, (solid[y] ? kTileSolid : 0) | ((k & 1) ? kStripDesc : 0) | (n << kStripRowsBit)});
+      y += n;
+    }
+  }
+  // row-major order (first row, then strip): the waves of a workgroup take
+  // consecutive items, side by side strips of the same rows, whose halo
+  // columns they then share in L2 (4096^2 Riemann stage-2 and stage-3 flux
+  // 1.75 and 2.17 ms in this order, 2.18 and 2.74 ms strip by strip)
+  std::stable_sort(out.begin() + first, out.end(),
+                   [](const TileRef& a, const TileRef& b) { return a.ty != b.ty ? a.ty < b.ty : a.tx < b.tx; });
+}
+
+// Rows of the items that count towards the size of a launch group (far_fp64).
+static constexpr int kStripBlock = 32;
+
+// Strip columns of an instance whose cells all take the logical stencil
+// addressing (none otherwise). Strip sx covers columns 58 sx .. 58 sx + 57.
+// A row of a strip is solid when the region its cells' stencils read (the
+// strip's 64 columns x0 - 3 .. x0 + 60 by rows y - 3 .. y + 3, each position
+// mapped as the kernels map it: periodic, mirrored or clamped) holds a solid
+// cell.
+static void mark_strips(Solver& s) {
+  s.strip_solid.clear();
+  s.strip_cols = s.strip_blocks = 0;
   if (s.any_phys) return;
   const int H = tile_halo();
   bool any_solid = false;
   for (size_t k = 0; k < s.ctype_host.size() && !any_solid; k++) any_solid = s.ctype_host[k] == 2;
-  const int nsx = (s.nx + kStripW - 1) / kStripW;
-  int m;
-  bool cl;
-  std::vector<int> xs(64), ys(s.ny + 2 * H);
-  for (int j = 0; j < s.ny + 2 * H; j++) ys[j] = ref_map(s, j - H, 1, m, cl);
-  std::vector<char> rs(s.ny + 2 * H, 0), rowsolid(s.ny, 0);
-  for (int sx = 0; sx < nsx; sx++) {
-    const int x0 = sx * kStripW;
-    if (any_solid) {
-      for (int l = 0; l < 64; l++) xs[l] = ref_map(s, x0 - H + l, 0, m, cl);
+  s.strip_cols = (s.nx + kStripW - 1) / kStripW;
+  s.strip_solid.assign((size_t)s.strip_cols * s.ny, 0);
+  if (any_solid) {
+    int m;
+    bool cl;
+    std::vector<int> xs(64), ys(s.ny + 2 * H);
+    for (int j = 0; j < s.ny + 2 * H; j++) ys[j] = ref_map(s, j - H, 1, m, cl);
+    std::vector<char> rs(s.ny + 2 * H, 0);
+    for (int sx = 0; sx < s.strip_cols; sx++) {
+      for (int l = 0; l < 64; l++) xs[l] = ref_map(s, sx * kStripW - H + l, 0, m, cl);
       for (int j = 0; j < s.ny + 2 * H; j++) {  // mapped row j - H across the strip's columns
         bool any = false;
         for (int l = 0; l < 64 && !any; l++) any = type_at(s, xs[l], ys[j]) == 2;
@@ -605,60 +631,53 @@ static void build_strips(const Solver& s, std::vector<TileRef>& fast, std::vecto
       for (int y = 0; y < s.ny; y++) {
         bool any = false;
         for (int k = 0; k <= 2 * H && !any; k++) any = rs[y + k];  // rows y - H .. y + H
-        rowsolid[y] = any;
+        s.strip_solid[(size_t)sx * s.ny + y] = any;
       }
     }
-    // the items of a strip column alternate between ascending and
-    // descending row order (kStripDesc), so that neighbours one above the
-    // other read the rows they share at about the same time
-    for (int y = 0, k = 0; y < s.ny; k++) {
-      const bool sol = rowsolid[y];
-      int n = 1;
-      while (y + n < s.ny && n < kStripH && (bool)rowsolid[y + n] == sol) n++;
-      (sol ? solid : fast).push_back(TileRef{0, sx, y, (sol ? kTileSolid : 0) | ((k & 1) ? kStripDesc : 0) | (n << 8)});
-      y += n;
-    }
   }
-  // row-major order (first row, then strip): the waves of a workgroup take
-  // consecutive items, side by side strips of the same rows, whose halo
-  // columns they then share in L2 (4096^2 Riemann stage-2 and stage-3 flux
-  // 1.75 and 2.17 ms in this order, 2.18 and 2.74 ms strip by strip)
-  auto row_major = [](const TileRef& a, const TileRef& b) { return a.ty != b.ty ? a.ty < b.ty : a.tx < b.tx; };
-  std::stable_sort(fast.begin(), fast.end(), row_major);
-  std::stable_sort(solid.begin(), solid.end(), row_major);
+  std::vector<TileRef> items;
+  strip_items(s, kStripBlock, 0, items);
+  s.strip_blocks = (int)items.size();
 }
 
 static int g_strips = 1;  // lbm_set_strips mode
 bool uqlbm::strips_enabled() { return g_strips != 0; }
 
-// A strip item is one wavefront's sequential march over 12 directions and
-// up to 32 rows, so a launch group takes the strip kernels only with enough
-// items to fill the GPU (two waves per SIMD of 256 CUs); smaller groups (one
-// small instance, the 512 x 256 plate) keep the tile kernels, which spread
-// an instance over many more workgroups.
-static constexpr int kStripMinItems = 2048;
-bool uqlbm::strips_for(int nstrips) {
-  return nstrips > 0 && (g_strips == 2 || (g_strips == 1 && nstrips >= kStripMinItems));
+// FP32 storage far from its reference equilibrium: FP64 stencils in groups
+// of at least 2048 items of 32 rows (3.6 million cells), where the shock
+// decks run their long solves; FP32 below.
+static constexpr int kFarMinBlocks = 2048;
+bool uqlbm::far_fp64(int blocks) { return g_strips == 2 || blocks >= kFarMinBlocks; }
+
+// Rows per strip item of a launch group: the most (32, 16, ... 2) that leave
+// kStripWaves wavefronts, `waves` of them per item (one per direction of
+// k_strip). Every item fills a six-row window and forms one face beyond its
+// own rows, so long items cost less, but with fewer than one to two
+// wavefronts per SIMD (1024 SIMDs) the group waits for its longest march.
+// FP64 us per step at 32 / 16 / 8 / 4 / 2 rows: 64^2 Couette 8 rows 50, 4 rows
+// 46.5, 2 rows 42.6 (384, 768 wavefronts at 4, 2); 301^2 block 16 rows 116,
+// 8 rows 97 (1354, 2709 wavefronts); 256^2 8 rows 51, 4 rows 55 (1920, 3840);
+// ensemble of 48 32 rows 1772, 64 rows 1809, 128 rows 1910; 3072^2 16 rows 4073,
+// 32 rows 4027, 64 rows 4057, 128 rows 4102.
+static constexpr int kStripWaves = 1536, kStripRows = 32, kStripRowsMin = 2;
+static int strip_rows(const std::vector<Solver*>& members, int waves) {
+  long long rows = 0;
+  for (const Solver* s : members) rows += (long long)s->strip_cols * s->ny;
+  int h = kStripRows;
+  while (h > kStripRowsMin && rows * waves < (long long)kStripWaves * h) h /= 2;
+  return h;
 }
 
-int uqlbm::group_strips(const std::vector<Solver*>& members, int shape, std::vector<TileRef>& out, int* tiles_rest) {
+void uqlbm::group_strips(const std::vector<Solver*>& members, int shape, std::vector<TileRef>& out, int* blocks,
+                         int* tiles_rest) {
   out.clear();
-  int nfast = 0, rest = 0;
-  for (size_t k = 0; k < members.size(); k++)
-    for (TileRef t : members[k]->strips_fast) {
-      t.inst = (int)k;
-      out.push_back(t);
-      nfast++;
-    }
-  for (size_t k = 0; k < members.size(); k++)
-    for (TileRef t : members[k]->strips_solid) {
-      t.inst = (int)k;
-      out.push_back(t);
-    }
-  for (Solver* s : members)
-    if (s->nstrips == 0) rest += (int)solver_tiles(*s, shape).size();
-  if (tiles_rest) *tiles_rest = rest;
-  return nfast;
+  *blocks = *tiles_rest = 0;
+  const int rows = strip_rows(members, 12);
+  for (size_t k = 0; k < members.size(); k++) {
+    strip_items(*members[k], rows, (int)k, out);
+    *blocks += members[k]->strip_blocks;
+    if (members[k]->strip_cols == 0) *tiles_rest += (int)solver_tiles(*members[k], shape).size();
+  }
 }
 
 const std::vector<TileRef>& uqlbm::solver_tiles(Solver& s, int shape) {
@@ -817,14 +836,14 @@ extern "C" int lbm_create(const lbm_params* params, int32_t nx, int32_t ny, cons
   }
   s->walls_host = std::move(walls);
   s->ptiles_host = std::move(ptiles);
-  build_strips(*s, s->strips_fast, s->strips_solid);
-  s->nstrips_fast = (int)s->strips_fast.size();
-  s->nstrips = s->nstrips_fast + (int)s->strips_solid.size();
+  mark_strips(*s);
+  std::vector<TileRef> strips;
+  int blocks = 0, rest = 0;
+  group_strips({s.get()}, s->flux_shape, strips, &blocks, &rest);
+  s->nstrips = (int)strips.size();
   if (s->nstrips) {
-    std::vector<TileRef> all(s->strips_fast);
-    all.insert(all.end(), s->strips_solid.begin(), s->strips_solid.end());
-    HIP_TRY(solver_alloc(*s, (void**)&s->strips_dev, all.size() * sizeof(TileRef)));
-    HIP_TRY(hipMemcpy(s->strips_dev, all.data(), all.size() * sizeof(TileRef), hipMemcpyHostToDevice));
+    HIP_TRY(solver_alloc(*s, (void**)&s->strips_dev, strips.size() * sizeof(TileRef)));
+    HIP_TRY(hipMemcpy(s->strips_dev, strips.data(), strips.size() * sizeof(TileRef), hipMemcpyHostToDevice));
   }
   const int st = upload_inst(*s);
   if (st != LBM_OK) return st;
@@ -964,7 +983,7 @@ int uqlbm::run_group(const std::vector<Solver*>& members, InstDev* table_dev, co
     table[k].res_last = members[k]->step + n;
     table[k].ptile0 = ptile0;
     table[k].nptiles = members[k]->nptiles;
-    table[k].strips = L.nstrips > 0 && members[k]->nstrips > 0 ? 1 : 0;
+    table[k].strips = L.nstrips > 0 && members[k]->strip_cols > 0 ? 1 : 0;
     ptile0 += members[k]->nptiles;
   }
   HIP_TRY(hipMemcpyAsync(table_dev, table.data(), table.size() * sizeof(InstDev), hipMemcpyHostToDevice, stream));
@@ -1020,10 +1039,10 @@ int uqlbm::run_group(const std::vector<Solver*>& members, InstDev* table_dev, co
 // `rows` holds ny + 1 doubles; the result is copied to *out.
 // The solver's strip list in its launch description (when strips are on).
 static void solver_strips(const Solver& s, StepLaunch& L) {
-  if (strips_for(s.nstrips)) {
+  if (strips_enabled() && s.nstrips > 0) {
     L.strips = s.strips_dev;
     L.nstrips = s.nstrips;
-    L.nstrips_fast = s.nstrips_fast;
+    L.far64 = far_fp64(s.strip_blocks);
     L.tiles_rest = 0;
   } else {
     L.tiles_rest = s.ntiles;
@@ -1423,7 +1442,7 @@ int uqlbm::batch_set_shape(Batch& b, int shape) {
   b.nphys = count_physical(tiles);
   b.tiles_rest = 0;
   for (Solver* m : b.members)
-    if (m->nstrips == 0) b.tiles_rest += (int)solver_tiles(*m, shape).size();
+    if (m->strip_cols == 0) b.tiles_rest += (int)solver_tiles(*m, shape).size();
   b.eq_kinds = eq_kinds_of(b.precision == LBM_PREC_FP64, b.members.begin(), b.members.end(),
                            [](const Solver* m) { return m->eq32; });
   b.flux_shape = shape;
@@ -1458,7 +1477,7 @@ int uqlbm::batch_finish(Batch& b, lbm_batch** out) {
   HIP_TRY(hipMalloc((void**)&b.ptiles_dev, ptiles.size() * sizeof(TileRef)));
   HIP_TRY(hipMemcpy(b.ptiles_dev, ptiles.data(), ptiles.size() * sizeof(TileRef), hipMemcpyHostToDevice));
   std::vector<TileRef> strips;
-  b.nstrips_fast = group_strips(b.members, b.flux_shape, strips, nullptr);
+  group_strips(b.members, b.flux_shape, strips, &b.strip_blocks, &b.tiles_rest);
   b.nstrips = (int)strips.size();
   if (!strips.empty()) {
     HIP_TRY(hipMalloc((void**)&b.strips_dev, strips.size() * sizeof(TileRef)));
@@ -1483,10 +1502,10 @@ int uqlbm::batch_step(Batch& b, int nsteps) {
                b.ptiles_dev, b.nptiles,   b.rk_method, b.step_ctr,  b.flux_shape};
   L.nphys = b.nphys;
   L.eq_kinds = b.eq_kinds;
-  if (strips_for(b.nstrips)) {
+  if (strips_enabled() && b.nstrips > 0) {
     L.strips = b.strips_dev;
     L.nstrips = b.nstrips;
-    L.nstrips_fast = b.nstrips_fast;
+    L.far64 = far_fp64(b.strip_blocks);
     L.tiles_rest = b.tiles_rest;
   } else {
     L.tiles_rest = b.ntiles;

@@ -54,7 +54,9 @@ struct Solver {
   std::vector<TileRef> tiles_shape[kFluxShapes];  // flux tiles per shape, built on first use
   std::vector<WallRef> walls_host;
   std::vector<TileRef> ptiles_host;
-  std::vector<TileRef> strips_fast, strips_solid;  // strip items (none when a cell needs physical addressing)
+  std::vector<char> strip_solid;    // [strip][y]: the row's stencils reach a solid cell within the strip
+  int strip_cols = 0;               // strips across (0 when a cell needs physical addressing: no strip items)
+  int strip_blocks = 0;             // 32-row strip items (the size of the launch group, far_fp64)
 
   hipStream_t stream = nullptr;
   void* state[2] = {nullptr, nullptr};
@@ -75,7 +77,7 @@ struct Solver {
   TileRef* tiles_dev = nullptr;
   WallRef* walls_dev = nullptr;
   TileRef* ptiles_dev = nullptr;
-  TileRef* strips_dev = nullptr;    // strips_fast then strips_solid
+  TileRef* strips_dev = nullptr;
   double* macro_dev = nullptr;
   int* step_ctr = nullptr;          // device step counter of this solver's launches
   int flux_shape = 0;               // flux tile shape of tiles_dev
@@ -91,7 +93,7 @@ struct Solver {
   std::vector<std::pair<void*, size_t>> owned;  // buffers from solver_alloc, returned to its cache
   int ntiles = 0, nwalls = 0, nptiles = 0;
   int nphys = 0;  // flux tiles flagged kTilePhysical
-  int nstrips = 0, nstrips_fast = 0;
+  int nstrips = 0;
   size_t device_bytes = 0;
 
   int cur = 0;    // state buffer holding the current state
@@ -123,7 +125,7 @@ struct Batch {
   int ntiles = 0, nwalls = 0, nptiles = 0;
   int nphys = 0;  // flux tiles flagged kTilePhysical
   int eq_kinds = 1;  // equilibrium precisions among the members (StepLaunch::eq_kinds)
-  int nstrips = 0, nstrips_fast = 0, tiles_rest = 0;
+  int nstrips = 0, strip_blocks = 0, tiles_rest = 0;
   Batch() = default;
   Batch(Batch&& o) noexcept { *this = std::move(o); }
   Batch& operator=(Batch&& o) noexcept {
@@ -147,7 +149,7 @@ struct Batch {
     nphys = o.nphys;
     eq_kinds = o.eq_kinds;
     nstrips = o.nstrips;
-    nstrips_fast = o.nstrips_fast;
+    strip_blocks = o.strip_blocks;
     tiles_rest = o.tiles_rest;
     o.stream = nullptr;
     o.inst_dev = nullptr;
@@ -167,14 +169,16 @@ int fail_with(int status, const char* fmt, ...);
 // destroyed solver on this device when there is one (contents undefined),
 // else hipMalloc; ~Solver returns it.
 hipError_t solver_alloc(Solver& s, void** p, size_t bytes);
-// Strip flux kernels in use (lbm_set_strips; default on), and whether a
-// launch group with `nstrips` strip items takes them.
+// Strip flux kernels in use (lbm_set_strips; default on), and whether the
+// FP32-storage instances far from their reference equilibrium take FP64
+// stencils in a launch group of `blocks` 32-row strip items.
 bool strips_enabled();
-bool strips_for(int nstrips);
-// Strip list of a launch group (member k's items with instance index k,
-// items without solids first; returns how many those are) and the number
-// of flux tiles of shape `shape` of the members not on strips.
-int group_strips(const std::vector<Solver*>& members, int shape, std::vector<TileRef>& out, int* tiles_rest);
+bool far_fp64(int blocks);
+// Strip list of a launch group (member k's items with instance index k), the
+// group's 32-row strip items, and the number of flux tiles of shape `shape`
+// of the members not on strips.
+void group_strips(const std::vector<Solver*>& members, int shape, std::vector<TileRef>& out, int* blocks,
+                  int* tiles_rest);
 const std::vector<TileRef>& solver_tiles(Solver& s, int shape);
 int default_flux_shape(int precision);
 int batch_set_shape(Batch& b, int shape);

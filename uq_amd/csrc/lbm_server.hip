@@ -68,7 +68,7 @@ struct Server {
   TileRef* strips_dev = nullptr;
   size_t tiles_cap = 0, walls_cap = 0, ptiles_cap = 0, strips_cap = 0;
   int ntiles = 0, nwalls = 0, nptiles = 0;
-  int nstrips = 0, nstrips_fast = 0, tiles_rest = 0;  // strip list of the active requests (StepLaunch)
+  int nstrips = 0, strip_blocks = 0, tiles_rest = 0;  // strip list of the active requests (StepLaunch)
   int nphys = 0;  // flux tiles flagged kTilePhysical
   int eq_kinds = 1;  // equilibrium precisions among the active requests (StepLaunch::eq_kinds)
   bool lists_dirty = true;
@@ -135,7 +135,7 @@ static int rebuild_lists(Server& sv) {
   members.reserve(sv.active.size());
   for (auto& a : sv.active) members.push_back(a.solver);
   std::vector<TileRef> strips;
-  sv.nstrips_fast = group_strips(members, sv.flux_shape, strips, &sv.tiles_rest);
+  group_strips(members, sv.flux_shape, strips, &sv.strip_blocks, &sv.tiles_rest);
   sv.nstrips = (int)strips.size();
   if (strips.size() > sv.strips_cap) {
     if (sv.strips_dev) SV_TRY(hipFree(sv.strips_dev));
@@ -365,10 +365,10 @@ extern "C" int lbm_server_tick(lbm_server* h, int32_t tick_steps, int32_t* activ
                  sv.ptiles_dev, sv.nptiles,   sv.rk_method, sv.step_ctr,  sv.flux_shape};
     L.nphys = sv.nphys;
     L.eq_kinds = sv.eq_kinds;
-    if (strips_for(sv.nstrips)) {
+    if (strips_enabled() && sv.nstrips > 0) {
       L.strips = sv.strips_dev;
       L.nstrips = sv.nstrips;
-      L.nstrips_fast = sv.nstrips_fast;
+      L.far64 = far_fp64(sv.strip_blocks);
       L.tiles_rest = sv.tiles_rest;
     } else {
       L.tiles_rest = sv.ntiles;

@@ -83,61 +83,25 @@ void launch_alpha(const StepLaunch& L, hipStream_t s, int which, int par) {
                                                                             L.step_ctr);
 }
 
-// Compute type of the strip kernels: FP64 for FP64 storage; for FP32
-// storage the precision of the instance's equilibria (FP32 for instances
-// near their reference equilibrium, FP64 for the others: on the 4096^2
-// Riemann deck FP32 stencil arithmetic on strips ended the mixed run at
-// step 1939, FP64 arithmetic completes the 2000 steps), each kind of
-// instance taken by its own launch over the same item list.
+// Compute type of the strip kernels: FP64 for FP64 storage; FP32 for FP32
+// storage near the reference equilibrium; for the other FP32-storage
+// instances FP64 in large launch groups (StepLaunch::far64: on the 4096^2
+// Riemann deck FP32 stencil arithmetic ended the mixed run at step 1939, FP64
+// arithmetic completes the 2000 steps) and FP32 in small ones. A group that
+// needs both has a launch of each over the same item list.
 template <typename TS, typename TC, int MODE>
-struct StripGrids {
-  int fast = 0, solid = 0;
-  static const StripGrids& get() {
-    static const StripGrids g = [] {
-      StripGrids r;
-      // FP64 arithmetic: three 4-wave blocks per CU (three waves per SIMD)
-      // even where the registers would allow four, which run slower (4096^2
-      // Riemann stage-2 flux 2.09 ms at four waves, 1.67 ms at three)
-      const int per = sizeof(TC) == 8 ? 3 : 0;
-      r.fast = grid_for((const void*)k_strip<TS, TC, MODE, false>, 256, per);
-      r.solid = grid_for((const void*)k_strip<TS, TC, MODE, true>, 256, per);
-      return r;
-    }();
-    return g;
-  }
-};
-
-template <typename TS, typename TC, int MODE>
-static void launch_strips_as(const StepLaunch& L, hipStream_t s, int par) {
-  const StripGrids<TS, TC, MODE>& g = StripGrids<TS, TC, MODE>::get();
-  const int nf = L.nstrips_fast, ns = L.nstrips - L.nstrips_fast;
-  if (nf > 0)
-    k_strip<TS, TC, MODE, false><<<blocks_for((nf + 3) / 4, g.fast), 256, 0, s>>>(L.insts, L.strips, nf, par,
-                                                                                  L.step_ctr);
-  if (ns > 0)
-    k_strip<TS, TC, MODE, true><<<blocks_for((ns + 3) / 4, g.solid), 256, 0, s>>>(L.insts, L.strips + nf, ns, par,
-                                                                                  L.step_ctr);
+static void launch_strips_as(const StepLaunch& L, hipStream_t s, int par, int all) {
+  const int chunk = (L.nstrips + 31) / 32 * 4;  // items per XCD, a multiple of a block's four
+  k_strip<TS, TC, MODE><<<8 * 12 * (chunk / 4), 256, 0, s>>>(L.insts, L.strips, L.nstrips, chunk, all, par, L.step_ctr);
 }
 
 template <typename TS, int MODE>
 void launch_strips(const StepLaunch& L, hipStream_t s, int par) {
   if constexpr (sizeof(TS) == 4) {
-    if (L.eq_kinds & 2) launch_strips_as<TS, float, MODE>(L, s, par);
-    if (L.eq_kinds & 1) launch_strips_as<TS, double, MODE>(L, s, par);
+    if ((L.eq_kinds & 2) || !L.far64) launch_strips_as<TS, float, MODE>(L, s, par, !L.far64);
+    if ((L.eq_kinds & 1) && L.far64) launch_strips_as<TS, double, MODE>(L, s, par, 0);
   } else {
-    launch_strips_as<TS, double, MODE>(L, s, par);
-  }
-}
-
-template <typename TS>
-void prepare_strips() {
-  (void)StripGrids<TS, double, 0>::get();
-  (void)StripGrids<TS, double, 2>::get();
-  if constexpr (sizeof(TS) == 8) {
-    (void)StripGrids<TS, double, 1>::get();
-  } else {
-    (void)StripGrids<TS, float, 0>::get();
-    (void)StripGrids<TS, float, 2>::get();
+    launch_strips_as<TS, double, MODE>(L, s, par, 1);
   }
 }
 
@@ -148,7 +112,5 @@ template void launch_strips<double, 1>(const StepLaunch&, hipStream_t, int);
 template void launch_strips<double, 2>(const StepLaunch&, hipStream_t, int);
 template void launch_strips<float, 0>(const StepLaunch&, hipStream_t, int);
 template void launch_strips<float, 2>(const StepLaunch&, hipStream_t, int);
-template void prepare_strips<double>();
-template void prepare_strips<float>();
 
 }  // namespace uqlbm

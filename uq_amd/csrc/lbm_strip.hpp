@@ -1,21 +1,22 @@
-// lbm_strip.hpp — strip flux kernels (k_strip) of the D2Q13 thermal FD-LBM,
-// included by lbm_strip.hip after the face reconstructions.
+// lbm_strip.hpp — strip flux kernels (k_strip, k_strip_mom) of the D2Q13
+// thermal FD-LBM, included by lbm_strip.hip after the face reconstructions.
 //
-// The net fluxes of MODE 0, 1 and 2 without moment sums (every flux stage
-// except the stage-3 flux of FP32 storage) for the instances whose cells all
-// take the logical stencil addressing. One wavefront per work item: a strip
-// of kStripW columns and up to kStripH rows of one instance, marched row by
-// row, one direction after the other. Lane l holds column x0 - 3 + l (a
-// 3-column halo on each side fills the 64 lanes); a lane's y stencil is a
-// window of six rows in its registers and its x stencil comes from the
-// neighbouring lanes by whole-wave DPP shifts, so a work item needs no LDS
-// and no barrier. Each face is computed once: the x face left of a lane's
-// column by that lane, the y face below a row when the window reaches it;
-// a cell's net flux takes the face it shares with its right neighbour from
-// that lane and the face below it from the previous row. The arithmetic of
-// every face and net flux is that of the tile kernels (face_flux, flux_dir).
-// The next row's loads are issued before the current row's faces, so their
-// latency hides behind them.
+// The net fluxes of every flux stage for the instances whose cells all take
+// the logical stencil addressing. A strip is kStripW columns and some rows of
+// one instance, marched row by row by one wavefront for one direction
+// (k_strip) or by a workgroup of four wavefronts, three directions each
+// (k_strip_mom: the stage-3 flux of FP32 storage, whose cells also sum the
+// moments of their net fluxes over the directions). Lane l holds column
+// x0 - 3 + l (a 3-column halo on each side fills the 64 lanes); a lane's y
+// stencil is a window of six rows in its registers and its x stencil comes
+// from the neighbouring lanes by whole-wave DPP shifts, so the faces need no
+// LDS and no barrier. Each face is computed once: the x face left of a
+// lane's column by that lane, the y face below a row when the window reaches
+// it; a cell's net flux takes the face it shares with its right neighbour
+// from that lane and the face below it from the previous row. The arithmetic
+// of every face and net flux is that of the tile kernels (face_flux,
+// flux_dir). The next row's loads are issued before the current row's faces,
+// so their latency hides behind them.
 // (Included inside namespace uqlbm, after the gptr global-pointer alias.)
 #pragma once
 
@@ -139,73 +140,73 @@ struct StripInst {
   double c;
 };
 
-// One direction over the rows of a work item. SX, SY: the signs of the
-// direction's lattice velocity in the march's row order; SOLID: the item's
-// region holds a solid cell; W5: WENO5 faces (else NND). flip: the march
-// takes the item's rows from the last to the first, as rows y0 .. y0 +
-// nrows - 1 of the item turned upside down (row y of the march is row
-// 2 y0 + nrows - 1 - y of the instance), called with SY the negated sign
-// of the direction: each face then has the same upwind owner and the same
-// stencil values in the same order as in the ascending march, so the two
-// orders give the same values bit for bit.
-template <typename TS, typename TC, int MODE, bool SOLID, bool W5, int SX, int SY>
-__device__ __forceinline__ void strip_dir(const StripInst<TS>& in, const StripLane<TC>& C, TC rf, TC rh, int I,
-                                          int y0, int nrows, int flip) {
-  constexpr bool HX = SX != 0, HY = SY != 0;
-  // the instance row of row y of the march
-  const int yflip = 2 * y0 + nrows - 1;
-  auto prow = [&](int y) { return flip ? yflip - y : y; };
-  const int pitch = in.pitch, ny = in.ny;
-  const int aex = c_lat_x[I] > 0 ? c_lat_x[I] : -c_lat_x[I];
-  const int aey = c_lat_y[I] > 0 ? c_lat_y[I] : -c_lat_y[I];
-  const TC vx = TC(double(aex) * in.c), vy = TC(double(aey) * in.c);
-  const int dew = c_mir_ew[I], dns = c_mir_ns[I], dboth = c_mir_ns[dew];
+// The row order of a march: rows y0 .. y0 + nrows - 1 of the item, or (flip)
+// the item turned upside down (row y of the march is row 2 y0 + nrows - 1 - y
+// of the instance), the direction's y sign then negated: each face has the
+// same upwind owner and the same stencil values in the same order either
+// way, so the two orders give the same values bit for bit.
+struct RowOrder {
+  int flip, yflip;
+  __device__ __forceinline__ int operator()(int y) const { return flip ? yflip - y : y; }
+};
+
+// One direction's march state: SX, SY the signs of its lattice velocity in
+// the march's row order; SOLID: the item's region holds a solid cell; W5:
+// WENO5 faces (else NND).
+template <typename TS, typename TC, bool SOLID, bool W5, int SX, int SY>
+struct March {
+  static constexpr bool HX = SX != 0, HY = SY != 0;
+  TC vx, vy;
+  TC rf, rh;  // reference equilibrium of the direction for the wall faces of FP32 storage
+              // (a mirror image of it has the same reference: it depends on |e|)
   // this lane's column in the planes of the direction staged at a row that
   // is not (0) or is (1) mirrored north/south
-  const int d0 = C.mx ? dew : I, d1 = C.mx ? dboth : dns;
-  const gptr<const TS> pf0 = in.src + (long long)d0 * in.P + C.X, ph0 = in.src + (long long)(kQ + d0) * in.P + C.X;
-  const gptr<const TS> pf1 = in.src + (long long)d1 * in.P + C.X, ph1 = in.src + (long long)(kQ + d1) * in.P + C.X;
-  const bool nsmir = (in.ms | in.mn) != 0;
-  const gptr<const uint8_t> ct = in.ct + C.X;
-  const gptr<const double> al = in.alpha + C.X;
-  // this lane's own cell in the planes it writes (MODE 0, 2: the dF planes
-  // of direction I; MODE 1: the state planes) and, MODE 1, in the planes of
-  // direction I it reads: the stored dF(f2) (FP32 storage: G, in the state
-  // planes it writes)
-  const gptr<TS> of = in.dst + (MODE == 1 ? (long long)I : (long long)(I - 1)) * in.P + C.X;
-  const gptr<TS> oh = in.dst + (MODE == 1 ? (long long)(kQ + I) : (long long)(12 + I - 1)) * in.P + C.X;
-  const gptr<const TS> df2 = kStage3G<TS> ? (gptr<const TS>)of : in.dfl + (long long)(I - 1) * in.P + C.X;
-  const gptr<const TS> dh2 = kStage3G<TS> ? (gptr<const TS>)oh : in.dfl + (long long)(12 + I - 1) * in.P + C.X;
+  gptr<const TS> pf0, ph0, pf1, ph1;
+  gptr<const uint8_t> ct;
+  gptr<const double> al;
+  SPos<TC> W[HY ? 6 : 1];  // rows F - 3 .. F + 2 of the y face F below row F
+  TC Fyf, Fyh;             // the y face below the next row
 
-  auto map_row = [&](int yl, unsigned& my) {
-    if (in.inner) {
-      my = 0;
-      return yl * pitch;
-    }
-    unsigned cy;
-    return map_axis(yl, ny, in.py, in.ms, in.mn, my, cy) * pitch;
-  };
-  auto load = [&](int yl) {
-    unsigned my;
-    const int ro = map_row(prow(yl), my);
-    const bool m = nsmir && my;
+  __device__ __forceinline__ void setup(const StripInst<TS>& in, const StripLane<TC>& C, TC rf_, TC rh_, int I) {
+    const int aex = c_lat_x[I] > 0 ? c_lat_x[I] : -c_lat_x[I];
+    const int aey = c_lat_y[I] > 0 ? c_lat_y[I] : -c_lat_y[I];
+    vx = TC(double(aex) * in.c);
+    vy = TC(double(aey) * in.c);
+    rf = rf_;
+    rh = rh_;
+    const int dew = c_mir_ew[I], dns = c_mir_ns[I], dboth = c_mir_ns[dew];
+    const int d0 = C.mx ? dew : I, d1 = C.mx ? dboth : dns;
+    pf0 = in.src + (long long)d0 * in.P + C.X;
+    ph0 = in.src + (long long)(kQ + d0) * in.P + C.X;
+    pf1 = in.src + (long long)d1 * in.P + C.X;
+    ph1 = in.src + (long long)(kQ + d1) * in.P + C.X;
+    ct = in.ct + C.X;
+    al = in.alpha + C.X;
+    Fyf = Fyh = TC(0);
+  }
+
+  // The staged position of logical row yl (an instance row).
+  __device__ __forceinline__ SPos<TC> load(const StripInst<TS>& in, int yl) const {
+    unsigned my = 0, cy;
+    const int ro = (in.inner ? yl : map_axis(yl, in.ny, in.py, in.ms, in.mn, my, cy)) * in.pitch;
+    const bool m = (in.ms | in.mn) != 0 && my;
     SPos<TC> p;
     p.f = TC((m ? pf1 : pf0)[ro]);
     p.h = TC((m ? ph1 : ph0)[ro]);
     p.type = SOLID ? int(ct[ro]) : 0;
     p.a = SOLID ? TC(al[ro]) : TC(0);
     return p;
-  };
-  auto clamped_row = [&](int yl) {
+  }
+  static __device__ __forceinline__ int clamped_row(const StripInst<TS>& in, int yl) {
     if (in.inner) return 0;
     unsigned my, cy;
-    (void)map_axis(prow(yl), ny, in.py, in.ms, in.mn, my, cy);
+    (void)map_axis(yl, in.ny, in.py, in.ms, in.mn, my, cy);
     return (int)cy;
-  };
+  }
 
   // x face left of this lane's column at a row: owner lane l - 1 (SX > 0) or
   // l (SX < 0); line owner - 2 sx .. owner + 2 sx across the lanes
-  auto xface = [&](const SPos<TC>& r, TC& vf, TC& vh) {
+  __device__ __forceinline__ void xface(const SPos<TC>& r, TC& vf, TC& vh) const {
     TC Lf[5], Lh[5];
     int sld[5] = {0, 0, 0, 0, 0};
     if constexpr (SX > 0) {
@@ -247,11 +248,11 @@ __device__ __forceinline__ void strip_dir(const StripInst<TS>& in, const StripLa
       }
     }
     strip_line<TC, SOLID, W5>(vx, Lf, Lh, sld, vf, vh);
-  };
+  }
 
   // y face F below the window's row F (window rows F - 3 .. F + 2): owner
   // row F - 1 (SY > 0, window 2) or F (SY < 0, window 3)
-  auto yface = [&](const SPos<TC> (&W)[6], TC& vf, TC& vh) {
+  __device__ __forceinline__ void yface(TC& vf, TC& vh) const {
     TC Lf[5], Lh[5];
     int sld[5];
 #pragma unroll
@@ -268,69 +269,42 @@ __device__ __forceinline__ void strip_dir(const StripInst<TS>& in, const StripLa
       }
     }
     strip_line<TC, SOLID, W5>(vy, Lf, Lh, sld, vf, vh);
-  };
-
-  // Everything a row needs from memory, loaded one row ahead: the staged
-  // position entering the window (row y + 3; row y itself without a y
-  // component), the own cell's type as loaded (0 fluid; 1 for lanes without
-  // an own cell), its row offset, (MODE 1) its stored dF(f2) (FP32
-  // storage: G), and dt/dy
-  // of the row (on a uniform grid the instance's own value, read with
-  // stride 0, so that every row issues the same loads).
-  struct Pre {
-    SPos<TC> p;
-    int ro, type;
-    TS f, h;
-    TC rdy;
-  };
-  auto fetch = [&](int y) {
-    Pre r;
-    r.p = load(HY ? y + 3 : y);
-    r.ro = prow(y) * pitch;
-    r.type = 1;
-    r.f = r.h = TS(0);
-    if (C.own) {
-      r.type = ct[r.ro];
-      if (MODE == 1) {
-        r.f = df2[r.ro];
-        r.h = dh2[r.ro];
-      }
-    }
-    r.rdy = TC(in.rdyp[prow(y) * in.rdy_stride]);
-    return r;
-  };
-  // a row's results, stored at the start of the next half iteration
-  struct Res {
-    int ro, on;
-    TS vf, vh;
-  };
-  auto store = [&](const Res& r) {
-    if (r.on) {
-      of[r.ro] = r.vf;
-      oh[r.ro] = r.vh;
-    }
-  };
-
-  SPos<TC> W[6];  // window rows F - 3 .. F + 2 of the y face F below row F
-  TC Fyf = 0, Fyh = 0;
-  if constexpr (HY) {
-#pragma unroll
-    for (int k = 0; k < 6; k++) W[k] = load(y0 - 3 + k);
   }
-  // row y from its prefetched data (registers only: no memory access)
-  auto row = [&](int y, const Pre& cc) {
-    // no contraction: the net flux and the state update round as the tile
-    // kernels (and the oracle) round them, so both paths agree bit for bit
+
+  // Fills the window for row y0 (call first_face once the loads have landed).
+  __device__ __forceinline__ void fill(const StripInst<TS>& in, const RowOrder& ro, int y0) {
+    if constexpr (HY) {
+#pragma unroll
+      for (int k = 0; k < 6; k++) W[k] = load(in, ro(y0 - 3 + k));
+    }
+  }
+  __device__ __forceinline__ void first_face() {
+    if constexpr (HY) yface(Fyf, Fyh);
+  }
+  // The position row y of the march needs from memory: the one entering the
+  // window (row y + 3), without a y component row y itself.
+  __device__ __forceinline__ SPos<TC> next(const StripInst<TS>& in, const RowOrder& ro, int y) const {
+    return load(in, ro(HY ? y + 3 : y));
+  }
+
+  // Net flux of row y's cell from its prefetched position (registers only:
+  // no memory access); own: the cell's staged values. No contraction: the net
+  // flux rounds as the tile kernels (and the oracle) round it, so both paths
+  // agree bit for bit.
+  __device__ __forceinline__ void net(const StripInst<TS>& in, const StripLane<TC>& C, const RowOrder& ro, int y,
+                                      const SPos<TC>& p, TC rdy, TC& dF, TC& dH, TC& ownf, TC& ownh) {
 #pragma clang fp contract(off)
     TC Gf = 0, Gh = 0, Ff = 0, Fh = 0, Nf = 0, Nh = 0;
-    SPos<TC> xr = cc.p;
+    SPos<TC> xr = p;
     if constexpr (HY) {
 #pragma unroll
       for (int k = 0; k < 5; k++) W[k] = W[k + 1];
-      W[5] = cc.p;
-      yface(W, Gf, Gh);  // face above row y
+      W[5] = p;
+      yface(Gf, Gh);  // face above row y
       xr = W[2];
     }
+    ownf = xr.f;
+    ownh = xr.h;
     if constexpr (HX) {
       xface(xr, Ff, Fh);
       Nf = lane_shift<kDppShl1>(Ff);  // face right of the column
@@ -352,41 +326,98 @@ __device__ __forceinline__ void strip_dir(const StripInst<TS>& in, const StripLa
       oyh = SY > 0 ? Gh : Fyh;
       iyf = SY > 0 ? Fyf : Gf;
       iyh = SY > 0 ? Fyh : Gh;
-      if (clamped_row(y - SY)) {
+      if (clamped_row(in, ro(y - SY))) {
         iyf = oyf;
         iyh = oyh;
       }
       Fyf = Gf;
       Fyh = Gh;
     }
-    TC dF, dH;
     if constexpr (HX && HY) {
-      dF = (C.rdx * oxf + cc.rdy * oyf) - (C.rdx * ixf + cc.rdy * iyf);
-      dH = (C.rdx * oxh + cc.rdy * oyh) - (C.rdx * ixh + cc.rdy * iyh);
+      dF = (C.rdx * oxf + rdy * oyf) - (C.rdx * ixf + rdy * iyf);
+      dH = (C.rdx * oxh + rdy * oyh) - (C.rdx * ixh + rdy * iyh);
     } else if constexpr (HX) {
       dF = C.rdx * oxf - C.rdx * ixf;
       dH = C.rdx * oxh - C.rdx * ixh;
     } else {
-      dF = cc.rdy * oyf - cc.rdy * iyf;
-      dH = cc.rdy * oyh - cc.rdy * iyh;
+      dF = rdy * oyf - rdy * iyf;
+      dH = rdy * oyh - rdy * iyh;
     }
+  }
+};
+
+// One direction over the rows of a work item.
+template <typename TS, typename TC, int MODE, bool SOLID, bool W5, int SX, int SY>
+__device__ __forceinline__ void strip_dir(const StripInst<TS>& in, const StripLane<TC>& C, TC rf, TC rh, int I,
+                                          int y0, int nrows, int flip, bool alive) {
+  using M = March<TS, TC, SOLID, W5, SX, SY>;
+  M m;
+  m.setup(in, C, rf, rh, I);
+  const RowOrder ro{flip, 2 * y0 + nrows - 1};
+  const int pitch = in.pitch;
+  // this lane's own cell in the planes it writes (MODE 0, 2: the dF planes
+  // of direction I; MODE 1: the state planes) and, MODE 1, in the planes of
+  // direction I it reads: the stored dF(f2)
+  const gptr<TS> of = in.dst + (MODE == 1 ? (long long)I : (long long)(I - 1)) * in.P + C.X;
+  const gptr<TS> oh = in.dst + (MODE == 1 ? (long long)(kQ + I) : (long long)(12 + I - 1)) * in.P + C.X;
+  const gptr<const TS> df2 = in.dfl + (long long)(I - 1) * in.P + C.X;
+  const gptr<const TS> dh2 = in.dfl + (long long)(12 + I - 1) * in.P + C.X;
+  const gptr<const uint8_t> ct = in.ct + C.X;
+
+  // Everything a row needs from memory, loaded one row ahead: the staged
+  // position, the own cell's type as loaded (0 fluid; 1 for lanes without an
+  // own cell), its row offset, (MODE 1) its stored dF(f2), and dt/dy of the
+  // row (on a uniform grid the instance's own value, read with stride 0, so
+  // that every row issues the same loads).
+  struct Pre {
+    SPos<TC> p;
+    int ro, type;
+    TS f, h;
+    TC rdy;
+  };
+  auto fetch = [&](int y) {
+    Pre r;
+    r.p = m.next(in, ro, y);
+    r.ro = ro(y) * pitch;
+    r.type = 1;
+    r.f = r.h = TS(0);
+    if (C.own) {
+      r.type = ct[r.ro];
+      if (MODE == 1) {
+        r.f = df2[r.ro];
+        r.h = dh2[r.ro];
+      }
+    }
+    r.rdy = TC(in.rdyp[ro(y) * in.rdy_stride]);
+    return r;
+  };
+  // a row's results, stored at the start of the next half iteration
+  struct Res {
+    int ro, on;
+    TS vf, vh;
+  };
+  auto store = [&](const Res& r) {
+    if (r.on) {
+      of[r.ro] = r.vf;
+      oh[r.ro] = r.vh;
+    }
+  };
+  // row y from its prefetched data (registers only: no memory access)
+  auto row = [&](int y, const Pre& cc) {
+#pragma clang fp contract(off)
+    TC dF, dH, of3, oh3;
+    m.net(in, C, ro, y, cc.p, cc.rdy, dF, dH, of3, oh3);
     Res r;
     r.ro = cc.ro;
-    r.on = cc.type == 0;
+    r.on = alive && cc.type == 0;
     if (MODE != 1) {
       r.vf = TS(dF);
       r.vh = TS(dH);
     } else {
-      // the new state f3 + (dF2 - dF3)/2 (FP32 storage: G - dF3/2), the
-      // final combination of the stage-3 kernel; the own cell's f3 is the
-      // staged value of row y
-      if constexpr (kStage3G<TS>) {
-        r.vf = TS(TC(cc.f) - TC(0.5) * dF);
-        r.vh = TS(TC(cc.h) - TC(0.5) * dH);
-      } else {
-        r.vf = TS(xr.f + TC(0.5) * (TC(cc.f) - dF));
-        r.vh = TS(xr.h + TC(0.5) * (TC(cc.h) - dH));
-      }
+      // the new state f3 + (dF2 - dF3)/2, the final combination of the
+      // stage-3 kernel; the own cell's f3 is the staged value of row y
+      r.vf = TS(of3 + TC(0.5) * (TC(cc.f) - dF));
+      r.vh = TS(oh3 + TC(0.5) * (TC(cc.h) - dH));
     }
     return r;
   };
@@ -398,10 +429,11 @@ __device__ __forceinline__ void strip_dir(const StripInst<TS>& in, const StripLa
   // stores the previous row, issues the next row's loads into the other
   // slot and computes its row from registers.
   const int end = y0 + nrows;
+  m.fill(in, ro, y0);
   Pre A = fetch(y0), B;
-  if constexpr (HY) {
+  if constexpr (M::HY) {
     __builtin_amdgcn_s_waitcnt(kWaitVmem);
-    yface(W, Fyf, Fyh);  // face below the first row
+    m.first_face();
   }
   Res R{0, 0, TS(0), TS(0)};
   for (int y = y0;; y += 2) {
@@ -419,50 +451,14 @@ __device__ __forceinline__ void strip_dir(const StripInst<TS>& in, const StripLa
   store(R);
 }
 
-// The twelve directions of a work item, one flux method. desc: the item
-// takes its rows from the last to the first in the directions with a y
-// component. Items alternate between the two orders down each strip column
-// (kStripDesc), so that two items one above the other reach the rows they
-// share (each one's rows next to the other, read by the other as its y
-// halo) at about the same time: the first read of such a row leaves it in
-// L2 for the second.
-template <typename TS, typename TC, int MODE, bool SOLID, bool W5>
-__device__ __forceinline__ void strip_dirs(const InstDev& in, const StripInst<TS>& si, const StripLane<TC>& C, int y0,
-                                           int nrows, bool desc) {
-  for (int I = 1; I < kQ; I++) {
-    const int sx = c_lat_x[I] > 0 ? 1 : (c_lat_x[I] < 0 ? -1 : 0);
-    const int sy0 = c_lat_y[I] > 0 ? 1 : (c_lat_y[I] < 0 ? -1 : 0);
-    const int fl = desc && sy0 != 0;
-    const int sy = fl ? -sy0 : sy0;  // the sign in the march's row order
-    // reference equilibrium of direction I for the wall faces of FP32
-    // storage (a mirror image of I has the same reference: it depends on |e|)
-    const TC rf = sizeof(TS) == 4 ? TC(in.ref[I]) : TC(0);
-    const TC rh = sizeof(TS) == 4 ? TC(in.ref[kQ + I]) : TC(0);
-    if (sy == 0) {
-      if (sx > 0) strip_dir<TS, TC, MODE, SOLID, W5, 1, 0>(si, C, rf, rh, I, y0, nrows, 0);
-      else strip_dir<TS, TC, MODE, SOLID, W5, -1, 0>(si, C, rf, rh, I, y0, nrows, 0);
-    } else if (sx == 0) {
-      if (sy > 0) strip_dir<TS, TC, MODE, SOLID, W5, 0, 1>(si, C, rf, rh, I, y0, nrows, fl);
-      else strip_dir<TS, TC, MODE, SOLID, W5, 0, -1>(si, C, rf, rh, I, y0, nrows, fl);
-    } else if (sy > 0) {
-      if (sx > 0) strip_dir<TS, TC, MODE, SOLID, W5, 1, 1>(si, C, rf, rh, I, y0, nrows, fl);
-      else strip_dir<TS, TC, MODE, SOLID, W5, -1, 1>(si, C, rf, rh, I, y0, nrows, fl);
-    } else {
-      if (sx > 0) strip_dir<TS, TC, MODE, SOLID, W5, 1, -1>(si, C, rf, rh, I, y0, nrows, fl);
-      else strip_dir<TS, TC, MODE, SOLID, W5, -1, -1>(si, C, rf, rh, I, y0, nrows, fl);
-    }
-  }
-}
-
-// All twelve directions of one work item.
-template <typename TS, typename TC, int MODE, bool SOLID>
-__device__ __forceinline__ void strip_item(const InstDev& in, const TileRef& sr, int par) {
+// The instance fields and lane constants of a work item.
+template <typename TS, typename TC>
+__device__ __forceinline__ void strip_setup(const InstDev& in, const TileRef& sr, const void* src, void* dst,
+                                            StripInst<TS>& si, StripLane<TC>& C) {
   const int lane = threadIdx.x & 63;
-  const int x0 = sr.tx * kStripW, y0 = sr.ty, nrows = sr.flags >> 8;
-  const bool desc = (sr.flags & kStripDesc) != 0;
-  StripInst<TS> si;
-  si.src = (gptr<const TS>)(MODE == 0 ? in.f2 : (MODE == 1 ? in.f3 : in.state[in.parity0 ^ par]));
-  si.dst = (gptr<TS>)(MODE == 1 ? in.state[1 ^ in.parity0 ^ par] : in.dflux);
+  const int x0 = sr.tx * kStripW, y0 = sr.ty, nrows = sr.flags >> kStripRowsBit;
+  si.src = (gptr<const TS>)src;
+  si.dst = (gptr<TS>)dst;
   si.dfl = (gptr<const TS>)in.dflux;
   si.ct = (gptr<const uint8_t>)in.ctype;
   si.alpha = (gptr<const double>)in.alpha;
@@ -476,7 +472,6 @@ __device__ __forceinline__ void strip_item(const InstDev& in, const TileRef& sr,
   si.mn = in.flags & kMirrorN;
   si.inner = y0 - kH >= 0 && y0 + nrows + kH <= in.ny;
   si.c = in.c;
-  StripLane<TC> C;
   C.xl = x0 - kH + lane;
   const int px = in.flags & kPeriodicX, mw = in.flags & kMirrorW, me = in.flags & kMirrorE;
   unsigned mx, cx, mt, cl, cr;
@@ -488,26 +483,69 @@ __device__ __forceinline__ void strip_item(const InstDev& in, const TileRef& sr,
   C.clampR = (int)cr;
   C.own = lane >= kH && lane < kH + kStripW && C.xl < in.nx;
   C.rdx = C.own ? TC(in.rdxs ? in.rdxs[C.xl] : in.rdx) : TC(0);
-  if (in.flux_method == 1) strip_dirs<TS, TC, MODE, SOLID, true>(in, si, C, y0, nrows, desc);
-  else strip_dirs<TS, TC, MODE, SOLID, false>(in, si, C, y0, nrows, desc);
 }
 
-// Persistent grid of 4-wave blocks; wave w of the (XCD-renumbered) grid
-// takes items w, w + 4 G, ... of the list. At most 168 registers (3 waves
-// per SIMD): capped at 128 for a fourth wave the FP64 kernels spill (up to
-// 73 slots) and run slower (4096^2 Riemann stage-2 and stage-3 flux 2.19
-// and 2.82 ms at 4 waves, 1.77 and 2.18 ms at 3).
-template <typename TS, typename TC, int MODE, bool SOLID>
+// One direction of a work item. desc: the item takes its rows from the last
+// to the first in the directions with a y component. Items alternate between
+// the two orders down each strip column (kStripDesc), so that two items one
+// above the other reach the rows they share (each one's rows next to the
+// other, read by the other as its y halo) at about the same time: the first
+// read of such a row leaves it in L2 for the second.
+template <typename TS, typename TC, int MODE, bool SOLID, bool W5>
+__device__ __forceinline__ void strip_item(const InstDev& in, const StripInst<TS>& si, const StripLane<TC>& C,
+                                           const TileRef& sr, int I, bool alive) {
+  const int y0 = sr.ty, nrows = sr.flags >> kStripRowsBit;
+  const int sx = c_lat_x[I] > 0 ? 1 : (c_lat_x[I] < 0 ? -1 : 0);
+  const int sy0 = c_lat_y[I] > 0 ? 1 : (c_lat_y[I] < 0 ? -1 : 0);
+  const int fl = (sr.flags & kStripDesc) != 0 && sy0 != 0;
+  const int sy = fl ? -sy0 : sy0;  // the sign in the march's row order
+  const TC rf = sizeof(TS) == 4 ? TC(in.ref[I]) : TC(0);
+  const TC rh = sizeof(TS) == 4 ? TC(in.ref[kQ + I]) : TC(0);
+  if (sy == 0) {
+    if (sx > 0) strip_dir<TS, TC, MODE, SOLID, W5, 1, 0>(si, C, rf, rh, I, y0, nrows, 0, alive);
+    else strip_dir<TS, TC, MODE, SOLID, W5, -1, 0>(si, C, rf, rh, I, y0, nrows, 0, alive);
+  } else if (sx == 0) {
+    if (sy > 0) strip_dir<TS, TC, MODE, SOLID, W5, 0, 1>(si, C, rf, rh, I, y0, nrows, fl, alive);
+    else strip_dir<TS, TC, MODE, SOLID, W5, 0, -1>(si, C, rf, rh, I, y0, nrows, fl, alive);
+  } else if (sy > 0) {
+    if (sx > 0) strip_dir<TS, TC, MODE, SOLID, W5, 1, 1>(si, C, rf, rh, I, y0, nrows, fl, alive);
+    else strip_dir<TS, TC, MODE, SOLID, W5, -1, 1>(si, C, rf, rh, I, y0, nrows, fl, alive);
+  } else {
+    if (sx > 0) strip_dir<TS, TC, MODE, SOLID, W5, 1, -1>(si, C, rf, rh, I, y0, nrows, fl, alive);
+    else strip_dir<TS, TC, MODE, SOLID, W5, -1, -1>(si, C, rf, rh, I, y0, nrows, fl, alive);
+  }
+}
+
+// Directions in the order a chunk of items takes them: the four with both
+// components, which cost twice the others, first.
+static __constant__ int c_strip_dir[12] = {5, 6, 7, 8, 2, 4, 10, 12, 1, 3, 9, 11};
+
+// One wavefront per work item and direction, four items of one direction per
+// workgroup. The items (in memory order) are cut into one contiguous chunk
+// per XCD, whose blocks take the chunk direction by direction: neighbouring
+// strips of a direction run together and share their halos in that XCD's L2.
+template <typename TS, typename TC, int MODE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_strip(
-    const InstDev* __restrict__ insts, const TileRef* __restrict__ strips, int nstrips, int par, const int* stepp) {
+    const InstDev* __restrict__ insts, const TileRef* __restrict__ strips, int nstrips, int chunk, int all, int par,
+    const int* stepp) {
   const int step = *stepp;
-  const int wave = __builtin_amdgcn_readfirstlane(first_tile() * 4 + (int)(threadIdx.x >> 6));
-  const int nw = gridDim.x * 4;
-  for (int it = wave; it < nstrips; it += nw) {
-    const TileRef sr = strips[it];
-    const InstDev& in = insts[sr.inst];
-    if (frozen_by_failure(in, step)) continue;
-    if (!eq_kernel_for<TS, TC>(in)) continue;  // FP32 storage: the other compute type's instance
-    strip_item<TS, TC, MODE, SOLID>(in, sr, par);
+  const int per = chunk / 4, b = blockIdx.x / 8;
+  const int I = c_strip_dir[b / per];
+  const int it = __builtin_amdgcn_readfirstlane((int)(blockIdx.x % 8) * chunk + (b % per) * 4 + (int)(threadIdx.x >> 6));
+  if (it >= nstrips) return;
+  const TileRef sr = strips[it];
+  const InstDev& in = insts[sr.inst];
+  if (!all && !eq_kernel_for<TS, TC>(in)) return;  // FP32 storage: the other compute type's instance
+  const bool alive = !frozen_by_failure(in, step);
+  StripInst<TS> si;
+  StripLane<TC> C;
+  const void* src = MODE == 0 ? in.f2 : (MODE == 1 ? in.f3 : in.state[in.parity0 ^ par]);
+  strip_setup<TS, TC>(in, sr, src, MODE == 1 ? in.state[1 ^ in.parity0 ^ par] : in.dflux, si, C);
+  if (sr.flags & kTileSolid) {
+    if (in.flux_method == 1) strip_item<TS, TC, MODE, true, true>(in, si, C, sr, I, alive);
+    else strip_item<TS, TC, MODE, true, false>(in, si, C, sr, I, alive);
+  } else {
+    if (in.flux_method == 1) strip_item<TS, TC, MODE, false, true>(in, si, C, sr, I, alive);
+    else strip_item<TS, TC, MODE, false, false>(in, si, C, sr, I, alive);
   }
 }

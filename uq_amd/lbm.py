@@ -122,8 +122,9 @@ def set_graphs(enable: bool) -> None:
 
 def set_strips(mode) -> None:
     """Flux kernels of instances with logical addressing: 0 (or False) tiles
-    only, 1 (or True; default) strips for launch groups large enough to fill
-    the GPU, 2 strips wherever possible."""
+    only, 1 (or True; default) and 2 strips wherever possible (2: FP64
+    stencils in strips of mixed-precision instances far from their reference
+    equilibrium also in small launch groups)."""
     mode = int(mode)
     _check(lib().lbm_set_strips(mode), "lbm_set_strips")
 
