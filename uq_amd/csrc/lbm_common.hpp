@@ -91,7 +91,7 @@ struct InstDev {
   int res_last;
   int ptile0, nptiles;
   // the group's strip list holds this instance: the tile flux kernels skip
-  // its tiles, except the moment-summing stage-3 flux of FP32 storage
+  // its tiles
   int strips;
 };
 

@@ -1345,7 +1345,7 @@ __device__ __forceinline__ void flux_tiles(const InstDev* insts, const TileRef* 
     const InstDev& in = insts[tr.inst];
     if (frozen_by_failure(in, step)) continue;
     if (tr.flags & kTilePhysical) continue;  // k_phys forms this tile's net fluxes
-    if (!MOM && in.strips) continue;         // the strip kernels form this instance's net fluxes
+    if (in.strips) continue;                 // the strip kernels form this instance's net fluxes
     __syncthreads();
     setup_region(R, in, tr.tx * Sh::TX, tr.ty * Sh::TY);
     __syncthreads();
@@ -1782,18 +1782,16 @@ static void launch_phys(const StepLaunch& L, hipStream_t s, int par) {
 }
 
 // One flux stage of MODE: the strip kernels for the instances on strips and
-// the tile kernel for the others (every instance for the moment-summing
-// stage-3 flux of FP32 storage, which has no strip form), then the
-// physical-addressing net fluxes of flagged tiles.
+// the tile kernel for the others, then the physical-addressing net fluxes of
+// flagged tiles.
 template <typename TS, typename TC, int MODE, bool MOM, typename Sh>
 static void launch_flux(const StepLaunch& L, hipStream_t s, int par, int grid_tiles) {
   const int* step = L.step_ctr;
-  bool tiles = true;
-  if constexpr (!MOM) {
-    if (L.nstrips > 0) launch_strips<TS, MODE>(L, s, par);
-    tiles = L.tiles_rest > 0;
+  if (L.nstrips > 0) {
+    if constexpr (MOM) launch_strips_mom(L, s, par);
+    else launch_strips<TS, MODE>(L, s, par);
   }
-  if (tiles)
+  if (L.tiles_rest > 0)
     FluxKernel<TS, TC, MODE, MOM, Sh>::fn<<<blocks_for(L.ntiles, grid_tiles), Sh::NT, 0, s>>>(L.insts, L.tiles,
                                                                                              L.ntiles, par, step);
   launch_phys<TS, TC, MODE, MOM, Sh>(L, s, par);

@@ -32,6 +32,8 @@ struct StepLaunch {
                                     // bit 1 FP32 (deviation form; FP32 storage only)
   const TileRef* strips = nullptr;  // strip work items (instances with InstDev::strips set)
   int nstrips = 0;
+  const TileRef* mstrips = nullptr;  // FP32 storage: strip items of the moment-summing stage-3 flux
+  int nmstrips = 0;
   int far64 = 0;                    // FP32 storage far from its reference: FP64 stencils on strips
   int tiles_rest = 0;               // flux tiles of the instances not on strips
 };
@@ -58,7 +60,8 @@ inline bool same_launch(const StepLaunch& a, const StepLaunch& b) {
          a.nwalls == b.nwalls && a.ptiles == b.ptiles && a.nptiles == b.nptiles && a.rk_method == b.rk_method &&
          a.step_ctr == b.step_ctr && a.flux_shape == b.flux_shape && a.res_partial == b.res_partial && a.ninst == b.ninst &&
          a.nphys == b.nphys && a.eq_kinds == b.eq_kinds && a.strips == b.strips && a.nstrips == b.nstrips &&
-         a.far64 == b.far64 && a.tiles_rest == b.tiles_rest;
+         a.mstrips == b.mstrips && a.nmstrips == b.nmstrips && a.far64 == b.far64 &&
+         a.tiles_rest == b.tiles_rest;
 }
 
 // Optional per-kernel timing with HIP events recorded on the launch stream
@@ -120,11 +123,12 @@ constexpr int kPointW = 64, kPointH = 4;  // pointwise tile: 64 x 4 cells, 256 t
 template <typename TS, typename TC>
 void launch_step(const StepLaunch& L, hipStream_t s, int par, KernelTimer* tm);
 
-// The strip flux kernels of one flux stage (MODE 0, 1, 2 of k_strip) and the
-// wall closure of the distributions `which` (0: f2 or f1, 1: f3, 2: the
+// The strip flux kernels of one flux stage (MODE 0, 1, 2 of k_strip; k_strip_mom:
+// stage 3 of FP32 storage) and the wall closure of the distributions `which` (0: f2 or f1, 1: f3, 2: the
 // current state).
 template <typename TS, int MODE>
 void launch_strips(const StepLaunch& L, hipStream_t s, int par);
+void launch_strips_mom(const StepLaunch& L, hipStream_t s, int par);
 template <typename TS>
 void launch_alpha(const StepLaunch& L, hipStream_t s, int which, int par);
 

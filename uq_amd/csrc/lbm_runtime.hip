@@ -668,16 +668,32 @@ static int strip_rows(const std::vector<Solver*>& members, int waves) {
   return h;
 }
 
-void uqlbm::group_strips(const std::vector<Solver*>& members, int shape, std::vector<TileRef>& out, int* blocks,
-                         int* tiles_rest) {
-  out.clear();
-  *blocks = *tiles_rest = 0;
+uqlbm::StripLists::StripLists(const std::vector<Solver*>& members, int shape) {
   const int rows = strip_rows(members, 12);
   for (size_t k = 0; k < members.size(); k++) {
-    strip_items(*members[k], rows, (int)k, out);
-    *blocks += members[k]->strip_blocks;
-    if (members[k]->strip_cols == 0) *tiles_rest += (int)solver_tiles(*members[k], shape).size();
+    strip_items(*members[k], rows, (int)k, items);
+    blocks += members[k]->strip_blocks;
+    if (members[k]->strip_cols == 0) tiles_rest += (int)solver_tiles(*members[k], shape).size();
   }
+  n = (int)items.size();
+  if (members.empty() || members[0]->precision == LBM_PREC_FP64) return;
+  const int mrows = strip_rows(members, 4);
+  for (size_t k = 0; k < members.size(); k++) strip_items(*members[k], mrows, (int)k, items);
+  nmom = (int)items.size() - n;
+}
+
+void uqlbm::launch_strips_of(StepLaunch& L, const TileRef* items_dev, int n, int nmom, int blocks, int tiles_rest,
+                             int ntiles) {
+  if (!strips_enabled() || n == 0) {
+    L.tiles_rest = ntiles;
+    return;
+  }
+  L.strips = items_dev;
+  L.nstrips = n;
+  L.mstrips = items_dev + n;
+  L.nmstrips = nmom;
+  L.far64 = far_fp64(blocks);
+  L.tiles_rest = tiles_rest;
 }
 
 const std::vector<TileRef>& uqlbm::solver_tiles(Solver& s, int shape) {
@@ -837,13 +853,12 @@ extern "C" int lbm_create(const lbm_params* params, int32_t nx, int32_t ny, cons
   s->walls_host = std::move(walls);
   s->ptiles_host = std::move(ptiles);
   mark_strips(*s);
-  std::vector<TileRef> strips;
-  int blocks = 0, rest = 0;
-  group_strips({s.get()}, s->flux_shape, strips, &blocks, &rest);
-  s->nstrips = (int)strips.size();
+  const StripLists strips({s.get()}, s->flux_shape);
+  s->nstrips = strips.n;
+  s->nmstrips = strips.nmom;
   if (s->nstrips) {
-    HIP_TRY(solver_alloc(*s, (void**)&s->strips_dev, strips.size() * sizeof(TileRef)));
-    HIP_TRY(hipMemcpy(s->strips_dev, strips.data(), strips.size() * sizeof(TileRef), hipMemcpyHostToDevice));
+    HIP_TRY(solver_alloc(*s, (void**)&s->strips_dev, strips.items.size() * sizeof(TileRef)));
+    HIP_TRY(hipMemcpy(s->strips_dev, strips.items.data(), strips.items.size() * sizeof(TileRef), hipMemcpyHostToDevice));
   }
   const int st = upload_inst(*s);
   if (st != LBM_OK) return st;
@@ -1037,18 +1052,6 @@ int uqlbm::run_group(const std::vector<Solver*>& members, InstDev* table_dev, co
 
 // Residual of the solver's last step on the device (cpuLBM.cpp:2322-2331):
 // `rows` holds ny + 1 doubles; the result is copied to *out.
-// The solver's strip list in its launch description (when strips are on).
-static void solver_strips(const Solver& s, StepLaunch& L) {
-  if (strips_enabled() && s.nstrips > 0) {
-    L.strips = s.strips_dev;
-    L.nstrips = s.nstrips;
-    L.far64 = far_fp64(s.strip_blocks);
-    L.tiles_rest = 0;
-  } else {
-    L.tiles_rest = s.ntiles;
-  }
-}
-
 static int device_residual(Solver& s, double* rows, double* out) {
   if (s.precision == LBM_PREC_FP64) launch_residual<double>(s.inst_dev, 0, 0, rows, s.nx, s.ny, s.stream);
   else launch_residual<float>(s.inst_dev, 0, 0, rows, s.nx, s.ny, s.stream);
@@ -1068,7 +1071,7 @@ extern "C" int lbm_step(lbm_solver* h, int32_t nsteps, int32_t want_residual, do
   StepLaunch L{s.inst_dev,    s.tiles_dev, s.ntiles,      s.walls_dev, s.nwalls,
                s.ptiles_dev, s.nptiles,   s.p.rk_method, s.step_ctr,  s.flux_shape};
   L.nphys = s.nphys;
-  solver_strips(s, L);
+  launch_strips_of(L, s.strips_dev, s.nstrips, s.nmstrips, s.strip_blocks, 0, s.ntiles);
   L.eq_kinds = s.precision == LBM_PREC_FP64 ? 1 : (s.eq32 ? 2 : 1);
   std::vector<Solver*> one{&s};
   const int st = run_group(one, s.inst_dev, L, s.precision, s.stream, nsteps, s.graphs.get(), s.fails_dev, true);
@@ -1137,7 +1140,7 @@ extern "C" int lbm_step_noalloc(lbm_solver* h, int32_t nsteps, int32_t want_resi
   StepLaunch L{s.inst_dev,    s.tiles_dev, s.ntiles,      s.walls_dev, s.nwalls,
                s.ptiles_dev, s.nptiles,   s.p.rk_method, s.step_ctr,  s.flux_shape};
   L.nphys = s.nphys;
-  solver_strips(s, L);
+  launch_strips_of(L, s.strips_dev, s.nstrips, s.nmstrips, s.strip_blocks, 0, s.ntiles);
   L.eq_kinds = s.precision == LBM_PREC_FP64 ? 1 : (s.eq32 ? 2 : 1);
   prepare_launch(s.precision == LBM_PREC_FP64);
   std::vector<Solver*> one{&s};
@@ -1476,12 +1479,14 @@ int uqlbm::batch_finish(Batch& b, lbm_batch** out) {
   }
   HIP_TRY(hipMalloc((void**)&b.ptiles_dev, ptiles.size() * sizeof(TileRef)));
   HIP_TRY(hipMemcpy(b.ptiles_dev, ptiles.data(), ptiles.size() * sizeof(TileRef), hipMemcpyHostToDevice));
-  std::vector<TileRef> strips;
-  group_strips(b.members, b.flux_shape, strips, &b.strip_blocks, &b.tiles_rest);
-  b.nstrips = (int)strips.size();
-  if (!strips.empty()) {
-    HIP_TRY(hipMalloc((void**)&b.strips_dev, strips.size() * sizeof(TileRef)));
-    HIP_TRY(hipMemcpy(b.strips_dev, strips.data(), strips.size() * sizeof(TileRef), hipMemcpyHostToDevice));
+  const StripLists strips(b.members, b.flux_shape);
+  b.nstrips = strips.n;
+  b.nmstrips = strips.nmom;
+  b.strip_blocks = strips.blocks;
+  b.tiles_rest = strips.tiles_rest;
+  if (b.nstrips) {
+    HIP_TRY(hipMalloc((void**)&b.strips_dev, strips.items.size() * sizeof(TileRef)));
+    HIP_TRY(hipMemcpy(b.strips_dev, strips.items.data(), strips.items.size() * sizeof(TileRef), hipMemcpyHostToDevice));
   }
   *out = reinterpret_cast<lbm_batch*>(new Batch(std::move(b)));
   return LBM_OK;
@@ -1502,14 +1507,7 @@ int uqlbm::batch_step(Batch& b, int nsteps) {
                b.ptiles_dev, b.nptiles,   b.rk_method, b.step_ctr,  b.flux_shape};
   L.nphys = b.nphys;
   L.eq_kinds = b.eq_kinds;
-  if (strips_enabled() && b.nstrips > 0) {
-    L.strips = b.strips_dev;
-    L.nstrips = b.nstrips;
-    L.far64 = far_fp64(b.strip_blocks);
-    L.tiles_rest = b.tiles_rest;
-  } else {
-    L.tiles_rest = b.ntiles;
-  }
+  launch_strips_of(L, b.strips_dev, b.nstrips, b.nmstrips, b.strip_blocks, b.tiles_rest, b.ntiles);
   int st = run_group(b.members, b.inst_dev, L, b.precision, b.stream, nsteps, b.graphs.get(), b.fails_dev, true);
   for (Solver* s : b.members) {
     int st2 = upload_inst(*s);

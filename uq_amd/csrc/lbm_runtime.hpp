@@ -93,7 +93,7 @@ struct Solver {
   std::vector<std::pair<void*, size_t>> owned;  // buffers from solver_alloc, returned to its cache
   int ntiles = 0, nwalls = 0, nptiles = 0;
   int nphys = 0;  // flux tiles flagged kTilePhysical
-  int nstrips = 0;
+  int nstrips = 0, nmstrips = 0;    // items of k_strip, then of k_strip_mom in strips_dev
   size_t device_bytes = 0;
 
   int cur = 0;    // state buffer holding the current state
@@ -125,7 +125,7 @@ struct Batch {
   int ntiles = 0, nwalls = 0, nptiles = 0;
   int nphys = 0;  // flux tiles flagged kTilePhysical
   int eq_kinds = 1;  // equilibrium precisions among the members (StepLaunch::eq_kinds)
-  int nstrips = 0, strip_blocks = 0, tiles_rest = 0;
+  int nstrips = 0, nmstrips = 0, strip_blocks = 0, tiles_rest = 0;
   Batch() = default;
   Batch(Batch&& o) noexcept { *this = std::move(o); }
   Batch& operator=(Batch&& o) noexcept {
@@ -149,6 +149,7 @@ struct Batch {
     nphys = o.nphys;
     eq_kinds = o.eq_kinds;
     nstrips = o.nstrips;
+    nmstrips = o.nmstrips;
     strip_blocks = o.strip_blocks;
     tiles_rest = o.tiles_rest;
     o.stream = nullptr;
@@ -174,11 +175,17 @@ hipError_t solver_alloc(Solver& s, void** p, size_t bytes);
 // stencils in a launch group of `blocks` 32-row strip items.
 bool strips_enabled();
 bool far_fp64(int blocks);
-// Strip list of a launch group (member k's items with instance index k), the
-// group's 32-row strip items, and the number of flux tiles of shape `shape`
-// of the members not on strips.
-void group_strips(const std::vector<Solver*>& members, int shape, std::vector<TileRef>& out, int* blocks,
-                  int* tiles_rest);
+// Strip items of a launch group (member k's with instance index k): `items`
+// holds those of k_strip and then (FP32 storage) those of k_strip_mom.
+struct StripLists {
+  std::vector<TileRef> items;
+  int n = 0, nmom = 0;  // items of k_strip, of k_strip_mom
+  int blocks = 0;       // the group's 32-row strip items
+  int tiles_rest = 0;   // flux tiles of shape `shape` of the members not on strips
+  StripLists(const std::vector<Solver*>& members, int shape);
+};
+// The strip fields of a launch description; `ntiles`: the group's flux tiles.
+void launch_strips_of(StepLaunch& L, const TileRef* items_dev, int n, int nmom, int blocks, int tiles_rest, int ntiles);
 const std::vector<TileRef>& solver_tiles(Solver& s, int shape);
 int default_flux_shape(int precision);
 int batch_set_shape(Batch& b, int shape);

@@ -68,7 +68,7 @@ struct Server {
   TileRef* strips_dev = nullptr;
   size_t tiles_cap = 0, walls_cap = 0, ptiles_cap = 0, strips_cap = 0;
   int ntiles = 0, nwalls = 0, nptiles = 0;
-  int nstrips = 0, strip_blocks = 0, tiles_rest = 0;  // strip list of the active requests (StepLaunch)
+  int nstrips = 0, nmstrips = 0, strip_blocks = 0, tiles_rest = 0;  // strip list of the active requests (StepLaunch)
   int nphys = 0;  // flux tiles flagged kTilePhysical
   int eq_kinds = 1;  // equilibrium precisions among the active requests (StepLaunch::eq_kinds)
   bool lists_dirty = true;
@@ -134,17 +134,19 @@ static int rebuild_lists(Server& sv) {
   std::vector<Solver*> members;
   members.reserve(sv.active.size());
   for (auto& a : sv.active) members.push_back(a.solver);
-  std::vector<TileRef> strips;
-  group_strips(members, sv.flux_shape, strips, &sv.strip_blocks, &sv.tiles_rest);
-  sv.nstrips = (int)strips.size();
-  if (strips.size() > sv.strips_cap) {
+  const StripLists strips(members, sv.flux_shape);
+  sv.nstrips = strips.n;
+  sv.nmstrips = strips.nmom;
+  sv.strip_blocks = strips.blocks;
+  sv.tiles_rest = strips.tiles_rest;
+  if (strips.items.size() > sv.strips_cap) {
     if (sv.strips_dev) SV_TRY(hipFree(sv.strips_dev));
-    sv.strips_cap = std::max(strips.size(), sv.strips_cap * 2);
+    sv.strips_cap = std::max(strips.items.size(), sv.strips_cap * 2);
     SV_TRY(hipMalloc((void**)&sv.strips_dev, sv.strips_cap * sizeof(TileRef)));
   }
-  if (!strips.empty())
-    SV_TRY(hipMemcpyAsync(sv.strips_dev, strips.data(), strips.size() * sizeof(TileRef), hipMemcpyHostToDevice,
-                          sv.stream));
+  if (sv.nstrips)
+    SV_TRY(hipMemcpyAsync(sv.strips_dev, strips.items.data(), strips.items.size() * sizeof(TileRef),
+                          hipMemcpyHostToDevice, sv.stream));
   if (ptiles.size() > sv.ptiles_cap) {
     if (sv.ptiles_dev) SV_TRY(hipFree(sv.ptiles_dev));
     if (sv.res_partial) SV_TRY(hipFree(sv.res_partial));
@@ -365,14 +367,7 @@ extern "C" int lbm_server_tick(lbm_server* h, int32_t tick_steps, int32_t* activ
                  sv.ptiles_dev, sv.nptiles,   sv.rk_method, sv.step_ctr,  sv.flux_shape};
     L.nphys = sv.nphys;
     L.eq_kinds = sv.eq_kinds;
-    if (strips_enabled() && sv.nstrips > 0) {
-      L.strips = sv.strips_dev;
-      L.nstrips = sv.nstrips;
-      L.far64 = far_fp64(sv.strip_blocks);
-      L.tiles_rest = sv.tiles_rest;
-    } else {
-      L.tiles_rest = sv.ntiles;
-    }
+    launch_strips_of(L, sv.strips_dev, sv.nstrips, sv.nmstrips, sv.strip_blocks, sv.tiles_rest, sv.ntiles);
     if (track) {
       L.res_partial = sv.res_partial;
       L.ninst = (int)members.size();

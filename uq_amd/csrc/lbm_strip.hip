@@ -1,5 +1,7 @@
 // lbm_strip.hip — strip flux kernels (lbm_strip.hpp) and the wall closure
 // kernel of the D2Q13 thermal FD-LBM, with their launchers.
+#include <type_traits>
+
 #include "lbm_stencil.hpp"
 
 namespace uqlbm {
@@ -103,6 +105,12 @@ void launch_strips(const StepLaunch& L, hipStream_t s, int par) {
   } else {
     launch_strips_as<TS, double, MODE>(L, s, par, 1);
   }
+}
+
+// Stage-3 flux of FP32 storage: FP32 stencils for every instance.
+void launch_strips_mom(const StepLaunch& L, hipStream_t s, int par) {
+  const int chunk = (L.nmstrips + 7) / 8;
+  k_strip_mom<float, float><<<8 * chunk, 256, 0, s>>>(L.insts, L.mstrips, L.nmstrips, chunk, par, L.step_ctr);
 }
 
 template void launch_alpha<double>(const StepLaunch&, hipStream_t, int, int);

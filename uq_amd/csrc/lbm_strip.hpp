@@ -58,7 +58,7 @@ struct SPos {
 // Per-lane constants of a work item.
 template <typename TC>
 struct StripLane {
-  int X;           // mapped column of the lane's logical column
+  unsigned X;      // mapped column of the lane's logical column
   int mx;          // the column is mirrored east/west
   int own;         // an own column of the item inside the instance
   int clampL;      // the logical column left of the lane is a clamped position
@@ -136,9 +136,20 @@ struct StripInst {
   int rdy_stride;
   long long P;
   int pitch, ny, py, ms, mn;
-  int inner;  // the item's rows and their 3-row halo lie inside the instance
+  int inner;   // the item's rows and their 3-row halo lie inside the instance
+  int colmir;  // some lane's column is mirrored east/west
   double c;
 };
+
+// Element at column X of the row `base` points at: base is the same for the
+// whole wavefront (planes and rows are), so the access takes it from scalar
+// registers with the lane's 32-bit byte offset, and neither 64-bit addresses
+// per lane nor vector instructions to form them are needed.
+template <typename T>
+__device__ __forceinline__ gptr<T> at_col(gptr<T> base, unsigned X) {
+  if constexpr (std::is_const<T>::value) return (gptr<T>)((gptr<const char>)base + X * unsigned(sizeof(T)));
+  else return (gptr<T>)((gptr<char>)base + X * unsigned(sizeof(T)));
+}
 
 // The row order of a march: rows y0 .. y0 + nrows - 1 of the item, or (flip)
 // the item turned upside down (row y of the march is row 2 y0 + nrows - 1 - y
@@ -159,11 +170,8 @@ struct March {
   TC vx, vy;
   TC rf, rh;  // reference equilibrium of the direction for the wall faces of FP32 storage
               // (a mirror image of it has the same reference: it depends on |e|)
-  // this lane's column in the planes of the direction staged at a row that
-  // is not (0) or is (1) mirrored north/south
-  gptr<const TS> pf0, ph0, pf1, ph1;
-  gptr<const uint8_t> ct;
-  gptr<const double> al;
+  gptr<const TS> pf0, ph0, pf1, ph1;  // planes staged at a row that is not (0) or is (1) mirrored north/south
+  long long pew0, pew1;               // from them to the planes of an east/west mirrored column
   SPos<TC> W[HY ? 6 : 1];  // rows F - 3 .. F + 2 of the y face F below row F
   TC Fyf, Fyh;             // the y face below the next row
 
@@ -174,27 +182,34 @@ struct March {
     vy = TC(double(aey) * in.c);
     rf = rf_;
     rh = rh_;
-    const int dew = c_mir_ew[I], dns = c_mir_ns[I], dboth = c_mir_ns[dew];
-    const int d0 = C.mx ? dew : I, d1 = C.mx ? dboth : dns;
-    pf0 = in.src + (long long)d0 * in.P + C.X;
-    ph0 = in.src + (long long)(kQ + d0) * in.P + C.X;
-    pf1 = in.src + (long long)d1 * in.P + C.X;
-    ph1 = in.src + (long long)(kQ + d1) * in.P + C.X;
-    ct = in.ct + C.X;
-    al = in.alpha + C.X;
+    const int dns = c_mir_ns[I];
+    pf0 = in.src + (long long)I * in.P;
+    ph0 = in.src + (long long)(kQ + I) * in.P;
+    pf1 = in.src + (long long)dns * in.P;
+    ph1 = in.src + (long long)(kQ + dns) * in.P;
+    pew0 = (long long)(c_mir_ew[I] - I) * in.P;
+    pew1 = (long long)(c_mir_ew[dns] - dns) * in.P;
     Fyf = Fyh = TC(0);
   }
 
   // The staged position of logical row yl (an instance row).
-  __device__ __forceinline__ SPos<TC> load(const StripInst<TS>& in, int yl) const {
+  __device__ __forceinline__ SPos<TC> load(const StripInst<TS>& in, const StripLane<TC>& C, int yl) const {
     unsigned my = 0, cy;
     const int ro = (in.inner ? yl : map_axis(yl, in.ny, in.py, in.ms, in.mn, my, cy)) * in.pitch;
     const bool m = (in.ms | in.mn) != 0 && my;
+    const gptr<const TS> pf = (m ? pf1 : pf0) + ro, ph = (m ? ph1 : ph0) + ro;
+    TS f = *at_col(pf, C.X), h = *at_col(ph, C.X);
+    if (in.colmir) {
+      const long long ew = m ? pew1 : pew0;
+      const TS fm = *at_col(pf + ew, C.X), hm = *at_col(ph + ew, C.X);
+      f = C.mx ? fm : f;
+      h = C.mx ? hm : h;
+    }
     SPos<TC> p;
-    p.f = TC((m ? pf1 : pf0)[ro]);
-    p.h = TC((m ? ph1 : ph0)[ro]);
-    p.type = SOLID ? int(ct[ro]) : 0;
-    p.a = SOLID ? TC(al[ro]) : TC(0);
+    p.f = TC(f);
+    p.h = TC(h);
+    p.type = SOLID ? int(*at_col(in.ct + ro, C.X)) : 0;
+    p.a = SOLID ? TC(*at_col(in.alpha + ro, C.X)) : TC(0);
     return p;
   }
   static __device__ __forceinline__ int clamped_row(const StripInst<TS>& in, int yl) {
@@ -272,10 +287,10 @@ struct March {
   }
 
   // Fills the window for row y0 (call first_face once the loads have landed).
-  __device__ __forceinline__ void fill(const StripInst<TS>& in, const RowOrder& ro, int y0) {
+  __device__ __forceinline__ void fill(const StripInst<TS>& in, const StripLane<TC>& C, const RowOrder& ro, int y0) {
     if constexpr (HY) {
 #pragma unroll
-      for (int k = 0; k < 6; k++) W[k] = load(in, ro(y0 - 3 + k));
+      for (int k = 0; k < 6; k++) W[k] = load(in, C, ro(y0 - 3 + k));
     }
   }
   __device__ __forceinline__ void first_face() {
@@ -283,8 +298,9 @@ struct March {
   }
   // The position row y of the march needs from memory: the one entering the
   // window (row y + 3), without a y component row y itself.
-  __device__ __forceinline__ SPos<TC> next(const StripInst<TS>& in, const RowOrder& ro, int y) const {
-    return load(in, ro(HY ? y + 3 : y));
+  __device__ __forceinline__ SPos<TC> next(const StripInst<TS>& in, const StripLane<TC>& C, const RowOrder& ro,
+                                               int y) const {
+    return load(in, C, ro(HY ? y + 3 : y));
   }
 
   // Net flux of row y's cell from its prefetched position (registers only:
@@ -355,14 +371,13 @@ __device__ __forceinline__ void strip_dir(const StripInst<TS>& in, const StripLa
   m.setup(in, C, rf, rh, I);
   const RowOrder ro{flip, 2 * y0 + nrows - 1};
   const int pitch = in.pitch;
-  // this lane's own cell in the planes it writes (MODE 0, 2: the dF planes
-  // of direction I; MODE 1: the state planes) and, MODE 1, in the planes of
-  // direction I it reads: the stored dF(f2)
-  const gptr<TS> of = in.dst + (MODE == 1 ? (long long)I : (long long)(I - 1)) * in.P + C.X;
-  const gptr<TS> oh = in.dst + (MODE == 1 ? (long long)(kQ + I) : (long long)(12 + I - 1)) * in.P + C.X;
-  const gptr<const TS> df2 = in.dfl + (long long)(I - 1) * in.P + C.X;
-  const gptr<const TS> dh2 = in.dfl + (long long)(12 + I - 1) * in.P + C.X;
-  const gptr<const uint8_t> ct = in.ct + C.X;
+  // the planes the item writes (MODE 0, 2: the dF planes of direction I;
+  // MODE 1: the state planes) and, MODE 1, those of direction I it reads:
+  // the stored dF(f2)
+  const gptr<TS> of = in.dst + (MODE == 1 ? (long long)I : (long long)(I - 1)) * in.P;
+  const gptr<TS> oh = in.dst + (MODE == 1 ? (long long)(kQ + I) : (long long)(12 + I - 1)) * in.P;
+  const gptr<const TS> df2 = in.dfl + (long long)(I - 1) * in.P;
+  const gptr<const TS> dh2 = in.dfl + (long long)(12 + I - 1) * in.P;
 
   // Everything a row needs from memory, loaded one row ahead: the staged
   // position, the own cell's type as loaded (0 fluid; 1 for lanes without an
@@ -377,15 +392,15 @@ __device__ __forceinline__ void strip_dir(const StripInst<TS>& in, const StripLa
   };
   auto fetch = [&](int y) {
     Pre r;
-    r.p = m.next(in, ro, y);
+    r.p = m.next(in, C, ro, y);
     r.ro = ro(y) * pitch;
     r.type = 1;
     r.f = r.h = TS(0);
     if (C.own) {
-      r.type = ct[r.ro];
+      r.type = *at_col(in.ct + r.ro, C.X);
       if (MODE == 1) {
-        r.f = df2[r.ro];
-        r.h = dh2[r.ro];
+        r.f = *at_col(df2 + r.ro, C.X);
+        r.h = *at_col(dh2 + r.ro, C.X);
       }
     }
     r.rdy = TC(in.rdyp[ro(y) * in.rdy_stride]);
@@ -398,8 +413,8 @@ __device__ __forceinline__ void strip_dir(const StripInst<TS>& in, const StripLa
   };
   auto store = [&](const Res& r) {
     if (r.on) {
-      of[r.ro] = r.vf;
-      oh[r.ro] = r.vh;
+      *at_col(of + r.ro, C.X) = r.vf;
+      *at_col(oh + r.ro, C.X) = r.vh;
     }
   };
   // row y from its prefetched data (registers only: no memory access)
@@ -429,7 +444,7 @@ __device__ __forceinline__ void strip_dir(const StripInst<TS>& in, const StripLa
   // stores the previous row, issues the next row's loads into the other
   // slot and computes its row from registers.
   const int end = y0 + nrows;
-  m.fill(in, ro, y0);
+  m.fill(in, C, ro, y0);
   Pre A = fetch(y0), B;
   if constexpr (M::HY) {
     __builtin_amdgcn_s_waitcnt(kWaitVmem);
@@ -475,8 +490,9 @@ __device__ __forceinline__ void strip_setup(const InstDev& in, const TileRef& sr
   C.xl = x0 - kH + lane;
   const int px = in.flags & kPeriodicX, mw = in.flags & kMirrorW, me = in.flags & kMirrorE;
   unsigned mx, cx, mt, cl, cr;
-  C.X = map_axis(C.xl, in.nx, px, mw, me, mx, cx);
+  C.X = (unsigned)map_axis(C.xl, in.nx, px, mw, me, mx, cx);
   C.mx = (int)mx;
+  si.colmir = __ballot(C.mx != 0) != 0;
   (void)map_axis(C.xl - 1, in.nx, px, mw, me, mt, cl);
   (void)map_axis(C.xl + 1, in.nx, px, mw, me, mt, cr);
   C.clampL = (int)cl;
@@ -547,5 +563,199 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
   } else {
     if (in.flux_method == 1) strip_item<TS, TC, MODE, false, true>(in, si, C, sr, I, alive);
     else strip_item<TS, TC, MODE, false, false>(in, si, C, sr, I, alive);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// k_strip_mom: the stage-3 flux of FP32 storage. Beside the new state
+// G - dF/2, each cell's net fluxes of all twelve directions are summed into
+// the FP64 moment planes, so one workgroup takes all of them: four
+// wavefronts march the same strip in step, each with one direction along x,
+// one along y and one diagonal (four net faces for f and h each: equal work),
+// and exchange a row's net fluxes through LDS; wavefront k then adds moment k
+// over the directions in their order (the tile kernel's order, the same
+// bits). One barrier per row: the rows alternate between two LDS buffers, so
+// a wavefront writes a buffer again only after every other one has passed
+// the barrier that follows its reads. Three marches per wavefront also
+// overlap each other's dependent arithmetic. Bound by HBM on large groups, by
+// the latency of one march on small ones. Against the tile kernel (twelve
+// directions one after the other per tile, two barriers each): 256-member
+// ensemble 3490 -> 2328 us per launch (2.4 -> 3.6 TB/s of its 352 B per
+// cell), Riemann 3072^2 1384 -> 920, shear 256^2 35 -> 20, couette 64^2 36 -> 17.
+// ---------------------------------------------------------------------------
+template <typename TC>
+struct MomRows {
+  TC v[2][2 * (kQ - 1)][64];  // [buffer][f and h net flux of directions 1..12][lane]
+};
+
+// Wavefront w: directions c_mom_dir[w] (x, y, diagonal), all of x sign
+// (w == 0 || w == 3) and y sign (w < 2).
+static __constant__ int c_mom_dir[4][3] = {{1, 2, 5}, {3, 10, 6}, {11, 4, 7}, {9, 12, 8}};
+
+// Moment k (0 mass, 1 and 2 x and y momentum, 3 energy) of a row's net fluxes.
+template <typename TC>
+__device__ __forceinline__ double mom_sum(const TC (&v)[2 * (kQ - 1)][64], int lane, int k, double c) {
+#pragma clang fp contract(off)
+  double s = 0;
+  if (k == 0) {
+#pragma unroll
+    for (int I = 1; I < kQ; I++) s += double(v[2 * (I - 1)][lane]);
+  } else if (k == 1) {
+#pragma unroll
+    for (int I = 1; I < kQ; I++) s += double(v[2 * (I - 1)][lane]) * (lat_x(I) * c);
+  } else if (k == 2) {
+#pragma unroll
+    for (int I = 1; I < kQ; I++) s += double(v[2 * (I - 1)][lane]) * (lat_y(I) * c);
+  } else {
+#pragma unroll
+    for (int I = 1; I < kQ; I++) s += double(v[2 * (I - 1) + 1][lane]);
+  }
+  return s;
+}
+
+template <typename TS, typename TC, bool SOLID, bool W5, int SX, int SY>
+__device__ __forceinline__ void strip_mom_rows(const InstDev& inst, const StripInst<TS>& in, const StripLane<TC>& C,
+                                               const TileRef& sr, int w, int flip, bool alive, gptr<double> momp,
+                                               MomRows<TC>& X) {
+  static_assert(kStage3G<TS>, "moment sums belong to the stage-3 flux of FP32 storage");
+  const int lane = threadIdx.x & 63, y0 = sr.ty, nrows = sr.flags >> kStripRowsBit, pitch = in.pitch;
+  const int Ix = c_mom_dir[w][0], Iy = c_mom_dir[w][1], Id = c_mom_dir[w][2];
+  March<TS, TC, SOLID, W5, SX, 0> mx;
+  March<TS, TC, SOLID, W5, 0, SY> my;
+  March<TS, TC, SOLID, W5, SX, SY> md;
+  mx.setup(in, C, TC(inst.ref[Ix]), TC(inst.ref[kQ + Ix]), Ix);
+  my.setup(in, C, TC(inst.ref[Iy]), TC(inst.ref[kQ + Iy]), Iy);
+  md.setup(in, C, TC(inst.ref[Id]), TC(inst.ref[kQ + Id]), Id);
+  const RowOrder ro{flip, 2 * y0 + nrows - 1};
+  const gptr<double> mom = momp + (long long)w * in.P;
+  const gptr<TS> st[6] = {in.dst + Ix * in.P, in.dst + (kQ + Ix) * in.P, in.dst + Iy * in.P, in.dst + (kQ + Iy) * in.P,
+                          in.dst + Id * in.P, in.dst + (kQ + Id) * in.P};
+
+  // A row's data from memory: the three staged positions, the own cell's
+  // type, its six G values and its moment w, dt/dy.
+  struct Pre {
+    SPos<TC> px, py, pd;
+    int ro, type;
+    TS g[6];
+    double m;
+    TC rdy;
+  };
+  auto fetch = [&](int y) {
+    Pre r;
+    r.px = mx.next(in, C, ro, y);
+    r.py = my.next(in, C, ro, y);
+    r.pd = md.next(in, C, ro, y);
+    r.ro = ro(y) * pitch;
+    r.type = 1;
+    r.m = 0;
+#pragma unroll
+    for (int k = 0; k < 6; k++) r.g[k] = TS(0);
+    if (C.own) {
+      r.type = *at_col(in.ct + r.ro, C.X);
+#pragma unroll
+      for (int k = 0; k < 6; k++) r.g[k] = *at_col(st[k] + r.ro, C.X);
+      r.m = *at_col(mom + r.ro, C.X);
+    }
+    r.rdy = TC(in.rdyp[ro(y) * in.rdy_stride]);
+    return r;
+  };
+  struct Res {
+    int ro, on;
+    TS v[6];
+    double m;
+  };
+  auto store = [&](const Res& r) {
+    if (r.on) {
+#pragma unroll
+      for (int k = 0; k < 6; k++) *at_col(st[k] + r.ro, C.X) = r.v[k];
+      *at_col(mom + r.ro, C.X) = r.m;
+    }
+  };
+  auto row = [&](int y, const Pre& cc, int buf) {
+#pragma clang fp contract(off)
+    TC d[6], a, b;
+    mx.net(in, C, ro, y, cc.px, cc.rdy, d[0], d[1], a, b);
+    my.net(in, C, ro, y, cc.py, cc.rdy, d[2], d[3], a, b);
+    md.net(in, C, ro, y, cc.pd, cc.rdy, d[4], d[5], a, b);
+    TC(&v)[2 * (kQ - 1)][64] = X.v[buf];
+    v[2 * (Ix - 1)][lane] = d[0];
+    v[2 * (Ix - 1) + 1][lane] = d[1];
+    v[2 * (Iy - 1)][lane] = d[2];
+    v[2 * (Iy - 1) + 1][lane] = d[3];
+    v[2 * (Id - 1)][lane] = d[4];
+    v[2 * (Id - 1) + 1][lane] = d[5];
+    Res r;
+    r.ro = cc.ro;
+    r.on = alive && cc.type == 0;
+#pragma unroll
+    for (int k = 0; k < 6; k++) r.v[k] = TS(TC(cc.g[k]) - TC(0.5) * d[k]);
+    // LDS only: the row's global loads and stores stay in flight across the
+    // barrier (each wavefront reads and writes its own planes)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    r.m = cc.m - 0.5 * mom_sum(v, lane, w, in.c);
+    return r;
+  };
+  // as strip_dir: one wait, the stores of the row before, the next row's loads
+  const int end = y0 + nrows;
+  my.fill(in, C, ro, y0);
+  md.fill(in, C, ro, y0);
+  Pre A = fetch(y0), B;
+  __builtin_amdgcn_s_waitcnt(kWaitVmem);
+  my.first_face();
+  md.first_face();
+  Res R{0, 0, {}, 0.0};
+  for (int y = y0;; y += 2) {
+    __builtin_amdgcn_s_waitcnt(kWaitVmem);
+    store(R);
+    if (y + 1 < end) B = fetch(y + 1);
+    R = row(y, A, 0);
+    if (y + 1 >= end) break;
+    __builtin_amdgcn_s_waitcnt(kWaitVmem);
+    store(R);
+    if (y + 2 < end) A = fetch(y + 2);
+    R = row(y + 1, B, 1);
+    if (y + 2 >= end) break;
+  }
+  store(R);
+}
+
+template <typename TS, typename TC, bool SOLID, bool W5>
+__device__ __forceinline__ void strip_mom_item(const InstDev& inst, const StripInst<TS>& si, const StripLane<TC>& C,
+                                               const TileRef& sr, int w, bool alive, gptr<double> momp,
+                                               MomRows<TC>& X) {
+  const int fl = (sr.flags & kStripDesc) != 0;
+  const bool px = w == 0 || w == 3, py = (w < 2) != (fl != 0);  // signs in the march's row order
+  if (px && py) strip_mom_rows<TS, TC, SOLID, W5, 1, 1>(inst, si, C, sr, w, fl, alive, momp, X);
+  else if (py) strip_mom_rows<TS, TC, SOLID, W5, -1, 1>(inst, si, C, sr, w, fl, alive, momp, X);
+  else if (px) strip_mom_rows<TS, TC, SOLID, W5, 1, -1>(inst, si, C, sr, w, fl, alive, momp, X);
+  else strip_mom_rows<TS, TC, SOLID, W5, -1, -1>(inst, si, C, sr, w, fl, alive, momp, X);
+}
+
+// One workgroup per work item, a contiguous chunk of the items per XCD.
+template <typename TS, typename TC>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_strip_mom(
+    const InstDev* __restrict__ insts, const TileRef* __restrict__ strips, int nstrips, int chunk, int par,
+    const int* stepp) {
+  __shared__ MomRows<TC> X;
+  const int step = *stepp;
+  const int it = (int)(blockIdx.x % 8) * chunk + (int)(blockIdx.x / 8);
+  if (it >= nstrips) return;
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const TileRef sr = strips[it];
+  const InstDev& in = insts[sr.inst];
+  const bool alive = !frozen_by_failure(in, step);
+  const int nxt = 1 ^ in.parity0 ^ par;
+  StripInst<TS> si;
+  StripLane<TC> C;
+  strip_setup<TS, TC>(in, sr, in.f3, in.state[nxt], si, C);
+  const gptr<double> momp = (gptr<double>)in.mom[nxt];
+  if (sr.flags & kTileSolid) {
+    if (in.flux_method == 1) strip_mom_item<TS, TC, true, true>(in, si, C, sr, w, alive, momp, X);
+    else strip_mom_item<TS, TC, true, false>(in, si, C, sr, w, alive, momp, X);
+  } else {
+    if (in.flux_method == 1) strip_mom_item<TS, TC, false, true>(in, si, C, sr, w, alive, momp, X);
+    else strip_mom_item<TS, TC, false, false>(in, si, C, sr, w, alive, momp, X);
   }
 }
