@@ -1498,24 +1498,40 @@ __global__ void k_init(const InstDev* insts, int inst, const int* ids, const dou
   }
 }
 
-// out: 5 planes of double [ny][pitch]: rho, ux, uy, p, T
+// outp: rho, ux, uy, p, T, each in the boundary's order [nx][ny]: a workgroup
+// reads a 32 x 32 tile of the state in row segments and writes each field in
+// columns through LDS (a row more per column: no bank conflicts).
+constexpr int kMacT = 32;
 template <typename TS>
-__global__ void k_macro(const InstDev* insts, int inst, int par, double* outp) {
+__global__ __launch_bounds__(256) void k_macro(const InstDev* insts, int inst, int par, double* outp) {
+  __shared__ double v[5][kMacT][kMacT + 1];
   const InstDev& in = insts[inst];
-  const long long n = (long long)in.ny * in.pitch;
+  const long long n = (long long)in.nx * in.ny;
   const TS* src = reinterpret_cast<const TS*>(in.state[in.parity0 ^ par]);
-  for (long long o = blockIdx.x * (long long)blockDim.x + threadIdx.x; o < n; o += (long long)gridDim.x * blockDim.x) {
-    const int x = (int)(o % in.pitch);
-    if (x >= in.nx) continue;
-    CellState<TS> cs;
-    load_state(in, src, in.mom[in.parity0 ^ par], o, cs);
-    Macro m;
-    finish_macro(in, cs.s[0], cs.s[1], cs.s[2], cs.s[3], m);
-    outp[o] = m.rho;
-    outp[n + o] = m.ux;
-    outp[2 * n + o] = m.uy;
-    outp[3 * n + o] = m.p;
-    outp[4 * n + o] = m.T;
+  const int tw = (in.nx + kMacT - 1) / kMacT, nt = tw * ((in.ny + kMacT - 1) / kMacT);
+  const int l = threadIdx.x % kMacT, r = threadIdx.x / kMacT;
+  for (int t = blockIdx.x; t < nt; t += gridDim.x) {
+    const int x0 = t % tw * kMacT, y0 = t / tw * kMacT;
+    for (int k = r; k < kMacT; k += 256 / kMacT) {
+      if (x0 + l >= in.nx || y0 + k >= in.ny) continue;
+      const long long o = (long long)(y0 + k) * in.pitch + x0 + l;
+      CellState<TS> cs;
+      load_state(in, src, in.mom[in.parity0 ^ par], o, cs);
+      Macro m;
+      finish_macro(in, cs.s[0], cs.s[1], cs.s[2], cs.s[3], m);
+      v[0][k][l] = m.rho;
+      v[1][k][l] = m.ux;
+      v[2][k][l] = m.uy;
+      v[3][k][l] = m.p;
+      v[4][k][l] = m.T;
+    }
+    __syncthreads();
+    for (int k = r; k < kMacT; k += 256 / kMacT) {
+      if (x0 + k >= in.nx || y0 + l >= in.ny) continue;
+#pragma unroll
+      for (int q = 0; q < 5; q++) outp[q * n + (long long)(x0 + k) * in.ny + y0 + l] = v[q][l][k];
+    }
+    __syncthreads();
   }
 }
 
@@ -1934,17 +1950,17 @@ void launch_init(const InstDev* insts, int inst, const int* ids, const double* p
 }
 
 template <typename TS>
-void launch_macro(const InstDev* insts, int inst, int par, double* out, long long cells, hipStream_t s) {
-  const int blocks = (int)((cells + 255) / 256 < 4096 ? (cells + 255) / 256 : 4096);
-  k_macro<TS><<<blocks, 256, 0, s>>>(insts, inst, par, out);
+void launch_macro(const InstDev* insts, int inst, int par, double* out, int nx, int ny, hipStream_t s) {
+  const long long tiles = (long long)((nx + kMacT - 1) / kMacT) * ((ny + kMacT - 1) / kMacT);
+  k_macro<TS><<<(int)(tiles < 4096 ? tiles : 4096), 256, 0, s>>>(insts, inst, par, out);
 }
 
 template void launch_step<double, double>(const StepLaunch&, hipStream_t, int, KernelTimer*);
 template void launch_step<float, float>(const StepLaunch&, hipStream_t, int, KernelTimer*);
 template void launch_init<double>(const InstDev*, int, const int*, const double*, long long, hipStream_t);
 template void launch_init<float>(const InstDev*, int, const int*, const double*, long long, hipStream_t);
-template void launch_macro<double>(const InstDev*, int, int, double*, long long, hipStream_t);
-template void launch_macro<float>(const InstDev*, int, int, double*, long long, hipStream_t);
+template void launch_macro<double>(const InstDev*, int, int, double*, int, int, hipStream_t);
+template void launch_macro<float>(const InstDev*, int, int, double*, int, int, hipStream_t);
 template void launch_totals<double>(const InstDev*, int, int, double*, long long, hipStream_t);
 template void launch_totals<float>(const InstDev*, int, int, double*, long long, hipStream_t);
 template void launch_residual<double>(const InstDev*, int, int, double*, int, int, hipStream_t);

@@ -141,7 +141,7 @@ void launch_init(const InstDev* insts, int inst, const int* ids, const double* p
                  hipStream_t s);
 
 template <typename TS>
-void launch_macro(const InstDev* insts, int inst, int par, double* out, long long cells, hipStream_t s);
+void launch_macro(const InstDev* insts, int inst, int par, double* out, int nx, int ny, hipStream_t s);
 
 // Conserved totals (mass, x and y momentum, total energy) of the fluid cells
 // of one instance; `scratch` holds totals_scratch_doubles() doubles and the

@@ -446,6 +446,7 @@ Solver::~Solver() {
 }
 
 extern "C" void lbm_release_cached(void) {
+  release_slots();
   BufferCache& c = buffer_cache();
   std::lock_guard<std::mutex> lock(c.mu);
   c.drop(-1);
@@ -892,18 +893,6 @@ int uqlbm::upload_inst(Solver& s) {
   return LBM_OK;
 }
 
-static int macro_into(Solver& s, std::vector<double>& host) {
-  const long long cells = (long long)s.pitch * s.ny;
-  if (s.precision == LBM_PREC_FP64) launch_macro<double>(s.inst_dev, 0, 0, s.macro_dev, cells, s.stream);
-  else launch_macro<float>(s.inst_dev, 0, 0, s.macro_dev, cells, s.stream);
-  HIP_TRY(hipGetLastError());
-  host.resize((size_t)cells * 5);
-  HIP_TRY(hipMemcpyAsync(host.data(), s.macro_dev, host.size() * sizeof(double), hipMemcpyDeviceToHost,
-                         s.stream));
-  HIP_TRY(hipStreamSynchronize(s.stream));
-  return LBM_OK;
-}
-
 static void launch_steps(const StepLaunch& L, int precision, hipStream_t stream, int nsteps,
                          KernelTimer* tm) {
   for (int k = 0; k < nsteps; k++) {
@@ -1159,16 +1148,12 @@ extern "C" int lbm_get_macro(lbm_solver* h, double* rho, double* ux, double* uy,
   if (!h) return fail_with(LBM_ERR_ARG, "null solver");
   Solver& s = *reinterpret_cast<Solver*>(h);
   if (!s.inited) return fail_with(LBM_ERR_STATE, "lbm_get_macro before lbm_init");
-  std::vector<double> m;
-  int st = macro_into(s, m);
-  if (st != LBM_OK) return st;
-  const size_t n = (size_t)s.pitch * s.ny;
-  double* outs[5] = {rho, ux, uy, p, T};
-  for (int k = 0; k < 5; k++) {
-    if (!outs[k]) continue;
-    for (int x = 0; x < s.nx; x++)
-      for (int y = 0; y < s.ny; y++) outs[k][(size_t)x * s.ny + y] = m[k * n + (size_t)y * s.pitch + x];
-  }
+  if (s.precision == LBM_PREC_FP64) launch_macro<double>(s.inst_dev, 0, 0, s.macro_dev, s.nx, s.ny, s.stream);
+  else launch_macro<float>(s.inst_dev, 0, 0, s.macro_dev, s.nx, s.ny, s.stream);
+  HIP_TRY(hipGetLastError());
+  const size_t field = (size_t)s.nx * s.ny * sizeof(double);
+  HIP_TRY(staged_copy((char*)s.macro_dev, {{rho, field}, {ux, field}, {uy, field}, {p, field}, {T, field}}, true,
+                      s.stream));
   return LBM_OK;
 }
 
@@ -1187,103 +1172,27 @@ extern "C" int lbm_get_totals(lbm_solver* h, double* out) {
   return LBM_OK;
 }
 
-// Host copies of the state: FP64 storage as stored; FP32 storage restores
-// deviation + reference and applies the moment correction of the kernels'
-// state loader (lbm_kernels.hip, load_state) with the FP64 moment planes.
-template <typename TS>
-static int read_state(Solver& s, std::vector<TS>& buf, std::vector<double>& mom) {
-  const size_t plane = (size_t)s.pitch * s.ny;
-  buf.resize(plane * kPlanes);
-  HIP_TRY(hipMemcpyAsync(buf.data(), s.state[s.cur], buf.size() * sizeof(TS), hipMemcpyDeviceToHost, s.stream));
-  if (s.precision != LBM_PREC_FP64) {
-    mom.resize(plane * 4);
-    HIP_TRY(hipMemcpyAsync(mom.data(), s.mom[s.cur], mom.size() * sizeof(double), hipMemcpyDeviceToHost, s.stream));
-  }
+// Distributions at the boundary: transposed on the device into (out of) the
+// stage buffers f2 and f3, which hold nothing between step calls (each has
+// 13 doubles per cell in both storage types), and copied from (to) there.
+static int get_dist(Solver& s, double* f, double* h) {
+  double *df = (double*)s.f2, *dh = (double*)s.f3;
+  launch_dist_out(s, f ? df : nullptr, h ? dh : nullptr);
+  HIP_TRY(hipGetLastError());
+  const size_t bytes = (size_t)s.nx * s.ny * kQ * sizeof(double);
+  if (f) HIP_TRY(staged_copy((char*)df, {{f, bytes}}, true, s.stream));
+  if (h) HIP_TRY(staged_copy((char*)dh, {{h, bytes}}, true, s.stream));
   HIP_TRY(hipStreamSynchronize(s.stream));
   return LBM_OK;
 }
 
-template <typename TS>
-static void cell_values(const Solver& s, const std::vector<TS>& buf, const std::vector<double>& mom, size_t o,
-                        double* f, double* h) {
-  const size_t plane = (size_t)s.pitch * s.ny;
-  for (int i = 0; i < kQ; i++) {
-    f[i] = double(buf[plane * i + o]);
-    h[i] = double(buf[plane * (kQ + i) + o]);
-  }
-  if (s.precision == LBM_PREC_FP64) return;
-  double t[4] = {0, 0, 0, 0};
-  for (int i = 0; i < kQ; i++) {
-    f[i] += s.ref[i];
-    h[i] += s.ref[kQ + i];
-    t[0] += f[i];
-    t[1] += f[i] * (lat_x(i) * s.c);
-    t[2] += f[i] * (lat_y(i) * s.c);
-    t[3] += h[i];
-  }
-  const double i2c = 0.5 / s.c;
-  const double dx = (mom[plane + o] - t[1]) * i2c, dy = (mom[2 * plane + o] - t[2]) * i2c;
-  f[0] += mom[o] - t[0];
-  f[1] += dx;
-  f[3] -= dx;
-  f[2] += dy;
-  f[4] -= dy;
-  h[0] += mom[3 * plane + o] - t[3];
-}
-
-template <typename TS>
-static int get_dist_t(Solver& s, double* f, double* hh) {
-  std::vector<TS> buf;
-  std::vector<double> mom;
-  int st = read_state(s, buf, mom);
-  if (st != LBM_OK) return st;
-  for (int x = 0; x < s.nx; x++)
-    for (int y = 0; y < s.ny; y++) {
-      double fv[kQ], hv[kQ];
-      cell_values(s, buf, mom, (size_t)y * s.pitch + x, fv, hv);
-      for (int i = 0; i < kQ; i++) {
-        const size_t k = ((size_t)x * s.ny + y) * kQ + i;
-        if (f) f[k] = fv[i];
-        if (hh) hh[k] = hv[i];
-      }
-    }
-  return LBM_OK;
-}
-
-template <typename TS>
-static int set_dist_t(Solver& s, const double* f, const double* hh) {
-  std::vector<TS> buf;
-  std::vector<double> mom;
-  int st = read_state(s, buf, mom);
-  if (st != LBM_OK) return st;
-  const size_t plane = (size_t)s.pitch * s.ny;
-  for (int x = 0; x < s.nx; x++)
-    for (int y = 0; y < s.ny; y++) {
-      const size_t o = (size_t)y * s.pitch + x;
-      double fv[kQ], hv[kQ];
-      cell_values(s, buf, mom, o, fv, hv);  // keeps the cell's values where f or h is not given
-      for (int i = 0; i < kQ; i++) {
-        const size_t k = ((size_t)x * s.ny + y) * kQ + i;
-        if (f) fv[i] = f[k];
-        if (hh) hv[i] = hh[k];
-      }
-      double t[4] = {0, 0, 0, 0};
-      for (int i = 0; i < kQ; i++) {
-        const double r = s.precision == LBM_PREC_FP64 ? 0.0 : s.ref[i];
-        const double rh = s.precision == LBM_PREC_FP64 ? 0.0 : s.ref[kQ + i];
-        buf[plane * i + o] = TS(fv[i] - r);
-        buf[plane * (kQ + i) + o] = TS(hv[i] - rh);
-        t[0] += fv[i];
-        t[1] += fv[i] * (lat_x(i) * s.c);
-        t[2] += fv[i] * (lat_y(i) * s.c);
-        t[3] += hv[i];
-      }
-      if (s.precision != LBM_PREC_FP64)
-        for (int k = 0; k < 4; k++) mom[k * plane + o] = t[k];
-    }
-  HIP_TRY(hipMemcpyAsync(s.state[s.cur], buf.data(), buf.size() * sizeof(TS), hipMemcpyHostToDevice, s.stream));
-  if (s.precision != LBM_PREC_FP64)
-    HIP_TRY(hipMemcpyAsync(s.mom[s.cur], mom.data(), mom.size() * sizeof(double), hipMemcpyHostToDevice, s.stream));
+static int set_dist(Solver& s, const double* f, const double* h) {
+  double *df = (double*)s.f2, *dh = (double*)s.f3;
+  const size_t bytes = (size_t)s.nx * s.ny * kQ * sizeof(double);
+  if (f) HIP_TRY(staged_copy((char*)df, {{const_cast<double*>(f), bytes}}, false, s.stream));
+  if (h) HIP_TRY(staged_copy((char*)dh, {{const_cast<double*>(h), bytes}}, false, s.stream));
+  launch_dist_in(s, f ? df : nullptr, h ? dh : nullptr);
+  HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(s.stream));
   return LBM_OK;
 }
@@ -1292,14 +1201,14 @@ extern "C" int lbm_get_dist(lbm_solver* h, double* f, double* hh) {
   if (!h) return fail_with(LBM_ERR_ARG, "null solver");
   Solver& s = *reinterpret_cast<Solver*>(h);
   if (!s.inited) return fail_with(LBM_ERR_STATE, "lbm_get_dist before lbm_init");
-  return s.precision == LBM_PREC_FP64 ? get_dist_t<double>(s, f, hh) : get_dist_t<float>(s, f, hh);
+  return get_dist(s, f, hh);
 }
 
 extern "C" int lbm_set_dist(lbm_solver* h, const double* f, const double* hh) {
   if (!h) return fail_with(LBM_ERR_ARG, "null solver");
   Solver& s = *reinterpret_cast<Solver*>(h);
   if (!s.inited) return fail_with(LBM_ERR_STATE, "lbm_set_dist before lbm_init");
-  return s.precision == LBM_PREC_FP64 ? set_dist_t<double>(s, f, hh) : set_dist_t<float>(s, f, hh);
+  return set_dist(s, f, hh);
 }
 
 extern "C" int lbm_get_info(const lbm_solver* h, lbm_info* out) {

@@ -165,6 +165,19 @@ struct Batch {
   ~Batch();
 };
 
+// The boundary's arrays (lbm_io.hip). Part of a device range and the host
+// array it is copied to or from (null: skipped).
+struct HostSeg {
+  void* host;
+  size_t bytes;
+};
+hipError_t staged_copy(char* dev, const std::vector<HostSeg>& segs, bool out, hipStream_t stream);
+void release_slots();
+// The solver's state to f, h in the boundary's [x][y][i] order and back, on its
+// stream; null arrays are not written, or keep the state's values.
+void launch_dist_out(Solver& s, double* f, double* h);
+void launch_dist_in(Solver& s, const double* f, const double* h);
+
 int fail_with(int status, const char* fmt, ...);
 // A device buffer of `bytes` for solver s: a kept buffer of that size from a
 // destroyed solver on this device when there is one (contents undefined),
