@@ -260,6 +260,7 @@ struct Macro {
 // mu_ref (T/T_ref)^1.5 (T_ref + S)/(T + S). Kept out of line so that the
 // constant-viscosity path carries none of pow's registers.
 __device__ __noinline__ static double viscosity_of(const InstDev& in, double T) {
+#pragma clang fp contract(off)  // the same roundings in every kernel source
   const double r = T * in.iT_ref_v;
   return in.visc_model == 1 ? in.mu_ref * pow(r, in.vexp)
                             : in.mu_ref * pow(r, 1.5) * ((in.T_ref_v + in.vS) / (T + in.vS));
@@ -322,8 +323,8 @@ __device__ __forceinline__ T minmod(T a, T b) {
   return a + b;  // NaN input only
 }
 
-__device__ __forceinline__ float fused(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
-__device__ __forceinline__ double fused(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__host__ __device__ __forceinline__ float fused(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__host__ __device__ __forceinline__ double fused(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
 // The reconstructions are written with every fused multiply-add explicit and
 // contraction off, so each inlined copy (the solid and solid-free face paths,

@@ -181,8 +181,9 @@ void launch_dist_in(Solver& s, const double* f, const double* h) {
 // pieces in turn, each with a slot and a stream of its own, so that the DMA of
 // one piece overlaps the host copies (and the first-touch page faults) of
 // others; a copy of one piece runs on the solver's stream in the calling
-// thread. Measured for the five fields of 3072^2 cells (377 MB): 420 ms with
-// one pageable copy and a transpose on one core.
+// thread. The five fields of 3072^2 cells (377 MB) take 10 ms (38 GB/s; the DMA
+// alone 57 GB/s), against 420 ms with one pageable copy and a transpose on one
+// core; a 256^2 checkpoint in and out 1.5 ms against 18 ms.
 //
 // Slots are kept for later copies, at most kSlotsKept of them in all
 // (lbm_release_cached returns them); a slot belongs to one copying thread at a

@@ -34,6 +34,7 @@
 
 #include "lbm_device.hpp"
 #include "lbm_launch.hpp"
+#include "lbm_point.hpp"
 #include "lbm_stencil.hpp"
 
 namespace uqlbm {
@@ -298,6 +299,7 @@ __device__ __forceinline__ PointCell point_cell(const InstDev& in, const TileRef
 template <typename TS, typename TC, typename TE, int... Is>
 __device__ __forceinline__ void s12_cell(const InstDev& in, gptr<const TS> src, gptr<const double> mom, gptr<TS> dst,
                                          long long o, int step, Seq<Is...>) {
+  static_assert(sizeof(TS) == 4, "FP64 storage: s12_cell64");
   const long long P = in.plane;
   CellState<TS> cs;
   load_state(in, src, mom, o, cs);
@@ -325,6 +327,43 @@ __device__ __forceinline__ void s12_cell(const InstDev& in, gptr<const TS> src, 
   flag_failure(in, step, m.rho, failure_mass<TS>(in, sumfe), eq_check_tol<TE>(sumabs));
 }
 
+// Sum of the equilibrium masses of a cell, in the order of cell_sums.
+__device__ __forceinline__ double eq_mass(const double* fe) {
+#pragma clang fp contract(off)
+  const double a = ((fe[1] + fe[2]) + fe[5]) + fe[0], b = (fe[3] + fe[10]) + fe[6];
+  const double c = (fe[11] + fe[4]) + fe[7], d = (fe[9] + fe[12]) + fe[8];
+  return ((a + b) + c) + d;
+}
+
+// FP64 storage: all 26 values of f2, the rest direction's too (stage 3 takes
+// the moments and the values of the state from them).
+template <int... Is>
+__device__ __forceinline__ void s12_cell64(const InstDev& in, gptr<const double> src, gptr<double> dst, long long o,
+                                           int step, Seq<Is...>) {
+  const long long P = in.plane;
+  double f[kQ], h[kQ], fes[kQ];
+#pragma unroll
+  for (int i = 0; i < kQ; i++) {
+    f[i] = __builtin_nontemporal_load(&src[P * i + o]);
+    h[i] = __builtin_nontemporal_load(&src[P * (kQ + i) + o]);
+  }
+  Macro m;
+  point_macro(in, cell_sums(f, h, true), m);
+  const PointEq e = point_eq(in, m);
+  const Relax12 r = make_relax12(in, m);
+  auto one = [&](auto Ic) {
+    constexpr int I = decltype(Ic)::value;
+    double fe, he, f2, h2;
+    eq_point<I>(in.kq, e, fe, he);
+    fes[I] = fe;
+    point_s12(r, lat_x(I), lat_y(I), f[I], h[I], fe, he, f2, h2);
+    __builtin_nontemporal_store(f2, &dst[P * I + o]);
+    __builtin_nontemporal_store(h2, &dst[P * (kQ + I) + o]);
+  };
+  (one(std::integral_constant<int, Is>{}), ...);
+  flag_failure(in, step, m.rho, eq_mass(fes), 1e-6);
+}
+
 template <typename TS, typename TC, typename TE>
 __global__ __launch_bounds__(kNT) void k_s12(const InstDev* __restrict__ insts, const TileRef* __restrict__ tiles,
                                              int ntiles, int par, const int* stepp) {
@@ -344,7 +383,8 @@ __global__ __launch_bounds__(kNT) void k_s12(const InstDev* __restrict__ insts, 
       for (int k = 0; k < kPlanes; k++) dst[in.plane * k + c.o] = src[in.plane * k + c.o];
       continue;
     }
-    s12_cell<TS, TC, TE>(in, src, as_global(in.mom[cur]), dst, c.o, step, MakeSeq<kQ>::type{});
+    if constexpr (sizeof(TS) == 8) s12_cell64(in, src, dst, c.o, step, MakeSeq<kQ>::type{});
+    else s12_cell<TS, TC, TE>(in, src, as_global(in.mom[cur]), dst, c.o, step, MakeSeq<kQ>::type{});
   }
 }
 
@@ -370,6 +410,7 @@ template <typename TS, typename TC, typename TE, int... Is>
 __device__ __forceinline__ void s3_cell(const InstDev& in, gptr<const TS> src, gptr<const double> mom,
                                         gptr<const TS> dfb, gptr<TS> f3b, gptr<TS> out, gptr<double> mom_out, long long o,
                                         int step, Seq<Is...>) {
+  static_assert(kStage3G<TS>, "FP64 storage: s3_cell64");
   const long long P = in.plane;
   CellState<TS> cs;
   load_state(in, src, mom, o, cs);
@@ -391,17 +432,13 @@ __device__ __forceinline__ void s3_cell(const InstDev& in, gptr<const TS> src, g
   Macro m1, m3;
   finish_macro(in, s[0], s[1], s[2], s[3], m1);
   finish_macro(in, s[0] - drho, s[1] - drux, s[2] - druy, s[3] - dsh, m3);
-  if constexpr (sizeof(TS) == 4) {
-    // conserved moments of the new state before its dF(f3)/2 term: the
-    // relaxation terms move none, so they are those of f - dF(f2)/2; the
-    // stage-3 flux kernel subtracts half those of dF(f3)
-    mom_out[o] = s[0] - 0.5 * drho;
-    mom_out[P + o] = s[1] - 0.5 * drux;
-    mom_out[2 * P + o] = s[2] - 0.5 * druy;
-    mom_out[3 * P + o] = s[3] - 0.5 * dsh;
-  } else {
-    (void)mom_out;
-  }
+  // conserved moments of the new state before its dF(f3)/2 term: the
+  // relaxation terms move none, so they are those of f - dF(f2)/2; the
+  // stage-3 flux kernel subtracts half those of dF(f3)
+  mom_out[o] = s[0] - 0.5 * drho;
+  mom_out[P + o] = s[1] - 0.5 * drux;
+  mom_out[2 * P + o] = s[2] - 0.5 * druy;
+  mom_out[3 * P + o] = s[3] - 0.5 * dsh;
   const Rec12<TC> r = make_rec12<TC>(in, m1);
   const EqDev qd1 = eq_dev_inputs(in, m1), qd3 = eq_dev_inputs(in, m3);
   const TC hdt = TC(in.dt) * TC(0.5);
@@ -432,26 +469,60 @@ __device__ __forceinline__ void s3_cell(const InstDev& in, gptr<const TS> src, g
     const TC eu3 = TC(lat_x(I)) * cU3 + TC(lat_y(I)) * cV3;
     const TC A3 = (eu3 * ithf3) * (fe3 - f3);
     const TC h3 = ((Qh - hdt * A3) + ah3 * he3) * iah3;
-    if constexpr (kStage3G<TS>) {
-      const TC gf = (Pf + TC(0.5) * dF) + af3 * (fe3 - f3);
-      const TC gh = ((Qh + TC(0.5) * dH) + ah3 * (he3 - h3)) - hdt * A3;
-      if constexpr (I != 0) {  // the rest direction of f3 has no flux and no wall term: nothing reads it
-        __builtin_nontemporal_store(TS(f3), &f3b[P * I + o]);
-        __builtin_nontemporal_store(TS(h3), &f3b[P * (kQ + I) + o]);
-      }
-      __builtin_nontemporal_store(TS(gf), &out[P * I + o]);
-      __builtin_nontemporal_store(TS(gh), &out[P * (kQ + I) + o]);
-    } else {
-      const gptr<TS> dst = I == 0 ? out : f3b;
-      __builtin_nontemporal_store(TS(f3), &dst[P * I + o]);
-      __builtin_nontemporal_store(TS(h3), &dst[P * (kQ + I) + o]);
+    const TC gf = (Pf + TC(0.5) * dF) + af3 * (fe3 - f3);
+    const TC gh = ((Qh + TC(0.5) * dH) + ah3 * (he3 - h3)) - hdt * A3;
+    if constexpr (I != 0) {  // the rest direction of f3 has no flux and no wall term: nothing reads it
+      __builtin_nontemporal_store(TS(f3), &f3b[P * I + o]);
+      __builtin_nontemporal_store(TS(h3), &f3b[P * (kQ + I) + o]);
     }
+    __builtin_nontemporal_store(TS(gf), &out[P * I + o]);
+    __builtin_nontemporal_store(TS(gh), &out[P * (kQ + I) + o]);
     // one direction at a time: keeps the scheduler from interleaving the
-    // directions' temporaries (FP32 storage: 38 spilled registers otherwise)
-    if constexpr (sizeof(TS) == 4) __builtin_amdgcn_sched_barrier(0);
+    // directions' temporaries (38 spilled registers otherwise)
+    __builtin_amdgcn_sched_barrier(0);
   };
   (one(std::integral_constant<int, Is>{}), ...);
   flag_failure(in, step, m3.rho, failure_mass<TS>(in, sumfe), eq_check_tol<TE>(sumabs));
+}
+
+// FP64 storage: stage 3 from f2 and dF(f2) (point_s3).
+template <int... Is>
+__device__ __forceinline__ void s3_cell64(const InstDev& in, gptr<const double> f2b, gptr<const double> dfb,
+                                          gptr<double> f3b, gptr<double> out, long long o, int step, Seq<Is...>) {
+  const long long P = in.plane;
+  double f[kQ], h[kQ], dF[kQ], dH[kQ], fes[kQ];
+#pragma unroll
+  for (int i = 0; i < kQ; i++) {
+    f[i] = __builtin_nontemporal_load(&f2b[P * i + o]);
+    h[i] = __builtin_nontemporal_load(&f2b[P * (kQ + i) + o]);
+  }
+  dF[0] = dH[0] = 0;
+#pragma unroll
+  for (int i = 1; i < kQ; i++) {
+    dF[i] = __builtin_nontemporal_load(&dfb[P * (i - 1) + o]);
+    dH[i] = __builtin_nontemporal_load(&dfb[P * (12 + i - 1) + o]);
+  }
+  const Sums s = cell_sums(f, h, true);
+  Macro m1, m3;
+  point_macro(in, s, m1);
+  point_macro(in, s - cell_sums(dF, dH, false), m3);
+  const PointEq e1 = point_eq(in, m1), e3 = point_eq(in, m3);
+  const Relax3 r = make_relax3(in, m1, m3);
+  auto one = [&](auto Ic) {
+    constexpr int I = decltype(Ic)::value;
+    double fe, he, fe3, he3, f3, h3;
+    eq_point<I>(in.kq, e1, fe, he);
+    eq_point<I>(in.kq, e3, fe3, he3);
+    fes[I] = fe3;
+    point_s3(r, lat_x(I), lat_y(I), f[I], h[I], dF[I], dH[I], fe, he, fe3, he3, f3, h3);
+    // the rest direction has no flux: its f3 is the new state
+    const gptr<double> dst = I == 0 ? out : f3b;
+    __builtin_nontemporal_store(f3, &dst[P * I + o]);
+    __builtin_nontemporal_store(h3, &dst[P * (kQ + I) + o]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  (one(std::integral_constant<int, Is>{}), ...);
+  flag_failure(in, step, m3.rho, eq_mass(fes), 1e-6);
 }
 
 // Frozen cell (permanent or solid) of a pointwise stage: the stored values
@@ -498,8 +569,12 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2))) void k
       copy_frozen(in, src, out, cur, nxt, c.o);
       continue;
     }
-    s3_cell<TS, TC, TE>(in, src, as_global(in.mom[cur]), as_global(reinterpret_cast<const TS*>(in.dflux)), f3b, out,
-                        as_global(in.mom[nxt]), c.o, step, MakeSeq<kQ>::type{});
+    const gptr<const TS> dfb = as_global(reinterpret_cast<const TS*>(in.dflux));
+    if constexpr (sizeof(TS) == 8)
+      s3_cell64(in, as_global(reinterpret_cast<const TS*>(in.f2)), dfb, f3b, out, c.o, step, MakeSeq<kQ>::type{});
+    else
+      s3_cell<TS, TC, TE>(in, src, as_global(in.mom[cur]), dfb, f3b, out, as_global(in.mom[nxt]), c.o, step,
+                          MakeSeq<kQ>::type{});
   }
 }
 

@@ -1,0 +1,256 @@
+// lbm_point.hpp — the pointwise arithmetic of the RK3 stages of FP64 storage:
+// moments, equilibria and relaxation of one cell, in a form that every kernel
+// of the step evaluates with the same roundings (contraction off, every fused
+// multiply-add explicit), whether it holds all thirteen directions of a cell
+// or four wavefronts share them.
+#pragma once
+
+#include "lbm_device.hpp"
+
+namespace uqlbm {
+
+// The directions moving cells share between four wavefronts: wavefront w has
+// one along x, one along y and one diagonal, all of x sign (w == 0 || w == 3)
+// and y sign (w < 2). Sums over the directions of a cell are formed by
+// wavefront, (x + y) + diagonal (+ the rest direction for w = 0), and then
+// over the wavefronts in order.
+__host__ __device__ constexpr int quad_x(int w) { return w == 0 ? 1 : w == 1 ? 3 : w == 2 ? 11 : 9; }
+__host__ __device__ constexpr int quad_y(int w) { return w == 0 ? 2 : w == 1 ? 10 : w == 2 ? 4 : 12; }
+__host__ __device__ constexpr int quad_d(int w) { return 5 + w; }
+
+// Mass, x and y momentum (in units of c) and energy.
+struct Sums {
+  double m, px, py, e;
+};
+
+// Wavefront w's part of a cell's sums. (Products with the lattice velocities
+// 1 and 2 are exact.)
+__host__ __device__ __forceinline__ Sums quad_sums(double exx, double exd, double eyy, double eyd, double fx, double fy,
+                                                   double fd, double hx, double hy, double hd) {
+#pragma clang fp contract(off)
+  Sums s;
+  s.m = (fx + fy) + fd;
+  s.px = fused(exx, fx, exd * fd);
+  s.py = fused(eyy, fy, eyd * fd);
+  s.e = (hx + hy) + hd;
+  return s;
+}
+__host__ __device__ __forceinline__ Sums operator+(const Sums& a, const Sums& b) {
+#pragma clang fp contract(off)
+  return Sums{a.m + b.m, a.px + b.px, a.py + b.py, a.e + b.e};
+}
+__host__ __device__ __forceinline__ Sums operator-(const Sums& a, const Sums& b) {
+#pragma clang fp contract(off)
+  return Sums{a.m - b.m, a.px - b.px, a.py - b.py, a.e - b.e};
+}
+
+template <int W>
+__host__ __device__ __forceinline__ Sums quad_sums_of(const double* f, const double* h) {
+  constexpr int X = quad_x(W), Y = quad_y(W), D = quad_d(W);
+  return quad_sums(lat_x(X), lat_x(D), lat_y(Y), lat_y(D), f[X], f[Y], f[D], h[X], h[Y], h[D]);
+}
+// Sums of all thirteen directions (rest: whether the rest direction counts).
+__host__ __device__ __forceinline__ Sums cell_sums(const double* f, const double* h, bool rest) {
+#pragma clang fp contract(off)
+  Sums a = quad_sums_of<0>(f, h);
+  if (rest) {
+    a.m = a.m + f[0];
+    a.e = a.e + h[0];
+  }
+  return ((a + quad_sums_of<1>(f, h)) + quad_sums_of<2>(f, h)) + quad_sums_of<3>(f, h);
+}
+
+// Moments of a cell (reference macroProp, cpuLBM.cpp:916-970).
+__device__ __forceinline__ void point_macro(const InstDev& in, const Sums& s, Macro& m) {
+#pragma clang fp contract(off)
+  const double irho = 1.0 / s.m;
+  m.rho = s.m;
+  m.ux = (s.px * in.c) * irho;
+  m.uy = (s.py * in.c) * irho;
+  const double usq = fused(m.ux, m.ux, m.uy * m.uy);
+  m.T = fused(2.0, s.e * irho, -usq) * in.ibR;
+  m.p = (m.rho * in.R) * m.T;
+  m.itf = in.visc_model == 0 ? m.p * in.imu : m.p / viscosity_of(in, m.T);
+  m.ith = m.itf * in.Pr;
+  m.ithf = m.itf * in.Pr_m1;
+}
+
+// Equilibria: the closed forms of eq_dir (reference inlineFunctions.cpp:10-61)
+// in nested form; kq: the coefficients that depend on the internal degrees of
+// freedom K (point_consts).
+enum { kqC3, kqK, kq6K, kq14K, kq19K, kqA, kqB, kqC, kqD, kq10C3, kq2C3, kqE, kqF, kqG, kqH, kqI, kqJ, kqC3T, kqCount };
+static_assert(kqCount <= kPointConsts, "InstDev::kq holds the coefficients");
+
+inline void point_consts(double K, double* kq) {
+  const double c3 = 16 + 3 * K;
+  kq[kqC3] = c3;
+  kq[kqK] = K;
+  kq[kq6K] = 6 + K;
+  kq[kq14K] = 14 + K;
+  kq[kq19K] = 19 + K;
+  kq[kqA] = -4 * (4 + K);
+  kq[kqB] = -4 * (7 + K);
+  kq[kqC] = 3 * (10 + K);
+  kq[kqD] = 3 * (14 + K);
+  kq[kq10C3] = 10 * c3;
+  kq[kq2C3] = 2 * c3;
+  kq[kqE] = 3 * (8 + 4 * K);
+  kq[kqF] = 3 * (20 + K);
+  kq[kqG] = -15 * (8 + K);
+  kq[kqH] = 3 * (20 + 2 * K);
+  kq[kqI] = 30 * (9 + K);
+  kq[kqJ] = -30 * (4 + K);
+  kq[kqC3T] = c3 / 3;
+}
+
+struct PointEq {
+  double u, v, t, u2, v2, s2;  // velocity / sqrt(R Tc), T / Tc, squares
+  double rho, sc;              // density, rho R Tc
+};
+
+__host__ __device__ __forceinline__ PointEq point_eq(const InstDev& in, const Macro& m) {
+#pragma clang fp contract(off)
+  PointEq e;
+  e.rho = m.rho;
+  e.u = m.ux * in.isRTc;
+  e.v = m.uy * in.isRTc;
+  e.t = m.T * in.iTc;
+  e.u2 = e.u * e.u;
+  e.v2 = e.v * e.v;
+  e.s2 = e.u2 + e.v2;
+  e.sc = m.rho * in.RTc;
+  return e;
+}
+
+// The four kinds of directions at (a, b): rest, axis, diagonal, double axis.
+__host__ __device__ __forceinline__ void eq_rest(const double* kq, const PointEq& e, double& fe, double& he) {
+#pragma clang fp contract(off)
+  const double uv = e.u2 * e.v2, t = e.t, s2 = e.s2;
+  const double Z = fused(s2, s2 - 5.0, fused(2.0, uv, 4.0));
+  fe = (e.rho * 0.25) * fused(10.0 * t, (t + s2) - 1.0, Z);
+  const double t1 = fused(s2, fused(kq[kqF], s2, kq[kqG]), fused(kq[kqH], uv, kq[kqE]));
+  const double t2 = fused(kq[kqI], s2, kq[kqJ]);
+  he = (e.sc * (1.0 / 24.0)) * fused(t, fused(t, fused(kq[kq10C3], t, t2), t1), 3.0 * (s2 * Z));
+}
+__host__ __device__ __forceinline__ void eq_axis(const double* kq, const PointEq& e, double a, double a2, double b2,
+                                                 double& fe, double& he) {
+#pragma clang fp contract(off)
+  const double t = e.t, g = a + a2;
+  const double w = fused(3.0, b2, a2 - 4.0), z = fused(6.0, g, fused(2.0, a2, w));
+  fe = (e.rho * (-1.0 / 6.0)) * fused(t, fused(6.0, t, z), g * w);
+  const double p = fused(a, fused(a, fused(kq[kq19K], a, kq[kq14K]), kq[kqB]), kq[kqA]);
+  const double r = fused(3.0, b2, fused(a, fused(kq[kqD], a, kq[kqC]), -4.0));
+  const double X = fused(a, p, b2 * r);
+  const double Y = fused(kq[kqK], z, fused(30.0, b2, fused(a, fused(78.0, a, 36.0), -16.0)));
+  he = (e.sc * (-1.0 / 12.0)) * fused(t, fused(t, fused(kq[kq2C3], t, Y), X), (g * e.s2) * w);
+}
+__host__ __device__ __forceinline__ void eq_diag(const double* kq, const PointEq& e, double a, double b, double a2,
+                                                 double b2, double& fe, double& he) {
+#pragma clang fp contract(off)
+  const double t = e.t, ga = a + a2, gb = b + b2, gg = ga * gb, ab = a * b;
+  fe = (e.rho * 0.25) * ((t + ga) * (t + gb));
+  const double t1 = fused(a2, ga, fused(b2, gb, fused(kq[kq6K], gg, (3.0 * ab) * fused(2.0, ab, a + b))));
+  const double t2 = fused(kq[kq6K], ga + gb, 3.0 * e.s2);
+  he = (e.sc * 0.125) * fused(t, fused(t, fused(kq[kqC3T], t, t2), t1), gg * e.s2);
+}
+__host__ __device__ __forceinline__ void eq_axis2(const double* kq, const PointEq& e, double a, double a2, double b2,
+                                                  double& fe, double& he) {
+#pragma clang fp contract(off)
+  const double t = e.t, g = a + a2, gp = g * (g - 2.0), s = fused(6.0, g, -1.0);
+  fe = (e.rho * (1.0 / 24.0)) * fused(t, fused(3.0, t, s), gp);
+  const double p = a * fused(a, fused(a, fused(16.0, a, 22.0), -7.0), -8.0);
+  const double X = fused(kq[kqK], gp, fused(s, b2, p));
+  const double Y = fused(kq[kqK], s, fused(3.0, b2, fused(a, fused(51.0, a, 36.0), -4.0)));
+  he = (e.sc * (1.0 / 48.0)) * fused(t, fused(t, fused(kq[kqC3], t, Y), X), gp * e.s2);
+}
+
+template <int I>
+__host__ __device__ __forceinline__ void eq_point(const double* kq, const PointEq& e, double& fe, double& he) {
+  constexpr int base = eq_base(I);
+  const double a = eq_sa(I) * (eq_swap(I) ? e.v : e.u), b = eq_sb(I) * (eq_swap(I) ? e.u : e.v);
+  const double a2 = eq_swap(I) ? e.v2 : e.u2, b2 = eq_swap(I) ? e.u2 : e.v2;
+  if constexpr (base == 0) eq_rest(kq, e, fe, he);
+  else if constexpr (base == 1) eq_axis(kq, e, a, a2, b2, fe, he);
+  else if constexpr (base == 5) eq_diag(kq, e, a, b, a2, b2, fe, he);
+  else eq_axis2(kq, e, a, a2, b2, fe, he);
+}
+
+// Stages 1 and 2 (cpuLBM.cpp:1819-1924) in closed form. With af = dt/(2 tf),
+// ah = dt/(2 th), ahf = dt/(2 thf), r = 1/(1 + af), rh = 1/(1 + ah) the two
+// implicit stages give (feq2 = feq1 = fe, heq2 = heq1 = he)
+//   f2 = fe + q (f - fe),   q = (1 + 2 af) r^2
+//   h2 = he + qh (h - he) + mu (e.u) (f - fe),
+//        qh = (1 + 2 ah) rh^2, mu = ahf rh (q - rh r).
+struct Relax12 {
+  double q, qh, mu;
+  double cU, cV;  // c ux, c uy: e.u = lat_x cU + lat_y cV
+};
+__host__ __device__ __forceinline__ Relax12 make_relax12(const InstDev& in, const Macro& m) {
+#pragma clang fp contract(off)
+  Relax12 R;
+  const double hdt = in.dt * 0.5, af = hdt * m.itf, ah = hdt * m.ith, ahf = hdt * m.ithf;
+  const double r = 1.0 / (1.0 + af), rh = 1.0 / (1.0 + ah);
+  R.q = fused(2.0, af, 1.0) * (r * r);
+  R.qh = fused(2.0, ah, 1.0) * (rh * rh);
+  R.mu = (ahf * rh) * fused(-rh, r, R.q);
+  R.cU = in.c * m.ux;
+  R.cV = in.c * m.uy;
+  return R;
+}
+__host__ __device__ __forceinline__ void point_s12(const Relax12& R, double lx, double ly, double f, double h, double fe,
+                                                   double he, double& f2, double& h2) {
+#pragma clang fp contract(off)
+  const double eu = fused(lx, R.cU, ly * R.cV), y = f - fe, x = h - he;
+  f2 = fused(R.q, y, fe);
+  h2 = fused(R.qh, x, fused(R.mu * eu, y, he));
+}
+
+// Stage 3 (cpuLBM.cpp:1926-1993) from the stage-2 distributions, which carry
+// the moments and, through the closed forms above, the values of f and h: with
+// D = fe - f2, E = he - h2, f = fe - D/q and h from h2 likewise,
+//   P = f - dF2 + af D            = fe - ka D - dF2
+//   Q = (h - dH2) - ahf eu D + ah E = he - kh E - la (e.u) D - dH2
+//   ka = (1 + af - af^2)/(1 + 2 af), kh the same in ah,
+//   la = ahf (ah + (1 + af)/(1 + 2 af))/(1 + 2 ah)
+//   f3 = (P + af3 fe3)/(1 + af3)
+//   h3 = (Q - ahf3 eu3 (fe3 - f3) + ah3 he3)/(1 + ah3).
+// So the state itself is not read again after stage 2. The rounding of f2
+// enters f3 as ka eps/(1 + af3), at most af/(1 + af3) eps as in the form with
+// f and af (fe - f2): bounded for stiff cells too.
+struct Relax3 {
+  double ka, kh, la, cU, cV;          // stage-1 moments
+  double af3, ah3, ahf3, iaf3, iah3;  // stage-3 moments
+  double cU3, cV3;
+};
+__host__ __device__ __forceinline__ Relax3 make_relax3(const InstDev& in, const Macro& m, const Macro& m3) {
+#pragma clang fp contract(off)
+  Relax3 R;
+  const double hdt = in.dt * 0.5, af = hdt * m.itf, ah = hdt * m.ith, ahf = hdt * m.ithf;
+  const double i1 = 1.0 / fused(2.0, af, 1.0), i2 = 1.0 / fused(2.0, ah, 1.0);
+  R.ka = fused(-af, af, 1.0 + af) * i1;
+  R.kh = fused(-ah, ah, 1.0 + ah) * i2;
+  R.la = (ahf * fused(1.0 + af, i1, ah)) * i2;
+  R.cU = in.c * m.ux;
+  R.cV = in.c * m.uy;
+  R.af3 = hdt * m3.itf;
+  R.ah3 = hdt * m3.ith;
+  R.ahf3 = hdt * m3.ithf;
+  R.iaf3 = 1.0 / (1.0 + R.af3);
+  R.iah3 = 1.0 / (1.0 + R.ah3);
+  R.cU3 = in.c * m3.ux;
+  R.cV3 = in.c * m3.uy;
+  return R;
+}
+__host__ __device__ __forceinline__ void point_s3(const Relax3& R, double lx, double ly, double f2, double h2, double dF,
+                                                  double dH, double fe, double he, double fe3, double he3, double& f3,
+                                                  double& h3) {
+#pragma clang fp contract(off)
+  const double eu = fused(lx, R.cU, ly * R.cV), eu3 = fused(lx, R.cU3, ly * R.cV3);
+  const double D = fe - f2, E = he - h2;
+  const double P = fused(-R.ka, D, fe) - dF;
+  const double Q = fused(-(R.la * eu), D, fused(-R.kh, E, he)) - dH;
+  f3 = fused(R.af3, fe3, P) * R.iaf3;
+  h3 = fused(R.ah3, he3, fused(-(R.ahf3 * eu3), fe3 - f3, Q)) * R.iah3;
+}
+
+}  // namespace uqlbm

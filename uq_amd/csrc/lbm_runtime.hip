@@ -21,6 +21,7 @@
 #include "lbm_common.hpp"
 #include "lbm_device.hpp"
 #include "lbm_launch.hpp"
+#include "lbm_point.hpp"
 #include "lbm_runtime.hpp"
 
 namespace uqlbm {
@@ -519,6 +520,7 @@ static void fill_inst(const Solver& s, InstDev& d) {
   d.ibR = 1.0 / d.bR;
   d.imu = 1.0 / d.mu;
   d.Pr_m1 = d.Pr - 1.0;
+  point_consts(s.K, d.kq);
   d.visc_model = s.visc_model;
   d.mu_ref = s.mu_ref;
   d.T_ref_v = s.T_ref_v;
