@@ -74,8 +74,8 @@ int main() {
           const double f = fe * (1 + 0.1 * amp * U(rng)), h = he * (1 + 0.1 * amp * U(rng));
           const double dF = 0.05 * fe * U(rng), dH = 0.05 * he * U(rng);
           double f2, h2, f3, h3;
-          point_s12(r, lat_x(I), lat_y(I), f, h, fe, he, f2, h2);
-          point_s3(r3, lat_x(I), lat_y(I), f2, h2, dF, dH, fe, he, fe3, he3, f3, h3);
+          point_s12(r, e, lat_x(I), lat_y(I), f, h, fe, he, f2, h2);
+          point_s3(r3, e, e3, lat_x(I), lat_y(I), f2, h2, dF, dH, fe, he, fe3, he3, f3, h3);
           const LD hdt = 0.5L, itf = m.itf, ith = m.ith, ithf = m.ithf, a = hdt * itf, b = hdt * ith;
           const LD eu = (LD)lat_x(I) * m.ux + (LD)lat_y(I) * m.uy;
           const LD f1 = (f + a * fe) / (1 + a), h1 = (h - hdt * ithf * eu * (fe - f1) + b * he) / (1 + b);

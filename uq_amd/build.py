@@ -18,7 +18,7 @@ OUT_DIR = os.path.join(HERE, "lib")
 LIB = os.path.join(OUT_DIR, "libuqlbm.so")
 OBJ_DIR = os.path.join(ROOT, "_build", "obj")
 
-SOURCES = ["lbm_kernels.hip", "lbm_strip.hip", "lbm_io.hip", "lbm_runtime.hip", "lbm_server.hip"]
+SOURCES = ["lbm_kernels.hip", "lbm_strip.hip", "lbm_fused.hip", "lbm_io.hip", "lbm_runtime.hip", "lbm_server.hip"]
 ARCH = "gfx950"
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 CXXFLAGS = [

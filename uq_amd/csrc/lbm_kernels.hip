@@ -348,7 +348,7 @@ __device__ __forceinline__ void s12_cell64(const InstDev& in, gptr<const double>
     h[i] = __builtin_nontemporal_load(&src[P * (kQ + i) + o]);
   }
   Macro m;
-  point_macro(in, cell_sums(f, h, true), m);
+  point_macro(in, in, cell_sums(f, h, true), m);
   const PointEq e = point_eq(in, m);
   const Relax12 r = make_relax12(in, m);
   auto one = [&](auto Ic) {
@@ -356,7 +356,7 @@ __device__ __forceinline__ void s12_cell64(const InstDev& in, gptr<const double>
     double fe, he, f2, h2;
     eq_point<I>(in.kq, e, fe, he);
     fes[I] = fe;
-    point_s12(r, lat_x(I), lat_y(I), f[I], h[I], fe, he, f2, h2);
+    point_s12(r, e, lat_x(I), lat_y(I), f[I], h[I], fe, he, f2, h2);
     __builtin_nontemporal_store(f2, &dst[P * I + o]);
     __builtin_nontemporal_store(h2, &dst[P * (kQ + I) + o]);
   };
@@ -366,7 +366,7 @@ __device__ __forceinline__ void s12_cell64(const InstDev& in, gptr<const double>
 
 template <typename TS, typename TC, typename TE>
 __global__ __launch_bounds__(kNT) void k_s12(const InstDev* __restrict__ insts, const TileRef* __restrict__ tiles,
-                                             int ntiles, int par, const int* stepp) {
+                                             int ntiles, int par, const int* stepp, int begin) {
   const int step = *stepp;
   for (int t = first_tile(); t < ntiles; t += gridDim.x) {
     const TileRef tr = tiles[t];
@@ -381,6 +381,16 @@ __global__ __launch_bounds__(kNT) void k_s12(const InstDev* __restrict__ insts, 
     if (as_global(in.ctype)[c.o] > 0) {
 #pragma unroll
       for (int k = 0; k < kPlanes; k++) dst[in.plane * k + c.o] = src[in.plane * k + c.o];
+      if (begin) {  // the fused step writes fluid cells only: f3 and both states once per sequence
+        const gptr<TS> f3b = as_global(reinterpret_cast<TS*>(in.f3));
+        const gptr<TS> other = as_global(reinterpret_cast<TS*>(in.state[1 ^ cur]));
+#pragma unroll
+        for (int k = 0; k < kPlanes; k++) {
+          const TS v = src[in.plane * k + c.o];
+          f3b[in.plane * k + c.o] = v;
+          other[in.plane * k + c.o] = v;
+        }
+      }
       continue;
     }
     if constexpr (sizeof(TS) == 8) s12_cell64(in, src, dst, c.o, step, MakeSeq<kQ>::type{});
@@ -504,8 +514,8 @@ __device__ __forceinline__ void s3_cell64(const InstDev& in, gptr<const double> 
   }
   const Sums s = cell_sums(f, h, true);
   Macro m1, m3;
-  point_macro(in, s, m1);
-  point_macro(in, s - cell_sums(dF, dH, false), m3);
+  point_macro(in, in, s, m1);
+  point_macro(in, in, s - cell_sums(dF, dH, false), m3);
   const PointEq e1 = point_eq(in, m1), e3 = point_eq(in, m3);
   const Relax3 r = make_relax3(in, m1, m3);
   auto one = [&](auto Ic) {
@@ -514,7 +524,7 @@ __device__ __forceinline__ void s3_cell64(const InstDev& in, gptr<const double> 
     eq_point<I>(in.kq, e1, fe, he);
     eq_point<I>(in.kq, e3, fe3, he3);
     fes[I] = fe3;
-    point_s3(r, lat_x(I), lat_y(I), f[I], h[I], dF[I], dH[I], fe, he, fe3, he3, f3, h3);
+    point_s3(r, e1, e3, lat_x(I), lat_y(I), f[I], h[I], dF[I], dH[I], fe, he, fe3, he3, f3, h3);
     // the rest direction has no flux: its f3 is the new state
     const gptr<double> dst = I == 0 ? out : f3b;
     __builtin_nontemporal_store(f3, &dst[P * I + o]);
@@ -1922,12 +1932,12 @@ static void launch_rk3(const StepLaunch& L, hipStream_t s, int par, KernelTimer*
   if (tm) tm->begin(0, s);
   per_eq_kind<TS>(L, [&](auto te, int k) {
     k_s12<TS, TP, decltype(te)><<<blocks_for(L.nptiles, G.s12[k]), kNT, 0, s>>>(L.insts, L.ptiles, L.nptiles, par,
-                                                                                step);
+                                                                                step, 0);
   });
   if (tm) tm->end(0, s);
   if (L.nwalls) {
     if (tm) tm->begin(1, s);
-    launch_alpha<TS>(L, s, 0, par);
+    launch_alpha<TS>(L, s, 0, par, step);
     if (tm) tm->end(1, s);
   }
   if (tm) tm->begin(2, s);
@@ -1941,12 +1951,33 @@ static void launch_rk3(const StepLaunch& L, hipStream_t s, int par, KernelTimer*
   if (tm) tm->end(3, s);
   if (L.nwalls) {
     if (tm) tm->begin(1, s);
-    launch_alpha<TS>(L, s, 1, par);
+    launch_alpha<TS>(L, s, 1, par, step);
     if (tm) tm->end(1, s);
   }
   if (tm) tm->begin(4, s);
   launch_flux<TS, TC, 1, kMom3<TS>, Sh>(L, s, par, g3);
   if (tm) tm->end(4, s);
+}
+
+void launch_fused_begin(const StepLaunch& L, hipStream_t s, KernelTimer* tm) {
+  static const int grid = grid_for((const void*)k_s12<double, TP, double>, kNT);
+  if (tm) tm->begin(0, s);
+  k_s12<double, TP, double><<<blocks_for(L.nptiles, grid), kNT, 0, s>>>(L.insts, L.ptiles, L.nptiles, 0, L.step_ctr, 1);
+  if (tm) tm->end(0, s);
+}
+
+void launch_fused_step(const StepLaunch& L, hipStream_t s, bool write_state, bool next_stages, KernelTimer* tm) {
+  for (int stage = 0; stage < 2; stage++) {
+    if (L.nwalls) {
+      if (tm) tm->begin(1, s);
+      launch_alpha<double>(L, s, stage, 0, L.step_ctr + stage);
+      if (tm) tm->end(1, s);
+    }
+    if (tm) tm->begin(stage ? 4 : 2, s);
+    if (stage == 0) launch_stage23(L, s);
+    else launch_stage31(L, s, write_state, next_stages);
+    if (tm) tm->end(stage ? 4 : 2, s);
+  }
 }
 
 // RKMETHOD 0, 2, 3: one flux stage.
@@ -1967,7 +1998,7 @@ static void launch_one_stage(const StepLaunch& L, hipStream_t s, int par, Kernel
   }
   if (L.nwalls) {
     if (tm) tm->begin(1, s);
-    launch_alpha<TS>(L, s, METHOD == 0 ? 0 : 2, par);
+    launch_alpha<TS>(L, s, METHOD == 0 ? 0 : 2, par, step);
     if (tm) tm->end(1, s);
   }
   if (tm) tm->begin(2, s);

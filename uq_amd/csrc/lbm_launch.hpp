@@ -22,7 +22,8 @@ struct StepLaunch {
   const TileRef* ptiles = nullptr;  // 64 x 4 row tiles of the pointwise kernels
   int nptiles = 0;
   int rk_method = 1;                // RKMETHOD shared by every instance of the group
-  int* step_ctr = nullptr;          // device step counter: step k of a sequence reads k + 1
+  int* step_ctr = nullptr;          // device step counter: step k of a sequence reads k + 1 (fused:
+                                    // two counters, of k_stage23 and of k_stage31)
   int flux_shape = 0;               // flux tile shape (flux_tile_dims); the tile list is built for it
   double* res_partial = nullptr;    // per pointwise tile residual partials (nptiles doubles) when
                                     // some instance tracks its residual; null otherwise
@@ -33,7 +34,8 @@ struct StepLaunch {
   const TileRef* strips = nullptr;  // strip work items (instances with InstDev::strips set)
   int nstrips = 0;
   const TileRef* mstrips = nullptr;  // FP32 storage: strip items of the moment-summing stage-3 flux
-  int nmstrips = 0;
+  int nmstrips = 0;                  // (FP64 storage: of the fused step)
+  int fused = 0;                    // FP64 RK3 in two launches per step (launch_fused_step)
   int far64 = 0;                    // FP32 storage far from its reference: FP64 stencils on strips
   int tiles_rest = 0;               // flux tiles of the instances not on strips
 };
@@ -60,7 +62,7 @@ inline bool same_launch(const StepLaunch& a, const StepLaunch& b) {
          a.nwalls == b.nwalls && a.ptiles == b.ptiles && a.nptiles == b.nptiles && a.rk_method == b.rk_method &&
          a.step_ctr == b.step_ctr && a.flux_shape == b.flux_shape && a.res_partial == b.res_partial && a.ninst == b.ninst &&
          a.nphys == b.nphys && a.eq_kinds == b.eq_kinds && a.strips == b.strips && a.nstrips == b.nstrips &&
-         a.mstrips == b.mstrips && a.nmstrips == b.nmstrips && a.far64 == b.far64 &&
+         a.fused == b.fused && a.mstrips == b.mstrips && a.nmstrips == b.nmstrips && a.far64 == b.far64 &&
          a.tiles_rest == b.tiles_rest;
 }
 
@@ -130,7 +132,16 @@ template <typename TS, int MODE>
 void launch_strips(const StepLaunch& L, hipStream_t s, int par);
 void launch_strips_mom(const StepLaunch& L, hipStream_t s, int par);
 template <typename TS>
-void launch_alpha(const StepLaunch& L, hipStream_t s, int which, int par);
+void launch_alpha(const StepLaunch& L, hipStream_t s, int which, int par, const int* step);
+
+// The RK3 step of FP64 storage in two launches (lbm_fused.hip): fused_begin
+// forms f2 of the first step from the state; then each step is
+// launch_fused_step, writing the new state (write_state) and f2 of the next
+// step (next_stages).
+void launch_stage23(const StepLaunch& L, hipStream_t s);
+void launch_stage31(const StepLaunch& L, hipStream_t s, bool write_state, bool next_stages);
+void launch_fused_begin(const StepLaunch& L, hipStream_t s, KernelTimer* tm);
+void launch_fused_step(const StepLaunch& L, hipStream_t s, bool write_state, bool next_stages, KernelTimer* tm);
 
 // Computes the persistent grid sizes of the step kernels (call before a
 // stream capture).

@@ -60,8 +60,13 @@ __host__ __device__ __forceinline__ Sums cell_sums(const double* f, const double
   return ((a + quad_sums_of<1>(f, h)) + quad_sums_of<2>(f, h)) + quad_sums_of<3>(f, h);
 }
 
+// The functions below take the instance record as they are given it (In: the
+// record, or the record in the constant address space) and the coefficients
+// as part of it (KQ).
+//
 // Moments of a cell (reference macroProp, cpuLBM.cpp:916-970).
-__device__ __forceinline__ void point_macro(const InstDev& in, const Sums& s, Macro& m) {
+template <typename In>
+__device__ __forceinline__ void point_macro(const In& in, const InstDev& inst, const Sums& s, Macro& m) {
 #pragma clang fp contract(off)
   const double irho = 1.0 / s.m;
   m.rho = s.m;
@@ -70,7 +75,7 @@ __device__ __forceinline__ void point_macro(const InstDev& in, const Sums& s, Ma
   const double usq = fused(m.ux, m.ux, m.uy * m.uy);
   m.T = fused(2.0, s.e * irho, -usq) * in.ibR;
   m.p = (m.rho * in.R) * m.T;
-  m.itf = in.visc_model == 0 ? m.p * in.imu : m.p / viscosity_of(in, m.T);
+  m.itf = in.visc_model == 0 ? m.p * in.imu : m.p / viscosity_of(inst, m.T);
   m.ith = m.itf * in.Pr;
   m.ithf = m.itf * in.Pr_m1;
 }
@@ -108,7 +113,8 @@ struct PointEq {
   double rho, sc;              // density, rho R Tc
 };
 
-__host__ __device__ __forceinline__ PointEq point_eq(const InstDev& in, const Macro& m) {
+template <typename In>
+__host__ __device__ __forceinline__ PointEq point_eq(const In& in, const Macro& m) {
 #pragma clang fp contract(off)
   PointEq e;
   e.rho = m.rho;
@@ -123,7 +129,8 @@ __host__ __device__ __forceinline__ PointEq point_eq(const InstDev& in, const Ma
 }
 
 // The four kinds of directions at (a, b): rest, axis, diagonal, double axis.
-__host__ __device__ __forceinline__ void eq_rest(const double* kq, const PointEq& e, double& fe, double& he) {
+template <typename KQ>
+__host__ __device__ __forceinline__ void eq_rest(const KQ& kq, const PointEq& e, double& fe, double& he) {
 #pragma clang fp contract(off)
   const double uv = e.u2 * e.v2, t = e.t, s2 = e.s2;
   const double Z = fused(s2, s2 - 5.0, fused(2.0, uv, 4.0));
@@ -132,7 +139,8 @@ __host__ __device__ __forceinline__ void eq_rest(const double* kq, const PointEq
   const double t2 = fused(kq[kqI], s2, kq[kqJ]);
   he = (e.sc * (1.0 / 24.0)) * fused(t, fused(t, fused(kq[kq10C3], t, t2), t1), 3.0 * (s2 * Z));
 }
-__host__ __device__ __forceinline__ void eq_axis(const double* kq, const PointEq& e, double a, double a2, double b2,
+template <typename KQ>
+__host__ __device__ __forceinline__ void eq_axis(const KQ& kq, const PointEq& e, double a, double a2, double b2,
                                                  double& fe, double& he) {
 #pragma clang fp contract(off)
   const double t = e.t, g = a + a2;
@@ -144,7 +152,8 @@ __host__ __device__ __forceinline__ void eq_axis(const double* kq, const PointEq
   const double Y = fused(kq[kqK], z, fused(30.0, b2, fused(a, fused(78.0, a, 36.0), -16.0)));
   he = (e.sc * (-1.0 / 12.0)) * fused(t, fused(t, fused(kq[kq2C3], t, Y), X), (g * e.s2) * w);
 }
-__host__ __device__ __forceinline__ void eq_diag(const double* kq, const PointEq& e, double a, double b, double a2,
+template <typename KQ>
+__host__ __device__ __forceinline__ void eq_diag(const KQ& kq, const PointEq& e, double a, double b, double a2,
                                                  double b2, double& fe, double& he) {
 #pragma clang fp contract(off)
   const double t = e.t, ga = a + a2, gb = b + b2, gg = ga * gb, ab = a * b;
@@ -153,7 +162,8 @@ __host__ __device__ __forceinline__ void eq_diag(const double* kq, const PointEq
   const double t2 = fused(kq[kq6K], ga + gb, 3.0 * e.s2);
   he = (e.sc * 0.125) * fused(t, fused(t, fused(kq[kqC3T], t, t2), t1), gg * e.s2);
 }
-__host__ __device__ __forceinline__ void eq_axis2(const double* kq, const PointEq& e, double a, double a2, double b2,
+template <typename KQ>
+__host__ __device__ __forceinline__ void eq_axis2(const KQ& kq, const PointEq& e, double a, double a2, double b2,
                                                   double& fe, double& he) {
 #pragma clang fp contract(off)
   const double t = e.t, g = a + a2, gp = g * (g - 2.0), s = fused(6.0, g, -1.0);
@@ -164,8 +174,8 @@ __host__ __device__ __forceinline__ void eq_axis2(const double* kq, const PointE
   he = (e.sc * (1.0 / 48.0)) * fused(t, fused(t, fused(kq[kqC3], t, Y), X), gp * e.s2);
 }
 
-template <int I>
-__host__ __device__ __forceinline__ void eq_point(const double* kq, const PointEq& e, double& fe, double& he) {
+template <int I, typename KQ>
+__host__ __device__ __forceinline__ void eq_point(const KQ& kq, const PointEq& e, double& fe, double& he) {
   constexpr int base = eq_base(I);
   const double a = eq_sa(I) * (eq_swap(I) ? e.v : e.u), b = eq_sb(I) * (eq_swap(I) ? e.u : e.v);
   const double a2 = eq_swap(I) ? e.v2 : e.u2, b2 = eq_swap(I) ? e.u2 : e.v2;
@@ -181,26 +191,26 @@ __host__ __device__ __forceinline__ void eq_point(const double* kq, const PointE
 //   f2 = fe + q (f - fe),   q = (1 + 2 af) r^2
 //   h2 = he + qh (h - he) + mu (e.u) (f - fe),
 //        qh = (1 + 2 ah) rh^2, mu = ahf rh (q - rh r).
+// e.u is R Tc (lat_x u + lat_y v) with the normalised velocity u, v of PointEq
+// (c = sqrt(R Tc)): the coefficients of e.u carry the factor R Tc.
 struct Relax12 {
   double q, qh, mu;
-  double cU, cV;  // c ux, c uy: e.u = lat_x cU + lat_y cV
 };
-__host__ __device__ __forceinline__ Relax12 make_relax12(const InstDev& in, const Macro& m) {
+template <typename In>
+__host__ __device__ __forceinline__ Relax12 make_relax12(const In& in, const Macro& m) {
 #pragma clang fp contract(off)
   Relax12 R;
   const double hdt = in.dt * 0.5, af = hdt * m.itf, ah = hdt * m.ith, ahf = hdt * m.ithf;
   const double r = 1.0 / (1.0 + af), rh = 1.0 / (1.0 + ah);
   R.q = fused(2.0, af, 1.0) * (r * r);
   R.qh = fused(2.0, ah, 1.0) * (rh * rh);
-  R.mu = (ahf * rh) * fused(-rh, r, R.q);
-  R.cU = in.c * m.ux;
-  R.cV = in.c * m.uy;
+  R.mu = ((ahf * rh) * fused(-rh, r, R.q)) * in.RTc;
   return R;
 }
-__host__ __device__ __forceinline__ void point_s12(const Relax12& R, double lx, double ly, double f, double h, double fe,
-                                                   double he, double& f2, double& h2) {
+__host__ __device__ __forceinline__ void point_s12(const Relax12& R, const PointEq& e, double lx, double ly, double f,
+                                                   double h, double fe, double he, double& f2, double& h2) {
 #pragma clang fp contract(off)
-  const double eu = fused(lx, R.cU, ly * R.cV), y = f - fe, x = h - he;
+  const double eu = fused(lx, e.u, ly * e.v), y = f - fe, x = h - he;
   f2 = fused(R.q, y, fe);
   h2 = fused(R.qh, x, fused(R.mu * eu, y, he));
 }
@@ -218,34 +228,30 @@ __host__ __device__ __forceinline__ void point_s12(const Relax12& R, double lx, 
 // enters f3 as ka eps/(1 + af3), at most af/(1 + af3) eps as in the form with
 // f and af (fe - f2): bounded for stiff cells too.
 struct Relax3 {
-  double ka, kh, la, cU, cV;          // stage-1 moments
+  double ka, kh, la;                  // stage-1 moments
   double af3, ah3, ahf3, iaf3, iah3;  // stage-3 moments
-  double cU3, cV3;
 };
-__host__ __device__ __forceinline__ Relax3 make_relax3(const InstDev& in, const Macro& m, const Macro& m3) {
+template <typename In>
+__host__ __device__ __forceinline__ Relax3 make_relax3(const In& in, const Macro& m, const Macro& m3) {
 #pragma clang fp contract(off)
   Relax3 R;
   const double hdt = in.dt * 0.5, af = hdt * m.itf, ah = hdt * m.ith, ahf = hdt * m.ithf;
   const double i1 = 1.0 / fused(2.0, af, 1.0), i2 = 1.0 / fused(2.0, ah, 1.0);
   R.ka = fused(-af, af, 1.0 + af) * i1;
   R.kh = fused(-ah, ah, 1.0 + ah) * i2;
-  R.la = (ahf * fused(1.0 + af, i1, ah)) * i2;
-  R.cU = in.c * m.ux;
-  R.cV = in.c * m.uy;
+  R.la = ((ahf * fused(1.0 + af, i1, ah)) * i2) * in.RTc;
   R.af3 = hdt * m3.itf;
   R.ah3 = hdt * m3.ith;
-  R.ahf3 = hdt * m3.ithf;
+  R.ahf3 = (hdt * m3.ithf) * in.RTc;
   R.iaf3 = 1.0 / (1.0 + R.af3);
   R.iah3 = 1.0 / (1.0 + R.ah3);
-  R.cU3 = in.c * m3.ux;
-  R.cV3 = in.c * m3.uy;
   return R;
 }
-__host__ __device__ __forceinline__ void point_s3(const Relax3& R, double lx, double ly, double f2, double h2, double dF,
-                                                  double dH, double fe, double he, double fe3, double he3, double& f3,
-                                                  double& h3) {
+__host__ __device__ __forceinline__ void point_s3(const Relax3& R, const PointEq& e, const PointEq& e3, double lx,
+                                                  double ly, double f2, double h2, double dF, double dH, double fe,
+                                                  double he, double fe3, double he3, double& f3, double& h3) {
 #pragma clang fp contract(off)
-  const double eu = fused(lx, R.cU, ly * R.cV), eu3 = fused(lx, R.cU3, ly * R.cV3);
+  const double eu = fused(lx, e.u, ly * e.v), eu3 = fused(lx, e3.u, ly * e3.v);
   const double D = fe - f2, E = he - h2;
   const double P = fused(-R.ka, D, fe) - dF;
   const double Q = fused(-(R.la * eu), D, fused(-R.kh, E, he)) - dH;

@@ -671,6 +671,17 @@ static int strip_rows(const std::vector<Solver*>& members, int waves) {
   return h;
 }
 
+// The fused step takes FP64 RK3 groups whose members all have strips and
+// arrays within the 32-bit offsets of its buffer accesses (19 million cells);
+// the others keep four launches a step. Not a matter of size otherwise: it is
+// the faster one from 64^2 (39 against 43 us per step) over an ensemble of 48
+// (1561, 1697) to 3072^2 (3287, 3943).
+static constexpr unsigned long long kFusedMaxBytes = 0xF0000000ull;
+static bool fused_instance(const Solver& s) {
+  return s.precision == LBM_PREC_FP64 && s.p.rk_method == 1 && s.strip_cols > 0 &&
+         (unsigned long long)s.pitch * s.ny * kPlanes * sizeof(double) <= kFusedMaxBytes;
+}
+
 uqlbm::StripLists::StripLists(const std::vector<Solver*>& members, int shape) {
   const int rows = strip_rows(members, 12);
   for (size_t k = 0; k < members.size(); k++) {
@@ -679,14 +690,18 @@ uqlbm::StripLists::StripLists(const std::vector<Solver*>& members, int shape) {
     if (members[k]->strip_cols == 0) tiles_rest += (int)solver_tiles(*members[k], shape).size();
   }
   n = (int)items.size();
-  if (members.empty() || members[0]->precision == LBM_PREC_FP64) return;
+  // items of k_strip_mom, or of the fused step: four wavefronts each
   const int mrows = strip_rows(members, 4);
-  for (size_t k = 0; k < members.size(); k++) strip_items(*members[k], mrows, (int)k, items);
+  fused = !members.empty();
+  for (size_t k = 0; k < members.size(); k++) {
+    strip_items(*members[k], mrows, (int)k, items);
+    fused = fused && fused_instance(*members[k]);
+  }
   nmom = (int)items.size() - n;
 }
 
-void uqlbm::launch_strips_of(StepLaunch& L, const TileRef* items_dev, int n, int nmom, int blocks, int tiles_rest,
-                             int ntiles) {
+void uqlbm::launch_strips_of(StepLaunch& L, const TileRef* items_dev, int n, int nmom, bool fused, int blocks,
+                             int tiles_rest, int ntiles) {
   if (!strips_enabled() || n == 0) {
     L.tiles_rest = ntiles;
     return;
@@ -695,6 +710,7 @@ void uqlbm::launch_strips_of(StepLaunch& L, const TileRef* items_dev, int n, int
   L.nstrips = n;
   L.mstrips = items_dev + n;
   L.nmstrips = nmom;
+  L.fused = fused;
   L.far64 = far_fp64(blocks);
   L.tiles_rest = tiles_rest;
 }
@@ -811,7 +827,7 @@ extern "C" int lbm_create(const lbm_params* params, int32_t nx, int32_t ny, cons
   HIP_TRY(solver_alloc(*s, (void**)&s->props_dev, s->props.size() * 4 * sizeof(double)));
   HIP_TRY(solver_alloc(*s, (void**)&s->inst_dev, sizeof(InstDev)));
   HIP_TRY(solver_alloc(*s, (void**)&s->macro_dev, plane * 5 * sizeof(double)));
-  HIP_TRY(solver_alloc(*s, (void**)&s->step_ctr, sizeof(int)));
+  HIP_TRY(solver_alloc(*s, (void**)&s->step_ctr, 2 * sizeof(int)));
   HIP_TRY(solver_alloc(*s, (void**)&s->fails_dev, sizeof(int)));
   s->device_bytes = solver_footprint(nx, ny, precision);
 
@@ -859,6 +875,7 @@ extern "C" int lbm_create(const lbm_params* params, int32_t nx, int32_t ny, cons
   const StripLists strips({s.get()}, s->flux_shape);
   s->nstrips = strips.n;
   s->nmstrips = strips.nmom;
+  s->fused = strips.fused;
   if (s->nstrips) {
     HIP_TRY(solver_alloc(*s, (void**)&s->strips_dev, strips.items.size() * sizeof(TileRef)));
     HIP_TRY(hipMemcpy(s->strips_dev, strips.items.data(), strips.items.size() * sizeof(TileRef), hipMemcpyHostToDevice));
@@ -895,6 +912,9 @@ int uqlbm::upload_inst(Solver& s) {
   return LBM_OK;
 }
 
+// Steps of a captured fused graph.
+static constexpr int kFusedGraph = 8;
+
 static void launch_steps(const StepLaunch& L, int precision, hipStream_t stream, int nsteps,
                          KernelTimer* tm) {
   for (int k = 0; k < nsteps; k++) {
@@ -923,6 +943,38 @@ static int capture_steps(const StepLaunch& L, int precision, hipStream_t stream,
   const hipError_t e2 = hipGraphInstantiate(out, g, nullptr, nullptr, 0);
   (void)hipGraphDestroy(g);
   if (e2 != hipSuccess) return fail_with(LBM_ERR_HIP, "graph instantiate: %s", hipGetErrorString(e2));
+  return LBM_OK;
+}
+
+// n steps of the fused step: the first step's f2 from the state, then steps
+// that keep the state in f2 (through a cached graph of kFusedGraph of them
+// where `gc` is given and the sequence is long enough), and the last two,
+// which write the state.
+static int fused_steps(GraphCache* gc, const StepLaunch& L, hipStream_t stream, int n, KernelTimer* tm) {
+  launch_fused_begin(L, stream, tm);
+  int left = n - 2;
+  if (gc && left >= kFusedGraph) {
+    if (gc->precision != LBM_PREC_FP64 || !same_launch(gc->key, L)) {
+      gc->clear();
+      hipGraph_t g = nullptr;
+      HIP_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
+      for (int k = 0; k < kFusedGraph; k++) launch_fused_step(L, stream, false, true, nullptr);
+      const hipError_t e = hipStreamEndCapture(stream, &g);
+      if (e != hipSuccess) return fail_with(LBM_ERR_HIP, "stream capture: %s", hipGetErrorString(e));
+      const hipError_t e2 = hipGraphInstantiate(&gc->two, g, nullptr, nullptr, 0);
+      (void)hipGraphDestroy(g);
+      if (e2 != hipSuccess) {
+        gc->clear();
+        return fail_with(LBM_ERR_HIP, "graph instantiate: %s", hipGetErrorString(e2));
+      }
+      gc->key = L;
+      gc->precision = LBM_PREC_FP64;
+    }
+    for (; left >= kFusedGraph; left -= kFusedGraph) HIP_TRY(hipGraphLaunch(gc->two, stream));
+  }
+  for (; left > 0; left--) launch_fused_step(L, stream, false, true, tm);
+  if (n > 1) launch_fused_step(L, stream, true, true, tm);
+  launch_fused_step(L, stream, true, false, tm);
   return LBM_OK;
 }
 
@@ -1001,8 +1053,12 @@ int uqlbm::run_group(const std::vector<Solver*>& members, InstDev* table_dev, co
     HIP_TRY(hipEventCreate(&e1));
     HIP_TRY(hipEventRecord(e0, stream));
   }
-  if (graphs && g_graphs_enabled && !tm) {
-    const int st = replay_steps(*graphs, L, precision, stream, n);
+  // per-step residuals need every step's state: four launches per step then
+  const bool fused = L.fused && !L.res_partial;
+  const bool replay = graphs && g_graphs_enabled && !tm;
+  if (fused || replay) {
+    const int st = fused ? fused_steps(replay ? graphs : nullptr, L, stream, n, tm)
+                         : replay_steps(*graphs, L, precision, stream, n);
     if (st != LBM_OK) {
       (void)hipStreamSynchronize(stream);
       return st;
@@ -1062,7 +1118,7 @@ extern "C" int lbm_step(lbm_solver* h, int32_t nsteps, int32_t want_residual, do
   StepLaunch L{s.inst_dev,    s.tiles_dev, s.ntiles,      s.walls_dev, s.nwalls,
                s.ptiles_dev, s.nptiles,   s.p.rk_method, s.step_ctr,  s.flux_shape};
   L.nphys = s.nphys;
-  launch_strips_of(L, s.strips_dev, s.nstrips, s.nmstrips, s.strip_blocks, 0, s.ntiles);
+  launch_strips_of(L, s.strips_dev, s.nstrips, s.nmstrips, s.fused, s.strip_blocks, 0, s.ntiles);
   L.eq_kinds = s.precision == LBM_PREC_FP64 ? 1 : (s.eq32 ? 2 : 1);
   std::vector<Solver*> one{&s};
   const int st = run_group(one, s.inst_dev, L, s.precision, s.stream, nsteps, s.graphs.get(), s.fails_dev, true);
@@ -1131,7 +1187,7 @@ extern "C" int lbm_step_noalloc(lbm_solver* h, int32_t nsteps, int32_t want_resi
   StepLaunch L{s.inst_dev,    s.tiles_dev, s.ntiles,      s.walls_dev, s.nwalls,
                s.ptiles_dev, s.nptiles,   s.p.rk_method, s.step_ctr,  s.flux_shape};
   L.nphys = s.nphys;
-  launch_strips_of(L, s.strips_dev, s.nstrips, s.nmstrips, s.strip_blocks, 0, s.ntiles);
+  launch_strips_of(L, s.strips_dev, s.nstrips, s.nmstrips, s.fused, s.strip_blocks, 0, s.ntiles);
   L.eq_kinds = s.precision == LBM_PREC_FP64 ? 1 : (s.eq32 ? 2 : 1);
   prepare_launch(s.precision == LBM_PREC_FP64);
   std::vector<Solver*> one{&s};
@@ -1380,7 +1436,7 @@ int uqlbm::batch_finish(Batch& b, lbm_batch** out) {
   b.nptiles = (int)ptiles.size();
   HIP_TRY(hipStreamCreateWithFlags(&b.stream, hipStreamNonBlocking));
   HIP_TRY(hipMalloc((void**)&b.inst_dev, b.members.size() * sizeof(InstDev)));
-  HIP_TRY(hipMalloc((void**)&b.step_ctr, sizeof(int)));
+  HIP_TRY(hipMalloc((void**)&b.step_ctr, 2 * sizeof(int)));
   HIP_TRY(hipMalloc((void**)&b.fails_dev, b.members.size() * sizeof(int)));
   int st = batch_set_shape(b, default_flux_shape(b.precision));
   if (st != LBM_OK) return st;
@@ -1393,6 +1449,7 @@ int uqlbm::batch_finish(Batch& b, lbm_batch** out) {
   const StripLists strips(b.members, b.flux_shape);
   b.nstrips = strips.n;
   b.nmstrips = strips.nmom;
+  b.fused = strips.fused;
   b.strip_blocks = strips.blocks;
   b.tiles_rest = strips.tiles_rest;
   if (b.nstrips) {
@@ -1418,7 +1475,7 @@ int uqlbm::batch_step(Batch& b, int nsteps) {
                b.ptiles_dev, b.nptiles,   b.rk_method, b.step_ctr,  b.flux_shape};
   L.nphys = b.nphys;
   L.eq_kinds = b.eq_kinds;
-  launch_strips_of(L, b.strips_dev, b.nstrips, b.nmstrips, b.strip_blocks, b.tiles_rest, b.ntiles);
+  launch_strips_of(L, b.strips_dev, b.nstrips, b.nmstrips, b.fused, b.strip_blocks, b.tiles_rest, b.ntiles);
   int st = run_group(b.members, b.inst_dev, L, b.precision, b.stream, nsteps, b.graphs.get(), b.fails_dev, true);
   for (Solver* s : b.members) {
     int st2 = upload_inst(*s);

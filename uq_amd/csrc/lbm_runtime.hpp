@@ -15,8 +15,9 @@
 namespace uqlbm {
 
 // Instantiated HIP graphs of one launch group's step sequence: two steps
-// (buffer parities 0 and 1, so that it replays back to back) and one step.
-// Valid while the group's launch description is unchanged.
+// (buffer parities 0 and 1, so that it replays back to back) and one step; of
+// the fused step kFusedGraph steps (`two`). Valid while the group's launch
+// description is unchanged.
 struct GraphCache {
   StepLaunch key{};
   int precision = -1;
@@ -93,7 +94,8 @@ struct Solver {
   std::vector<std::pair<void*, size_t>> owned;  // buffers from solver_alloc, returned to its cache
   int ntiles = 0, nwalls = 0, nptiles = 0;
   int nphys = 0;  // flux tiles flagged kTilePhysical
-  int nstrips = 0, nmstrips = 0;    // items of k_strip, then of k_strip_mom in strips_dev
+  int nstrips = 0, nmstrips = 0;    // items of k_strip, then of k_strip_mom (FP64: the fused step) in strips_dev
+  bool fused = false;               // takes the fused step (StripLists)
   size_t device_bytes = 0;
 
   int cur = 0;    // state buffer holding the current state
@@ -126,6 +128,7 @@ struct Batch {
   int nphys = 0;  // flux tiles flagged kTilePhysical
   int eq_kinds = 1;  // equilibrium precisions among the members (StepLaunch::eq_kinds)
   int nstrips = 0, nmstrips = 0, strip_blocks = 0, tiles_rest = 0;
+  bool fused = false;
   Batch() = default;
   Batch(Batch&& o) noexcept { *this = std::move(o); }
   Batch& operator=(Batch&& o) noexcept {
@@ -150,6 +153,7 @@ struct Batch {
     eq_kinds = o.eq_kinds;
     nstrips = o.nstrips;
     nmstrips = o.nmstrips;
+    fused = o.fused;
     strip_blocks = o.strip_blocks;
     tiles_rest = o.tiles_rest;
     o.stream = nullptr;
@@ -195,10 +199,12 @@ struct StripLists {
   int n = 0, nmom = 0;  // items of k_strip, of k_strip_mom
   int blocks = 0;       // the group's 32-row strip items
   int tiles_rest = 0;   // flux tiles of shape `shape` of the members not on strips
+  bool fused = false;   // the members take the fused step
   StripLists(const std::vector<Solver*>& members, int shape);
 };
 // The strip fields of a launch description; `ntiles`: the group's flux tiles.
-void launch_strips_of(StepLaunch& L, const TileRef* items_dev, int n, int nmom, int blocks, int tiles_rest, int ntiles);
+void launch_strips_of(StepLaunch& L, const TileRef* items_dev, int n, int nmom, bool fused, int blocks, int tiles_rest,
+                      int ntiles);
 const std::vector<TileRef>& solver_tiles(Solver& s, int shape);
 int default_flux_shape(int precision);
 int batch_set_shape(Batch& b, int shape);

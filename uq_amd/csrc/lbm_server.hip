@@ -68,7 +68,8 @@ struct Server {
   TileRef* strips_dev = nullptr;
   size_t tiles_cap = 0, walls_cap = 0, ptiles_cap = 0, strips_cap = 0;
   int ntiles = 0, nwalls = 0, nptiles = 0;
-  int nstrips = 0, nmstrips = 0, strip_blocks = 0, tiles_rest = 0;  // strip list of the active requests (StepLaunch)
+  int nstrips = 0, nmstrips = 0, strip_blocks = 0, tiles_rest = 0;
+  bool fused = false;  // strip list of the active requests (StepLaunch)
   int nphys = 0;  // flux tiles flagged kTilePhysical
   int eq_kinds = 1;  // equilibrium precisions among the active requests (StepLaunch::eq_kinds)
   bool lists_dirty = true;
@@ -137,6 +138,7 @@ static int rebuild_lists(Server& sv) {
   const StripLists strips(members, sv.flux_shape);
   sv.nstrips = strips.n;
   sv.nmstrips = strips.nmom;
+  sv.fused = strips.fused;
   sv.strip_blocks = strips.blocks;
   sv.tiles_rest = strips.tiles_rest;
   if (strips.items.size() > sv.strips_cap) {
@@ -301,7 +303,7 @@ extern "C" int lbm_server_create(int32_t precision, int32_t rk_method, size_t hb
   sv->max_slots = max_slots;
   SV_TRY(hipStreamCreateWithFlags(&sv->stream, hipStreamNonBlocking));
   SV_TRY(hipMalloc((void**)&sv->table_dev, (size_t)max_slots * sizeof(InstDev)));
-  SV_TRY(hipMalloc((void**)&sv->step_ctr, sizeof(int)));
+  SV_TRY(hipMalloc((void**)&sv->step_ctr, 2 * sizeof(int)));
   SV_TRY(hipMalloc((void**)&sv->fails_dev, (size_t)max_slots * sizeof(int)));
   *out = reinterpret_cast<lbm_server*>(sv.release());
   return LBM_OK;
@@ -367,7 +369,7 @@ extern "C" int lbm_server_tick(lbm_server* h, int32_t tick_steps, int32_t* activ
                  sv.ptiles_dev, sv.nptiles,   sv.rk_method, sv.step_ctr,  sv.flux_shape};
     L.nphys = sv.nphys;
     L.eq_kinds = sv.eq_kinds;
-    launch_strips_of(L, sv.strips_dev, sv.nstrips, sv.nmstrips, sv.strip_blocks, sv.tiles_rest, sv.ntiles);
+    launch_strips_of(L, sv.strips_dev, sv.nstrips, sv.nmstrips, sv.fused, sv.strip_blocks, sv.tiles_rest, sv.ntiles);
     if (track) {
       L.res_partial = sv.res_partial;
       L.ninst = (int)members.size();

@@ -79,10 +79,10 @@ __global__ __launch_bounds__(kWallBlock) void k_alpha(const InstDev* __restrict_
 }
 
 template <typename TS>
-void launch_alpha(const StepLaunch& L, hipStream_t s, int which, int par) {
+void launch_alpha(const StepLaunch& L, hipStream_t s, int which, int par, const int* step) {
   constexpr int cells = kWallBlock / kWallLanes;
   k_alpha<TS, double><<<(L.nwalls + cells - 1) / cells, kWallBlock, 0, s>>>(L.insts, L.walls, L.nwalls, which, par,
-                                                                            L.step_ctr);
+                                                                            step);
 }
 
 // Compute type of the strip kernels: FP64 for FP64 storage; FP32 for FP32
@@ -113,8 +113,8 @@ void launch_strips_mom(const StepLaunch& L, hipStream_t s, int par) {
   k_strip_mom<float, float><<<8 * chunk, 256, 0, s>>>(L.insts, L.mstrips, L.nmstrips, chunk, par, L.step_ctr);
 }
 
-template void launch_alpha<double>(const StepLaunch&, hipStream_t, int, int);
-template void launch_alpha<float>(const StepLaunch&, hipStream_t, int, int);
+template void launch_alpha<double>(const StepLaunch&, hipStream_t, int, int, const int*);
+template void launch_alpha<float>(const StepLaunch&, hipStream_t, int, int, const int*);
 template void launch_strips<double, 0>(const StepLaunch&, hipStream_t, int);
 template void launch_strips<double, 1>(const StepLaunch&, hipStream_t, int);
 template void launch_strips<double, 2>(const StepLaunch&, hipStream_t, int);
