@@ -30,6 +30,7 @@
 // second LDS buffer with direct-to-LDS loads while the faces of the current
 // one are computed; FP64 stages through registers.
 #include <climits>
+#include <cstring>
 #include <type_traits>
 
 #include "lbm_device.hpp"
@@ -1706,7 +1707,9 @@ int totals_scratch_doubles() { return 4 * kRedBlocks + 4; }
 // other state buffer, which a step leaves untouched) and the current one.
 // Deterministic two-level FP64 reduction: one partial sum per grid row
 // (rows[y], wavefront shuffles within the row's block), then one block adds
-// the rows in a fixed order and writes sqrt(sum / (nx ny)) to rows[ny].
+// the rows in a fixed order and writes sqrt(sum / (nx ny)) to *out. Launched
+// behind a sequence of `nsteps` steps, with the record it began with: where
+// the instance failed inside the sequence, the last step is the failing one.
 // ---------------------------------------------------------------------------
 template <typename TS>
 __device__ __forceinline__ double cell_T(const InstDev& in, int k, long long o) {
@@ -1718,10 +1721,11 @@ __device__ __forceinline__ double cell_T(const InstDev& in, int k, long long o) 
 }
 
 template <typename TS>
-__global__ __launch_bounds__(256) void k_resid_rows(const InstDev* insts, int inst, int par, double* rows) {
+__global__ __launch_bounds__(256) void k_resid_rows(const InstDev* insts, int inst, int nsteps, double* rows) {
   __shared__ double lds4[4];
   const InstDev& in = insts[inst];
-  const int now = in.parity0 ^ par, prev = 1 ^ now;
+  const int taken = *in.fail == INT_MAX ? nsteps : *in.fail - in.step_base;
+  const int now = in.parity0 ^ (taken & 1), prev = 1 ^ now;
   for (int y = blockIdx.x; y < in.ny; y += gridDim.x) {
     double acc = 0;
     for (int x = threadIdx.x; x < in.nx; x += blockDim.x) {
@@ -1734,12 +1738,12 @@ __global__ __launch_bounds__(256) void k_resid_rows(const InstDev* insts, int in
   }
 }
 
-__global__ __launch_bounds__(256) void k_resid_final(double* rows, int ny, double cells) {
+__global__ __launch_bounds__(256) void k_resid_final(const double* rows, int ny, double cells, double* out) {
   __shared__ double lds4[4];
   double v = 0;
   for (int j = threadIdx.x; j < ny; j += blockDim.x) v += rows[j];
   const double b = block_sum(v, lds4);
-  if (threadIdx.x == 0) rows[ny] = sqrt(b / cells);
+  if (threadIdx.x == 0) *out = sqrt(b / cells);
 }
 
 // Per-step residual of the tracked instances of a launch group (served
@@ -1797,16 +1801,39 @@ __global__ void k_gather_fail(const InstDev* insts, int n, int* out) {
   for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) out[k] = *insts[k].fail;
 }
 
+// An instance record (and the step counter, where given) set by a launch that
+// carries it as its argument. Copies from pageable host memory cross to
+// another queue and back: a one-step call on 96^2, which had three of them
+// and two of results, took 84 us (108 with its residual) for 30 us of step
+// kernels; with this launch and results that the last kernels write into
+// pinned memory 57 us (63).
+struct InstWords {
+  static constexpr int kWords = sizeof(InstDev) / sizeof(unsigned long long);
+  static_assert(sizeof(InstDev) % sizeof(unsigned long long) == 0 && sizeof(InstDev) <= 2048, "kernel argument");
+  unsigned long long w[kWords];
+};
+__global__ __launch_bounds__(256) void k_put_inst(const InstWords rec, unsigned long long* dst, int* step_ctr) {
+  for (int k = threadIdx.x; k < InstWords::kWords; k += blockDim.x) dst[k] = rec.w[k];
+  if (step_ctr && threadIdx.x == 0) *step_ctr = 1;
+}
+
+void launch_put_inst(const InstDev& rec, InstDev* dst, int* step_ctr, hipStream_t s) {
+  InstWords words;
+  std::memcpy(&words, &rec, sizeof(InstDev));
+  k_put_inst<<<1, 256, 0, s>>>(words, reinterpret_cast<unsigned long long*>(dst), step_ctr);
+}
+
 void launch_gather_fail(const InstDev* insts, int n, int* out, hipStream_t s) {
   const int blocks = (n + 255) / 256 < 64 ? (n + 255) / 256 : 64;
   k_gather_fail<<<blocks, 256, 0, s>>>(insts, n, out);
 }
 
 template <typename TS>
-void launch_residual(const InstDev* insts, int inst, int par, double* rows, int nx, int ny, hipStream_t s) {
+void launch_residual(const InstDev* insts, int inst, int nsteps, double* rows, double* out, int nx, int ny,
+                     hipStream_t s) {
   const int blocks = ny < 2048 ? ny : 2048;
-  k_resid_rows<TS><<<blocks, 256, 0, s>>>(insts, inst, par, rows);
-  k_resid_final<<<1, 256, 0, s>>>(rows, ny, (double)nx * (double)ny);
+  k_resid_rows<TS><<<blocks, 256, 0, s>>>(insts, inst, nsteps, rows);
+  k_resid_final<<<1, 256, 0, s>>>(rows, ny, (double)nx * (double)ny, out);
 }
 
 // ---------------------------------------------------------------------------
@@ -2069,7 +2096,7 @@ template void launch_macro<double>(const InstDev*, int, int, double*, int, int, 
 template void launch_macro<float>(const InstDev*, int, int, double*, int, int, hipStream_t);
 template void launch_totals<double>(const InstDev*, int, int, double*, long long, hipStream_t);
 template void launch_totals<float>(const InstDev*, int, int, double*, long long, hipStream_t);
-template void launch_residual<double>(const InstDev*, int, int, double*, int, int, hipStream_t);
-template void launch_residual<float>(const InstDev*, int, int, double*, int, int, hipStream_t);
+template void launch_residual<double>(const InstDev*, int, int, double*, double*, int, int, hipStream_t);
+template void launch_residual<float>(const InstDev*, int, int, double*, double*, int, int, hipStream_t);
 
 }  // namespace uqlbm

@@ -161,13 +161,18 @@ template <typename TS>
 void launch_totals(const InstDev* insts, int inst, int par, double* scratch, long long cells, hipStream_t s);
 int totals_scratch_doubles();
 
-// Copies *insts[k].fail into out[k] for the n members of a launch group.
+// Copies *insts[k].fail into out[k] (device or pinned host memory) for the n
+// members of a launch group.
 void launch_gather_fail(const InstDev* insts, int n, int* out, hipStream_t s);
 
-// Residual of the last step of one instance (RMS change of T over all
-// cells between the other state buffer and state `par`): rows holds ny + 1
-// doubles, per-row sums then the residual in rows[ny].
+// Sets *dst, and *step_ctr to the first step of a sequence where it is given.
+void launch_put_inst(const InstDev& rec, InstDev* dst, int* step_ctr, hipStream_t s);
+
+// Residual of the last step of one instance (RMS change of T over all cells
+// between its two state buffers) behind a sequence of nsteps steps: rows takes
+// ny per-row sums, *out (device or pinned host memory) the residual.
 template <typename TS>
-void launch_residual(const InstDev* insts, int inst, int par, double* rows, int nx, int ny, hipStream_t s);
+void launch_residual(const InstDev* insts, int inst, int nsteps, double* rows, double* out, int nx, int ny,
+                     hipStream_t s);
 
 }  // namespace uqlbm

@@ -444,6 +444,7 @@ Solver::~Solver() {
     }
   }
   if (stream) (void)hipStreamDestroy(stream);
+  if (result) (void)hipHostFree(result);
 }
 
 extern "C" void lbm_release_cached(void) {
@@ -908,7 +909,8 @@ extern "C" int lbm_init(lbm_solver* h) {
 // its stream; later work on that stream sees it in order.
 int uqlbm::upload_inst(Solver& s) {
   fill_inst(s, s.inst_host);
-  HIP_TRY(hipMemcpyAsync(s.inst_dev, &s.inst_host, sizeof(InstDev), hipMemcpyHostToDevice, s.stream));
+  launch_put_inst(s.inst_host, s.inst_dev, nullptr, s.stream);
+  HIP_TRY(hipGetLastError());
   return LBM_OK;
 }
 
@@ -1029,9 +1031,12 @@ static void record_timing(double total_ms, KernelTimer* tm) {
 // account each member's steps, stopping a member at its failing step
 // (reference main loop stop on runOne failure, main.cpp:21,56,73). With
 // `graphs` null the kernels are launched directly; with `timed` the call's
-// device time is recorded (lbm_get_timing).
+// device time is recorded (lbm_get_timing). A lone solver with `result` gets
+// its failure step and, where `resid_rows` is given (ny doubles), its residual
+// there instead: one wait and no copies for the whole call.
 int uqlbm::run_group(const std::vector<Solver*>& members, InstDev* table_dev, const StepLaunch& L, int precision,
-                     hipStream_t stream, int n, GraphCache* graphs, int* fails_dev, bool timed) {
+                     hipStream_t stream, int n, GraphCache* graphs, int* fails_dev, bool timed, StepResult* result,
+                     double* resid_rows) {
   static const int kFirstStep = 1;
   std::vector<InstDev> table(members.size());
   int ptile0 = 0;
@@ -1044,8 +1049,12 @@ int uqlbm::run_group(const std::vector<Solver*>& members, InstDev* table_dev, co
     table[k].strips = L.nstrips > 0 && members[k]->strip_cols > 0 ? 1 : 0;
     ptile0 += members[k]->nptiles;
   }
-  HIP_TRY(hipMemcpyAsync(table_dev, table.data(), table.size() * sizeof(InstDev), hipMemcpyHostToDevice, stream));
-  HIP_TRY(hipMemcpyAsync(L.step_ctr, &kFirstStep, sizeof(int), hipMemcpyHostToDevice, stream));
+  if (table.size() == 1) {
+    launch_put_inst(table[0], table_dev, L.step_ctr, stream);
+  } else {
+    HIP_TRY(hipMemcpyAsync(table_dev, table.data(), table.size() * sizeof(InstDev), hipMemcpyHostToDevice, stream));
+    HIP_TRY(hipMemcpyAsync(L.step_ctr, &kFirstStep, sizeof(int), hipMemcpyHostToDevice, stream));
+  }
   KernelTimer* tm = timed ? active_timer() : nullptr;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (timed) {
@@ -1068,11 +1077,23 @@ int uqlbm::run_group(const std::vector<Solver*>& members, InstDev* table_dev, co
   }
   if (timed) HIP_TRY(hipEventRecord(e1, stream));
   std::vector<int> fail_step(members.size(), INT_MAX);
-  launch_gather_fail(table_dev, (int)members.size(), fails_dev, stream);
-  HIP_TRY(hipMemcpyAsync(fail_step.data(), fails_dev, fail_step.size() * sizeof(int), hipMemcpyDeviceToHost,
-                         stream));
+  if (result) {
+    Solver& s = *members[0];
+    if (resid_rows) {
+      if (precision == LBM_PREC_FP64)
+        launch_residual<double>(table_dev, 0, n, resid_rows, &result->residual, s.nx, s.ny, stream);
+      else
+        launch_residual<float>(table_dev, 0, n, resid_rows, &result->residual, s.nx, s.ny, stream);
+    }
+    launch_gather_fail(table_dev, 1, &result->fail, stream);
+  } else {
+    launch_gather_fail(table_dev, (int)members.size(), fails_dev, stream);
+    HIP_TRY(hipMemcpyAsync(fail_step.data(), fails_dev, fail_step.size() * sizeof(int), hipMemcpyDeviceToHost,
+                           stream));
+  }
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(stream));
+  if (result) fail_step[0] = result->fail;
   if (timed) {
     float ms = 0;
     HIP_TRY(hipEventElapsedTime(&ms, e0, e1));
@@ -1097,11 +1118,12 @@ int uqlbm::run_group(const std::vector<Solver*>& members, InstDev* table_dev, co
   return status;
 }
 
-// Residual of the solver's last step on the device (cpuLBM.cpp:2322-2331):
-// `rows` holds ny + 1 doubles; the result is copied to *out.
+// Residual of the solver's last step on the device (cpuLBM.cpp:2322-2331),
+// after the call's steps: `rows` holds ny + 1 doubles; the result is copied to
+// *out.
 static int device_residual(Solver& s, double* rows, double* out) {
-  if (s.precision == LBM_PREC_FP64) launch_residual<double>(s.inst_dev, 0, 0, rows, s.nx, s.ny, s.stream);
-  else launch_residual<float>(s.inst_dev, 0, 0, rows, s.nx, s.ny, s.stream);
+  if (s.precision == LBM_PREC_FP64) launch_residual<double>(s.inst_dev, 0, 0, rows, rows + s.ny, s.nx, s.ny, s.stream);
+  else launch_residual<float>(s.inst_dev, 0, 0, rows, rows + s.ny, s.nx, s.ny, s.stream);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipMemcpyAsync(out, rows + s.ny, sizeof(double), hipMemcpyDeviceToHost, s.stream));
   HIP_TRY(hipStreamSynchronize(s.stream));
@@ -1120,18 +1142,16 @@ extern "C" int lbm_step(lbm_solver* h, int32_t nsteps, int32_t want_residual, do
   L.nphys = s.nphys;
   launch_strips_of(L, s.strips_dev, s.nstrips, s.nmstrips, s.fused, s.strip_blocks, 0, s.ntiles);
   L.eq_kinds = s.precision == LBM_PREC_FP64 ? 1 : (s.eq32 ? 2 : 1);
+  const bool resid = want_residual && residual_out;
+  if (!s.result) HIP_TRY(hipHostMalloc((void**)&s.result, sizeof(StepResult), hipHostMallocDefault));
+  if (resid && !s.resid_dev) HIP_TRY(solver_alloc(s, (void**)&s.resid_dev, (size_t)s.ny * sizeof(double)));
   std::vector<Solver*> one{&s};
-  const int st = run_group(one, s.inst_dev, L, s.precision, s.stream, nsteps, s.graphs.get(), s.fails_dev, true);
+  const int st = run_group(one, s.inst_dev, L, s.precision, s.stream, nsteps, s.graphs.get(), s.fails_dev, true,
+                           s.result, resid ? s.resid_dev : nullptr);
   const int st2 = upload_inst(s);
   if (st < 0) return st;
   if (st2 != LBM_OK) return st2;
-  if (want_residual && residual_out) {
-    // the previous state is still in the other state buffer: the RMS change
-    // of T over the last step is reduced on the device
-    if (!s.resid_dev) HIP_TRY(solver_alloc(s, (void**)&s.resid_dev, ((size_t)s.ny + 1) * sizeof(double)));
-    const int st3 = device_residual(s, s.resid_dev, residual_out);
-    if (st3 != LBM_OK) return st3;
-  }
+  if (resid) *residual_out = s.result->residual;
   return st;
 }
 

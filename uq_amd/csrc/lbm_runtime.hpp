@@ -40,6 +40,13 @@ struct PropRow {
 };
 
 // One solver instance: the deck, its derived constants and its device state.
+// What a step call returns to the host, written by the last kernels of its
+// sequence into pinned memory.
+struct StepResult {
+  double residual;
+  int fail;  // as InstDev::fail
+};
+
 struct Solver {
   lbm_params p{};
   int nx = 0, ny = 0, pitch = 0;
@@ -87,7 +94,8 @@ struct Solver {
   std::vector<double> dxs, dys;     // non-uniform spacing (lbm_set_spacing), empty when uniform
   double* spacing_dev = nullptr;    // dt/dx[nx], dt/dy[ny], dx[nx], dy[ny]
   double* totals_dev = nullptr;     // conserved-totals reduction scratch (allocated on first use)
-  double* resid_dev = nullptr;      // residual row sums, ny + 1 doubles (allocated on first use)
+  double* resid_dev = nullptr;      // residual row sums, ny doubles (allocated on first use)
+  StepResult* result = nullptr;     // pinned (allocated by the first lbm_step)
   double* res_hist = nullptr;       // served with a tolerance: per-step residual history (kResHist)
   int* fails_dev = nullptr;         // failure step gathered for the host (one int)
   std::unique_ptr<GraphCache> graphs{new GraphCache()};
@@ -213,6 +221,7 @@ int upload_inst(Solver& s);
 int batch_finish(Batch& b, lbm_batch** out);
 int batch_step(Batch& b, int nsteps);
 int run_group(const std::vector<Solver*>& members, InstDev* table_dev, const StepLaunch& L, int precision,
-              hipStream_t stream, int n, GraphCache* graphs, int* fails_dev, bool timed);
+              hipStream_t stream, int n, GraphCache* graphs, int* fails_dev, bool timed, StepResult* result = nullptr,
+              double* resid_rows = nullptr);
 
 }  // namespace uqlbm
