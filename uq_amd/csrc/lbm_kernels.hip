@@ -554,14 +554,25 @@ __device__ __forceinline__ void copy_frozen(const InstDev& in, gptr<const TS> sr
   }
 }
 
+// Step counters of a launch sequence, so that a captured one replays for any
+// step: the kernels of a step of parity `par` read its number from ctr[par],
+// and one kernel of every step (k_s3, k_fin) sets the other for the next. With
+// a launch of its own for the count a step of 201^2 in FP32 storage took 45.4
+// us, without it 43.4; RKMETHOD 0 on 250^2 48.9 and 47.5.
+__device__ __forceinline__ int step_of(const int* ctr, int par) { return ctr[par]; }
+__device__ __forceinline__ void set_next_step(int* ctr, int par, int step) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) ctr[1 ^ par] = step + 1;
+}
+
 // Two waves per SIMD (FP64 arithmetic for both storage types): the
 // instantiation otherwise takes 262 registers (one wave per SIMD); capping
 // it at 256 costs a few spills and hides twice the memory latency (4096^2
 // FP64: 5.9 -> 4.2 ms per launch).
 template <typename TS, typename TC, typename TE>
 __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2))) void k_s3(
-    const InstDev* __restrict__ insts, const TileRef* __restrict__ tiles, int ntiles, int par, const int* stepp) {
-  const int step = *stepp;
+    const InstDev* __restrict__ insts, const TileRef* __restrict__ tiles, int ntiles, int par, int* ctr) {
+  const int step = step_of(ctr, par);
+  set_next_step(ctr, par, step);
   for (int t = first_tile(); t < ntiles; t += gridDim.x) {
     const TileRef tr = tiles[t];
     const InstDev& in = insts[tr.inst];
@@ -736,8 +747,9 @@ __device__ __forceinline__ void fin_cell(const InstDev& in, gptr<const TS> src, 
 
 template <typename TS, typename TC, typename TE, int METHOD>
 __global__ __launch_bounds__(kNT) void k_fin(const InstDev* __restrict__ insts, const TileRef* __restrict__ tiles,
-                                             int ntiles, int par, const int* stepp) {
-  const int step = *stepp;
+                                             int ntiles, int par, int* ctr) {
+  const int step = step_of(ctr, par);
+  set_next_step(ctr, par, step);
   for (int t = first_tile(); t < ntiles; t += gridDim.x) {
     const TileRef tr = tiles[t];
     const InstDev& in = insts[tr.inst];
@@ -1906,7 +1918,7 @@ template <typename TS, typename TC, int MODE, bool MOM, typename Sh>
 static void launch_phys(const StepLaunch& L, hipStream_t s, int par) {
   if (L.nphys > 0)
     k_phys<TS, TC, MODE, MOM, Sh><<<L.ntiles < 1024 ? L.ntiles : 1024, 256, 0, s>>>(L.insts, L.tiles, L.ntiles, par,
-                                                                                  L.step_ctr);
+                                                                                  L.step_ctr + par);
 }
 
 // One flux stage of MODE: the strip kernels for the instances on strips and
@@ -1914,7 +1926,7 @@ static void launch_phys(const StepLaunch& L, hipStream_t s, int par) {
 // flagged tiles.
 template <typename TS, typename TC, int MODE, bool MOM, typename Sh>
 static void launch_flux(const StepLaunch& L, hipStream_t s, int par, int grid_tiles) {
-  const int* step = L.step_ctr;
+  const int* step = L.step_ctr + par;
   if (L.nstrips > 0) {
     if constexpr (MOM) launch_strips_mom(L, s, par);
     else launch_strips<TS, MODE>(L, s, par);
@@ -1953,7 +1965,7 @@ static void per_eq_kind(const StepLaunch& L, F&& launch) {
 
 template <typename TS, typename TC, typename Sh>
 static void launch_rk3(const StepLaunch& L, hipStream_t s, int par, KernelTimer* tm) {
-  const int* step = L.step_ctr;
+  const int* step = L.step_ctr + par;
   const StepGrids<TS, TC, Sh>& G = StepGrids<TS, TC, Sh>::get();
   const int g1 = G.flux0, g3 = G.flux3;
   if (tm) tm->begin(0, s);
@@ -1973,7 +1985,7 @@ static void launch_rk3(const StepLaunch& L, hipStream_t s, int par, KernelTimer*
   if (tm) tm->begin(3, s);
   per_eq_kind<TS>(L, [&](auto te, int k) {
     k_s3<TS, TP, decltype(te)><<<blocks_for(L.nptiles, G.s3[k]), kNT, 0, s>>>(L.insts, L.ptiles, L.nptiles, par,
-                                                                              step);
+                                                                              L.step_ctr);
   });
   if (tm) tm->end(3, s);
   if (L.nwalls) {
@@ -2010,7 +2022,7 @@ void launch_fused_step(const StepLaunch& L, hipStream_t s, bool write_state, boo
 // RKMETHOD 0, 2, 3: one flux stage.
 template <typename TS, typename TC, int METHOD, typename Sh>
 static void launch_one_stage(const StepLaunch& L, hipStream_t s, int par, KernelTimer* tm) {
-  const int* step = L.step_ctr;
+  const int* step = L.step_ctr + par;
   constexpr int FM = METHOD == 0 ? 0 : 2;
   const StepGrids<TS, TC, Sh>& G = StepGrids<TS, TC, Sh>::get();
   const int g1 = FM == 0 ? G.flux0 : G.fluxe;
@@ -2034,7 +2046,7 @@ static void launch_one_stage(const StepLaunch& L, hipStream_t s, int par, Kernel
   if (tm) tm->begin(3, s);
   per_eq_kind<TS>(L, [&](auto te, int k) {
     k_fin<TS, TP, decltype(te), METHOD><<<blocks_for(L.nptiles, g2[k]), kNT, 0, s>>>(L.insts, L.ptiles, L.nptiles,
-                                                                                     par, step);
+                                                                                     par, L.step_ctr);
   });
   if (tm) tm->end(3, s);
 }
@@ -2049,17 +2061,11 @@ static void launch_step_shape(const StepLaunch& L, hipStream_t s, int par, Kerne
   }
 }
 
-// Advances the step counter of a launch sequence: the kernels of step k read
-// k + 1 from it, so one captured sequence replays for any step.
-__global__ void k_tick(int* ctr) {
-  if (threadIdx.x == 0) ctr[0] = ctr[0] + 1;
-}
-
 template <typename TS>
 static void launch_track(const StepLaunch& L, hipStream_t s, int par, int ninst) {
   k_track_tiles<TS><<<L.nptiles < 8192 ? L.nptiles : 8192, kNT, 0, s>>>(L.insts, L.ptiles, L.nptiles, par,
-                                                                        L.step_ctr, L.res_partial);
-  k_track_sum<<<ninst < 1024 ? ninst : 1024, 256, 0, s>>>(L.insts, ninst, L.step_ctr, L.res_partial);
+                                                                        L.step_ctr + par, L.res_partial);
+  k_track_sum<<<ninst < 1024 ? ninst : 1024, 256, 0, s>>>(L.insts, ninst, L.step_ctr + par, L.res_partial);
 }
 
 template <typename TS, typename TC>
@@ -2072,7 +2078,6 @@ void launch_step(const StepLaunch& L, hipStream_t s, int par, KernelTimer* tm) {
     default: launch_step_shape<TS, TC, Shape0>(L, s, par, tm); break;
   }
   if (L.res_partial && L.nptiles > 0) launch_track<TS>(L, s, par, L.ninst);
-  k_tick<<<1, 64, 0, s>>>(L.step_ctr);
 }
 
 template <typename TS>

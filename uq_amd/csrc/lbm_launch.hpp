@@ -22,8 +22,8 @@ struct StepLaunch {
   const TileRef* ptiles = nullptr;  // 64 x 4 row tiles of the pointwise kernels
   int nptiles = 0;
   int rk_method = 1;                // RKMETHOD shared by every instance of the group
-  int* step_ctr = nullptr;          // device step counter: step k of a sequence reads k + 1 (fused:
-                                    // two counters, of k_stage23 and of k_stage31)
+  int* step_ctr = nullptr;          // two device step counters, of the even and of the odd steps of a
+                                    // sequence (fused: of k_stage23 and of k_stage31)
   int flux_shape = 0;               // flux tile shape (flux_tile_dims); the tile list is built for it
   double* res_partial = nullptr;    // per pointwise tile residual partials (nptiles doubles) when
                                     // some instance tracks its residual; null otherwise

@@ -94,7 +94,8 @@ void launch_alpha(const StepLaunch& L, hipStream_t s, int which, int par, const 
 template <typename TS, typename TC, int MODE>
 static void launch_strips_as(const StepLaunch& L, hipStream_t s, int par, int all) {
   const int chunk = (L.nstrips + 31) / 32 * 4;  // items per XCD, a multiple of a block's four
-  k_strip<TS, TC, MODE><<<8 * 12 * (chunk / 4), 256, 0, s>>>(L.insts, L.strips, L.nstrips, chunk, all, par, L.step_ctr);
+  k_strip<TS, TC, MODE><<<8 * 12 * (chunk / 4), 256, 0, s>>>(L.insts, L.strips, L.nstrips, chunk, all, par,
+                                                              L.step_ctr + par);
 }
 
 template <typename TS, int MODE>
@@ -110,7 +111,8 @@ void launch_strips(const StepLaunch& L, hipStream_t s, int par) {
 // Stage-3 flux of FP32 storage: FP32 stencils for every instance.
 void launch_strips_mom(const StepLaunch& L, hipStream_t s, int par) {
   const int chunk = (L.nmstrips + 7) / 8;
-  k_strip_mom<float, float><<<8 * chunk, 256, 0, s>>>(L.insts, L.mstrips, L.nmstrips, chunk, par, L.step_ctr);
+  k_strip_mom<float, float><<<8 * chunk, 256, 0, s>>>(L.insts, L.mstrips, L.nmstrips, chunk, par,
+                                                       L.step_ctr + par);
 }
 
 template void launch_alpha<double>(const StepLaunch&, hipStream_t, int, int, const int*);
