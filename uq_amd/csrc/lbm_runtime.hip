@@ -574,12 +574,12 @@ static std::vector<TileRef> build_flux_tiles(const Solver& s, int shape) {
   return tiles;
 }
 
-// Strip work items of up to `rows` rows of an instance (instance index
-// `inst`), appended to out. Consecutive rows of the same kind (solid or not)
+// Strip work items of up to `rows` rows (`most_solid` of them near solids) of
+// an instance (instance index `inst`), appended to out. Consecutive rows of the same kind (solid or not)
 // form an item, so that only the rows near a solid take the solid path.
 // TileRef: tx = strip index, ty = first row, flags = kTileSolid (solid rows)
 // | kStripDesc (every second item of a column) | row count << kStripRowsBit.
-static void strip_items(const Solver& s, int rows, int inst, std::vector<TileRef>& out) {
+static void strip_items(const Solver& s, int rows, int most_solid, int inst, std::vector<TileRef>& out) {
   const size_t first = out.size();
   for (int sx = 0; sx < s.strip_cols; sx++) {
     const char* solid = s.strip_solid.data() + (size_t)sx * s.ny;
@@ -588,7 +588,8 @@ static void strip_items(const Solver& s, int rows, int inst, std::vector<TileRef
     // other read the rows they share at about the same time
     for (int y = 0, k = 0; y < s.ny; k++) {
       int n = 1;
-      while (y + n < s.ny && n < rows && solid[y + n] == solid[y]) n++;
+      const int most = solid[y] ? most_solid : rows;
+      while (y + n < s.ny && n < most && solid[y + n] == solid[y]) n++;
       out.push_back(TileRef{inst, sx, y, (solid[y] ? kTileSolid : 0) | ((k & 1) ? kStripDesc : 0) | (n << kStripRowsBit)});
       y += n;
     }
@@ -612,6 +613,7 @@ static constexpr int kStripBlock = 32;
 // cell.
 static void mark_strips(Solver& s) {
   s.strip_solid.clear();
+  s.strip_runs.clear();
   s.strip_cols = s.strip_blocks = 0;
   if (s.any_phys) return;
   const int H = tile_halo();
@@ -640,8 +642,15 @@ static void mark_strips(Solver& s) {
     }
   }
   std::vector<TileRef> items;
-  strip_items(s, kStripBlock, 0, items);
+  strip_items(s, kStripBlock, kStripBlock, 0, items);
   s.strip_blocks = (int)items.size();
+  for (int sx = 0; sx < s.strip_cols; sx++)
+    for (int y = 0, n; y < s.ny; y += n) {
+      const char* solid = s.strip_solid.data() + (size_t)sx * s.ny + y;
+      for (n = 1; y + n < s.ny && solid[n] == solid[0]; n++) {
+      }
+      s.strip_runs.push_back(solid[0] ? -n : n);
+    }
 }
 
 static int g_strips = 1;  // lbm_set_strips mode
@@ -653,23 +662,42 @@ bool uqlbm::strips_enabled() { return g_strips != 0; }
 static constexpr int kFarMinBlocks = 2048;
 bool uqlbm::far_fp64(int blocks) { return g_strips == 2 || blocks >= kFarMinBlocks; }
 
-// Rows per strip item of a launch group: the most (32, 16, ... 2) that leave
-// kStripWaves wavefronts, `waves` of them per item (one per direction of
-// k_strip). Every item fills a six-row window and forms one face beyond its
-// own rows, so long items cost less, but with fewer than one to two
-// wavefronts per SIMD (1024 SIMDs) the group waits for its longest march.
-// FP64 us per step at 32 / 16 / 8 / 4 / 2 rows: 64^2 Couette 8 rows 50, 4 rows
-// 46.5, 2 rows 42.6 (384, 768 wavefronts at 4, 2); 301^2 block 16 rows 116,
-// 8 rows 97 (1354, 2709 wavefronts); 256^2 8 rows 51, 4 rows 55 (1920, 3840);
-// ensemble of 48 32 rows 1772, 64 rows 1809, 128 rows 1910; 3072^2 16 rows 4073,
-// 32 rows 4027, 64 rows 4057, 128 rows 4102.
-static constexpr int kStripWaves = 1536, kStripRows = 32, kStripRowsMin = 2;
-static int strip_rows(const std::vector<Solver*>& members, int waves) {
-  long long rows = 0;
-  for (const Solver* s : members) rows += (long long)s->strip_cols * s->ny;
-  int h = kStripRows;
-  while (h > kStripRowsMin && rows * waves < (long long)kStripWaves * h) h /= 2;
-  return h;
+// Rows per strip item of a launch group, 1 to kStripRows: those of the least
+// (n + 1) * (rows + 2), with n the workgroups of the busiest CU, `blocks` of
+// them per item (three of k_strip's directions, one of four wavefronts). A
+// row of the march takes the longer the more workgroups share the CU, but a
+// lone one cannot fill it (stage23: 3.0, 4.5, 5.9 and 7.8 us per row with one
+// to four), and the window that an item fills costs about two rows. Whole
+// numbers of workgroups per CU matter as much as the length: 512^2 at 6 rows
+// has 774 items, four on some CUs, at 7 rows 666, three: 122 and 107 us.
+// us per step (FP64) or launch at 1 / 2 / 4 / 8 / 16 / 32 rows, and at the rule's:
+//   64^2 Couette, step           31 / 40 / 54 / 67 / 110 / 199       1: 31
+//   256^2 shear, step            47 / 46 / 53 / 64 / 108 / 197       3: 45
+//   512^2 shear, step            126 / 104 / 107 / 118 / 158 / 199   5: 107
+//   ensemble of 48, step         2283 / 1815 / 1549 / 1421 / 1431 / 1514   12: 1396 (1417 with the s12 launch)
+//   512^2, FP32 k_strip          62 / 44 / 36 / 33 / 35 / 49         8: 33
+//   1100^2, FP32 k_strip_mom     266 / 199 / 164 / 147 / 150 / 150   12: 141
+// (without the launch that begins an FP64 sequence).
+// Items near solids have half as many: their rows take about twice as long,
+// and the launch waits for the last of them (301^2 with a block, FP64 step 87
+// us with all rows, 67 with half, 67 with a third; FP32 storage 110, 94, 94).
+static constexpr int kStripRows = 32, kCus = 256;
+static int solid_rows(int rows) { return (rows + 1) / 2; }
+static int strip_rows(const std::vector<Solver*>& members, int blocks) {
+  long long least = LLONG_MAX;
+  int best = 1;
+  for (int h = 1; h <= kStripRows; h++) {
+    long long items = 0;
+    for (const Solver* s : members)
+      for (const int run : s->strip_runs)
+        items += run > 0 ? (run + h - 1) / h : (solid_rows(h) - run - 1) / solid_rows(h);
+    const long long cost = ((items * blocks + kCus - 1) / kCus + 1) * (h + 2);
+    if (cost < least) {
+      least = cost;
+      best = h;
+    }
+  }
+  return best;
 }
 
 // The fused step takes FP64 RK3 groups whose members all have strips and
@@ -684,18 +712,18 @@ static bool fused_instance(const Solver& s) {
 }
 
 uqlbm::StripLists::StripLists(const std::vector<Solver*>& members, int shape) {
-  const int rows = strip_rows(members, 12);
+  const int rows = strip_rows(members, 3);
   for (size_t k = 0; k < members.size(); k++) {
-    strip_items(*members[k], rows, (int)k, items);
+    strip_items(*members[k], rows, solid_rows(rows), (int)k, items);
     blocks += members[k]->strip_blocks;
     if (members[k]->strip_cols == 0) tiles_rest += (int)solver_tiles(*members[k], shape).size();
   }
   n = (int)items.size();
   // items of k_strip_mom, or of the fused step: four wavefronts each
-  const int mrows = strip_rows(members, 4);
+  const int mrows = strip_rows(members, 1);
   fused = !members.empty();
   for (size_t k = 0; k < members.size(); k++) {
-    strip_items(*members[k], mrows, (int)k, items);
+    strip_items(*members[k], mrows, solid_rows(mrows), (int)k, items);
     fused = fused && fused_instance(*members[k]);
   }
   nmom = (int)items.size() - n;

@@ -62,6 +62,7 @@ struct Solver {
   std::vector<TileRef> tiles_shape[kFluxShapes];  // flux tiles per shape, built on first use
   std::vector<WallRef> walls_host;
   std::vector<TileRef> ptiles_host;
+  std::vector<int> strip_runs;      // lengths of the runs of strip_solid, negative those of solid rows
   std::vector<char> strip_solid;    // [strip][y]: the row's stencils reach a solid cell within the strip
   int strip_cols = 0;               // strips across (0 when a cell needs physical addressing: no strip items)
   int strip_blocks = 0;             // 32-row strip items (the size of the launch group, far_fp64)
