@@ -5,7 +5,7 @@ one MI355X.
 Headline (`value`): aggregate MLUPS of the batched FP64 UQ ensemble — 256
 Couette / periodic shear-wave instances, square sides drawn from
 {64,128,256,512}, sampled wall speed, Mach, Pr and tau (seed 2026), all
-advanced together with one launch per RK stage. A step is one RK step of
+advanced together, two launches per step. A step is one RK step of
 every instance; MLUPS = sum(nx*ny) * steps / seconds / 1e6, with the
 seconds taken by the host clock around exactly `--steps` steps (the batch
 call synchronises the stream before returning), state resident in HBM.
@@ -54,25 +54,23 @@ def log(msg: str) -> None:
 
 
 def kernel_bytes_per_lup(es: int) -> dict:
-    """Compulsory HBM traffic of each kernel per lattice update, for values
+    """Compulsory HBM traffic of each launch per lattice update, for values
     of `es` bytes, counting the planes each kernel touches (13 f and 13 h
-    directions; the rest direction has no flux). s12 reads the state and
-    writes f2 but for its rest direction (26 + 24 values); flux2 reads the
-    24 moving directions of f2 and writes the 24 net-flux planes (48). FP64
-    storage: s3 reads the state and the net fluxes (summing the net fluxes'
-    moments in a first pass whose lines the second pass finds in L2) and
-    writes f3, its rest direction straight into the new state (26 + 24 +
-    26); flux3 reads f3 and the stage-2 net fluxes and writes the new state
-    f3 + (dF2 - dF3)/2 (24 + 24 + 24). FP32 storage: s3 writes f3 but for
-    its rest direction and G = f3 + dF2/2 (26 + 24 + 24 + 26) and flux3
-    reads f3 and G (24 + 24 + 24),
-    and the 4 FP64 conserved-moment planes of the state add 32 B to s12
-    (read), 64 B to s3 (read, written for G) and 64 B to flux3 (read and
-    written). Halo re-reads, the cell-type map and the wall-closure kernels
-    are excluded."""
+    directions; the rest direction has no flux). FP64 storage steps in two
+    launches, timed as flux2 and flux3: k_stage23 reads f2 and writes f3 and
+    the 24 net-flux planes, k_stage31 reads f3 and those and writes f2 of the
+    next step (26 + 26 + 24 each); the last two steps of a call write the
+    state too, and one s12 (26 + 26) begins it. FP32 storage takes four: s12
+    reads the state and writes f2 but for its rest direction (26 + 24);
+    flux2 reads the 24 moving directions of f2 and writes the net-flux
+    planes (48); s3 writes f3 but for its rest direction and G = f3 + dF2/2
+    (26 + 24 + 24 + 26); flux3 reads f3 and G (24 + 24 + 24); and the 4 FP64
+    conserved-moment planes of the state add 32 B to s12 (read), 64 B to s3
+    (read, written for G) and 64 B to flux3 (read and written). Halo
+    re-reads, the cell-type map and the wall-closure kernels are excluded."""
     if es == 4:
         return {"s12": 50 * es + 32, "flux2": 48 * es, "s3": 100 * es + 64, "flux3": 72 * es + 64}
-    return {"s12": 50 * es, "flux2": 48 * es, "s3": 76 * es, "flux3": 72 * es}
+    return {"s12": 52 * es, "flux2": 76 * es, "s3": 0, "flux3": 76 * es}
 
 
 def measured_traffic(kernel: str, workload: str, shape: int):

@@ -1107,7 +1107,7 @@ int uqlbm::run_group(const std::vector<Solver*>& members, InstDev* table_dev, co
   std::vector<int> fail_step(members.size(), INT_MAX);
   if (result) {
     Solver& s = *members[0];
-    if (resid_rows) {
+    if (resid_rows) {  // the previous state is still in the other state buffer
       if (precision == LBM_PREC_FP64)
         launch_residual<double>(table_dev, 0, n, resid_rows, &result->residual, s.nx, s.ny, stream);
       else
@@ -1171,15 +1171,22 @@ extern "C" int lbm_step(lbm_solver* h, int32_t nsteps, int32_t want_residual, do
   launch_strips_of(L, s.strips_dev, s.nstrips, s.nmstrips, s.fused, s.strip_blocks, 0, s.ntiles);
   L.eq_kinds = s.precision == LBM_PREC_FP64 ? 1 : (s.eq32 ? 2 : 1);
   const bool resid = want_residual && residual_out;
-  if (!s.result) HIP_TRY(hipHostMalloc((void**)&s.result, sizeof(StepResult), hipHostMallocDefault));
-  if (resid && !s.resid_dev) HIP_TRY(solver_alloc(s, (void**)&s.resid_dev, (size_t)s.ny * sizeof(double)));
+  if (!s.result && hipHostMalloc((void**)&s.result, sizeof(StepResult), hipHostMallocDefault) != hipSuccess) {
+    s.result = nullptr;  // no pinned memory to be had: the results are copied
+    (void)hipGetLastError();
+  }
+  if (resid && !s.resid_dev) HIP_TRY(solver_alloc(s, (void**)&s.resid_dev, ((size_t)s.ny + 1) * sizeof(double)));
   std::vector<Solver*> one{&s};
   const int st = run_group(one, s.inst_dev, L, s.precision, s.stream, nsteps, s.graphs.get(), s.fails_dev, true,
                            s.result, resid ? s.resid_dev : nullptr);
   const int st2 = upload_inst(s);
   if (st < 0) return st;
   if (st2 != LBM_OK) return st2;
-  if (resid) *residual_out = s.result->residual;
+  if (resid && s.result) *residual_out = s.result->residual;
+  if (resid && !s.result) {
+    const int st3 = device_residual(s, s.resid_dev, residual_out);
+    if (st3 != LBM_OK) return st3;
+  }
   return st;
 }
 

@@ -95,7 +95,7 @@ struct Solver {
   std::vector<double> dxs, dys;     // non-uniform spacing (lbm_set_spacing), empty when uniform
   double* spacing_dev = nullptr;    // dt/dx[nx], dt/dy[ny], dx[nx], dy[ny]
   double* totals_dev = nullptr;     // conserved-totals reduction scratch (allocated on first use)
-  double* resid_dev = nullptr;      // residual row sums, ny doubles (allocated on first use)
+  double* resid_dev = nullptr;      // residual row sums, ny + 1 doubles (allocated on first use)
   StepResult* result = nullptr;     // pinned (allocated by the first lbm_step)
   double* res_hist = nullptr;       // served with a tolerance: per-step residual history (kResHist)
   int* fails_dev = nullptr;         // failure step gathered for the host (one int)
