@@ -497,7 +497,7 @@ def main() -> int:
         "dtype": "f64",
         "data": "synthetic (seeded UQ ensemble decks, seed %d)" % args.seed,
         "config": {
-            "workload": f"uq_ensemble_{len(members)} batched FP64, one launch per RK stage for all instances",
+            "workload": f"uq_ensemble_{len(members)} batched FP64, two launches per step for all instances",
             "instances": len(members), "cells": cells, "seed": args.seed,
             "sides": [64, 128, 256, 512], "kinds": ["couette", "shear"],
             "rk_method": 1, "flux_method": "WENO5", "parallelism": "single GPU",

@@ -260,6 +260,23 @@ void host_piece(const std::vector<HostSeg>& segs, bool out, char* slot, size_t a
     at += g.bytes;
   }
 }
+
+// The same part between the device range and the host segments, without a slot.
+hipError_t direct_piece(char* dev, const std::vector<HostSeg>& segs, bool out, size_t a, size_t b, hipStream_t stream) {
+  size_t at = 0;
+  for (const HostSeg& g : segs) {
+    const size_t lo = std::max(a, at), hi = std::min(b, at + g.bytes);
+    if (lo < hi && g.host) {
+      char* host = (char*)g.host + (lo - at);
+      const hipError_t e = out ? hipMemcpyAsync(host, dev + lo, hi - lo, hipMemcpyDeviceToHost, stream)
+                               : hipMemcpyAsync(dev + lo, host, hi - lo, hipMemcpyHostToDevice, stream);
+      const hipError_t e2 = hipStreamSynchronize(stream);
+      if (e != hipSuccess || e2 != hipSuccess) return e != hipSuccess ? e : e2;
+    }
+    at += g.bytes;
+  }
+  return hipSuccess;
+}
 }  // namespace
 
 void release_slots() {
@@ -281,7 +298,15 @@ hipError_t staged_copy(char* dev, const std::vector<HostSeg>& segs, bool out, hi
   std::atomic<int> err{(int)hipSuccess};
   auto pieces = [&](size_t first, size_t step, bool own_stream) {
     SlotUse u(device);
-    hipError_t e = u.err;
+    if (u.err != hipSuccess) {  // no pinned memory to be had: pageable copies
+      (void)hipGetLastError();
+      hipError_t e = hipSuccess;
+      for (size_t k = first; k < n && e == hipSuccess; k += step)
+        e = direct_piece(dev, segs, out, k * kSlotBytes, std::min(total, (k + 1) * kSlotBytes), stream);
+      if (e != hipSuccess) err.store((int)e);
+      return;
+    }
+    hipError_t e = hipSuccess;
     const hipStream_t st = own_stream ? u.s.stream : stream;
     for (size_t k = first; k < n && e == hipSuccess && err.load() == (int)hipSuccess; k += step) {
       const size_t a = k * kSlotBytes, b = std::min(total, a + kSlotBytes);

@@ -1,9 +1,10 @@
 // lbm_kernels.hip — gfx950 kernels of the D2Q13 thermal FD-LBM.
 //
 // One step of the reference's RKMETHOD = 1 stepper (IMEX-SSP2(3,2,2),
-// reference RK3, cpuLBM.cpp:1738-2103) is four tile launches, each walking
-// every tile of every instance of the group in one grid-stride (persistent)
-// loop, plus the wall closure when the group has walls:
+// reference RK3, cpuLBM.cpp:1738-2103) is the two launches of lbm_fused.hip
+// for FP64 storage, k_s12 here beginning a sequence; elsewhere it is four
+// launches, each over every tile or strip item of every instance of the group,
+// plus the wall closure when the group has walls:
 //
 //   k_s12      pointwise: moments, stage-1 equilibrium, implicit stages 1-2
 //              -> f2 (cpuLBM.cpp:1819-1924)
@@ -13,14 +14,15 @@
 //              x/y face fluxes (WENO5 or NND), net flux dF(f2) -> dF planes
 //              (posFluxes + cFLUX, cpuLBM.cpp:1436-1500)
 //   k_s3       pointwise: moments of f - dF(f2), stage-3 equilibrium,
-//              implicit stage 3 -> f3 (cpuLBM.cpp:1926-1993)
+//              implicit stage 3 -> f3 (cpuLBM.cpp:1926-1993); FP64 storage
+//              takes f from f2 (lbm_point.hpp)
 //  [k_alpha    same for f3]
 //   k_flux<1>  stencil: net flux dF(f3); the final combination, new state
 //              f3 + (dF(f2) - dF(f3))/2 (cpuLBM.cpp:2009-2042)
 //
-// On launch groups large enough to fill the GPU the stencil stages run on
-// the strip kernels of lbm_strip.hpp (one wavefront per 58-column strip,
-// rows marched through registers) instead of the tile kernels below.
+// The stencil stages run on the strip kernels of lbm_strip.hpp (wavefronts
+// that march the rows of 58-column strips through registers) instead of the
+// tile kernels below, but for instances that need the physical addressing.
 //
 // The stencil kernels run one direction at a time through a runtime loop
 // (one copy of the flux code, low register use) on tiles of one of five
