@@ -277,7 +277,8 @@ int lbm_set_graphs(int32_t enable);
 /*
  * Flux stages of instances whose cells all take the logical stencil
  * addressing run on the strip kernels (one wavefront per direction of a
- * 58-column strip of 2 to 32 rows, marched row by row) instead of the flux
+ * 58-column strip of 1 to 32 rows, marched row by row; LBM_PREC_FP64 RK3: four
+ * per strip, the whole step in two launches) instead of the flux
  * tile kernels (LBM_PREC_MIXED stage 3: one workgroup for all directions).
  * mode 0: every flux stage on the tile kernels; 1 (default) and 2: strips
  * wherever an instance can take them. Results are bitwise equal either way,
