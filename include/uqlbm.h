@@ -226,9 +226,10 @@ void lbm_batch_destroy(lbm_batch* b);
 
 /*
  * Device time of the last lbm_step / lbm_batch_step call: total elapsed
- * milliseconds between HIP events recorded on the solver's stream, and the
- * per-kernel average durations when timing was enabled with
- * lbm_set_kernel_timing (events around every launch).
+ * milliseconds of the steps on the solver's stream (HIP events; lbm_step: the
+ * device's clock, read by its first and last launch), and the per-kernel
+ * average durations when timing was enabled with lbm_set_kernel_timing (events
+ * around every launch).
  */
 typedef struct lbm_timing {
   double total_ms;

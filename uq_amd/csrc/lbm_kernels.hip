@@ -1811,7 +1811,8 @@ __global__ __launch_bounds__(256) void k_track_sum(const InstDev* insts, int nin
 
 // Failure steps of the members of a launch group gathered into one array,
 // so that the host reads them with a single copy.
-__global__ void k_gather_fail(const InstDev* insts, int n, int* out) {
+__global__ void k_gather_fail(const InstDev* insts, int n, int* out, long long* clock) {
+  if (clock && blockIdx.x == 0 && threadIdx.x == 0) *clock = wall_clock64();
   for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) out[k] = *insts[k].fail;
 }
 
@@ -1820,26 +1821,29 @@ __global__ void k_gather_fail(const InstDev* insts, int n, int* out) {
 // another queue and back: a one-step call on 96^2, which had three of them
 // and two of results, took 84 us (108 with its residual) for 30 us of step
 // kernels; with this launch and results that the last kernels write into
-// pinned memory 57 us (63).
+// pinned memory 57 us (63), and with the device's clock read by the first and
+// the last launch instead of events recorded around the steps 47 us (52).
 struct InstWords {
   static constexpr int kWords = sizeof(InstDev) / sizeof(unsigned long long);
   static_assert(sizeof(InstDev) % sizeof(unsigned long long) == 0 && sizeof(InstDev) <= 2048, "kernel argument");
   unsigned long long w[kWords];
 };
-__global__ __launch_bounds__(256) void k_put_inst(const InstWords rec, unsigned long long* dst, int* step_ctr) {
+__global__ __launch_bounds__(256) void k_put_inst(const InstWords rec, unsigned long long* dst, int* step_ctr,
+                                                  long long* clock) {
   for (int k = threadIdx.x; k < InstWords::kWords; k += blockDim.x) dst[k] = rec.w[k];
   if (step_ctr && threadIdx.x == 0) *step_ctr = 1;
+  if (clock && threadIdx.x == 0) *clock = wall_clock64();
 }
 
-void launch_put_inst(const InstDev& rec, InstDev* dst, int* step_ctr, hipStream_t s) {
+void launch_put_inst(const InstDev& rec, InstDev* dst, int* step_ctr, long long* clock, hipStream_t s) {
   InstWords words;
   std::memcpy(&words, &rec, sizeof(InstDev));
-  k_put_inst<<<1, 256, 0, s>>>(words, reinterpret_cast<unsigned long long*>(dst), step_ctr);
+  k_put_inst<<<1, 256, 0, s>>>(words, reinterpret_cast<unsigned long long*>(dst), step_ctr, clock);
 }
 
-void launch_gather_fail(const InstDev* insts, int n, int* out, hipStream_t s) {
+void launch_gather_fail(const InstDev* insts, int n, int* out, long long* clock, hipStream_t s) {
   const int blocks = (n + 255) / 256 < 64 ? (n + 255) / 256 : 64;
-  k_gather_fail<<<blocks, 256, 0, s>>>(insts, n, out);
+  k_gather_fail<<<blocks, 256, 0, s>>>(insts, n, out, clock);
 }
 
 template <typename TS>

@@ -162,11 +162,13 @@ void launch_totals(const InstDev* insts, int inst, int par, double* scratch, lon
 int totals_scratch_doubles();
 
 // Copies *insts[k].fail into out[k] (device or pinned host memory) for the n
-// members of a launch group.
-void launch_gather_fail(const InstDev* insts, int n, int* out, hipStream_t s);
+// members of a launch group, and the device's clock into *clock (null: not
+// wanted).
+void launch_gather_fail(const InstDev* insts, int n, int* out, long long* clock, hipStream_t s);
 
-// Sets *dst, and *step_ctr to the first step of a sequence where it is given.
-void launch_put_inst(const InstDev& rec, InstDev* dst, int* step_ctr, hipStream_t s);
+// Sets *dst and, where they are given, *step_ctr to the first step of a sequence
+// and *clock to the device's clock.
+void launch_put_inst(const InstDev& rec, InstDev* dst, int* step_ctr, long long* clock, hipStream_t s);
 
 // Residual of the last step of one instance (RMS change of T over all cells
 // between its two state buffers) behind a sequence of nsteps steps: rows takes

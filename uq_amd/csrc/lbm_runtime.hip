@@ -937,7 +937,7 @@ extern "C" int lbm_init(lbm_solver* h) {
 // its stream; later work on that stream sees it in order.
 int uqlbm::upload_inst(Solver& s) {
   fill_inst(s, s.inst_host);
-  launch_put_inst(s.inst_host, s.inst_dev, nullptr, s.stream);
+  launch_put_inst(s.inst_host, s.inst_dev, nullptr, nullptr, s.stream);
   HIP_TRY(hipGetLastError());
   return LBM_OK;
 }
@@ -1078,14 +1078,15 @@ int uqlbm::run_group(const std::vector<Solver*>& members, InstDev* table_dev, co
     ptile0 += members[k]->nptiles;
   }
   if (table.size() == 1) {
-    launch_put_inst(table[0], table_dev, L.step_ctr, stream);
+    launch_put_inst(table[0], table_dev, L.step_ctr, result ? &result->begin : nullptr, stream);
   } else {
     HIP_TRY(hipMemcpyAsync(table_dev, table.data(), table.size() * sizeof(InstDev), hipMemcpyHostToDevice, stream));
     HIP_TRY(hipMemcpyAsync(L.step_ctr, &kFirstStep, sizeof(int), hipMemcpyHostToDevice, stream));
   }
   KernelTimer* tm = timed ? active_timer() : nullptr;
   hipEvent_t e0 = nullptr, e1 = nullptr;
-  if (timed) {
+  const bool events = timed && !result;  // a lone solver's first and last launch read the clock
+  if (events) {
     HIP_TRY(hipEventCreate(&e0));
     HIP_TRY(hipEventCreate(&e1));
     HIP_TRY(hipEventRecord(e0, stream));
@@ -1103,31 +1104,36 @@ int uqlbm::run_group(const std::vector<Solver*>& members, InstDev* table_dev, co
   } else {
     launch_steps(L, precision, stream, n, tm);
   }
-  if (timed) HIP_TRY(hipEventRecord(e1, stream));
+  if (events) HIP_TRY(hipEventRecord(e1, stream));
   std::vector<int> fail_step(members.size(), INT_MAX);
   if (result) {
     Solver& s = *members[0];
+    launch_gather_fail(table_dev, 1, &result->fail, &result->end, stream);
     if (resid_rows) {  // the previous state is still in the other state buffer
       if (precision == LBM_PREC_FP64)
         launch_residual<double>(table_dev, 0, n, resid_rows, &result->residual, s.nx, s.ny, stream);
       else
         launch_residual<float>(table_dev, 0, n, resid_rows, &result->residual, s.nx, s.ny, stream);
     }
-    launch_gather_fail(table_dev, 1, &result->fail, stream);
   } else {
-    launch_gather_fail(table_dev, (int)members.size(), fails_dev, stream);
+    launch_gather_fail(table_dev, (int)members.size(), fails_dev, nullptr, stream);
     HIP_TRY(hipMemcpyAsync(fail_step.data(), fails_dev, fail_step.size() * sizeof(int), hipMemcpyDeviceToHost,
                            stream));
   }
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(stream));
   if (result) fail_step[0] = result->fail;
-  if (timed) {
+  if (events) {
     float ms = 0;
     HIP_TRY(hipEventElapsedTime(&ms, e0, e1));
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     record_timing(ms, tm);
+  } else if (timed) {
+    int dev = 0, khz = 0;
+    HIP_TRY(hipGetDevice(&dev));
+    HIP_TRY(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
+    record_timing((double)(result->end - result->begin) / khz, tm);
   }
   int status = LBM_OK;
   for (size_t k = 0; k < members.size(); k++) {

@@ -44,7 +44,8 @@ struct PropRow {
 // sequence into pinned memory.
 struct StepResult {
   double residual;
-  int fail;  // as InstDev::fail
+  long long begin, end;  // device clock around the steps
+  int fail;              // as InstDev::fail
 };
 
 struct Solver {
