@@ -122,7 +122,10 @@ __device__ __forceinline__ Sums get_sums(const QuadRows<N>& X, int buf, int col,
 // Hides where a scalar value comes from: what is formed from it is formed
 // again in every row, by scalar instructions and loads that run beside the
 // vector ones, instead of being kept over the rows in scalar registers, which
-// are too few for the descriptors, constants and signs of a row together.
+// are too few for the descriptors, constants and signs of a row together. (Or
+// as a flag per lane: QuadItem::upcol compared outside the rows took a vector
+// register over all of them, and the compiler spilled it at the merge behind a
+// wall's branch, before the other lanes were on again: their flag was lost.)
 template <typename T>
 __device__ __forceinline__ T again(T v) {
   asm volatile("" : "+s"(v));
@@ -183,7 +186,8 @@ struct QuadItem {
   // direction, and of the diagonal at a row that is not or is mirrored
   unsigned Xx, Xd[2];
   int col;       // its column of the strip's 64
-  int own, up;   // own column; the upwind column is clamped
+  int own;       // own column
+  int upcol;     // the strip's column whose upwind column is clamped (of those within the instance at most one)
   double rdx;
 };
 
@@ -215,14 +219,13 @@ __device__ __forceinline__ void quad_setup(const InstDev* inst, const TileRef& s
   Q.col = neg ? 63 - lane : lane;
   const int xl = x0 - kH + Q.col;
   const int px = flags & kPeriodicX, mw = flags & kMirrorW, me = flags & kMirrorE;
-  unsigned mx, cx, mt, cl;
+  unsigned mx, cx;
   Q.X8 = (unsigned)map_axis(xl, nx, px, mw, me, mx, cx) * 8u;
   const unsigned pair = (unsigned)(w & 1) ^ mx;  // the pairs 1, 3; 9, 11 (two planes apart); 5, 6; 7, 8
   Q.Xx = Q.X8 + (w < 2 ? pair : 1u - pair) * 2u * Q.P8;
   Q.Xd[0] = Q.X8 + pair * Q.P8;
   Q.Xd[1] = Q.X8 + (1u - pair) * Q.P8;
-  (void)map_axis(neg ? xl + 1 : xl - 1, nx, px, mw, me, mt, cl);
-  Q.up = (int)cl;
+  Q.upcol = __builtin_amdgcn_readfirstlane(neg ? (px || me ? -1 : nx - 1 - x0 + kH) : (px || mw ? -1 : kH - x0));
   Q.own = lane >= kH && lane < kH + kStripW && xl < nx;
   Q.rdx = Q.own ? (in->rdxs ? in->rdxs[xl] : in->rdx) : 0.0;
 }
@@ -311,12 +314,12 @@ __device__ __forceinline__ void quad_xface(const QuadItem& Q, double f, double h
   Lf[4] = lane_shift<kDppShl1>(Lf[3]);
   Lh[4] = lane_shift<kDppShl1>(Lh[3]);
   if constexpr (SOLID) {
-    const int lane = threadIdx.x & 63;
+    // shifted as a scalar mask: five flags per lane, formed from the lane's
+    // number, are kept over the rows in registers that k_stage23 does not have
+    // (33 of them spilled; at most 5 this way)
 #pragma unroll
-    for (int k = 0; k < 5; k++) {
-      const int pl = lane - 3 + k;
-      sld[k] = (pl >= 0 && pl < 64) ? int((solid >> pl) & 1ull) : 0;
-    }
+    for (int k = 0; k < 5; k++)
+      sld[k] = __builtin_amdgcn_inverse_ballot_w64(k < 3 ? solid << (3 - k) : solid >> (k - 3)) ? 1 : 0;
     if (solid) {
       const double a = lane_shift<kDppShr1>(quad_alpha(Q, y));
       if (sld[2]) {
@@ -358,7 +361,7 @@ __device__ __forceinline__ void quad_net_y(const QuadItem& Q, QuadWin& W, unsign
     double ixf, ixh;
     quad_xface<SOLID, W5>(Q, of, oh, xsolid, y, vx, ixf, ixh);
     const double oxf = lane_shift<kDppShl1>(ixf), oxh = lane_shift<kDppShl1>(ixh);
-    if (Q.up) {
+    if (Q.col == again(Q.upcol)) {
       ixf = oxf;
       ixh = oxh;
     }
@@ -376,7 +379,7 @@ __device__ __forceinline__ void quad_net_x(const QuadItem& Q, unsigned long long
   double ixf, ixh;
   quad_xface<SOLID, W5>(Q, f, h, xsolid, y, vx, ixf, ixh);
   const double oxf = lane_shift<kDppShl1>(ixf), oxh = lane_shift<kDppShl1>(ixh);
-  if (Q.up) {
+  if (Q.col == again(Q.upcol)) {
     ixf = oxf;
     ixh = oxh;
   }
