@@ -11,11 +11,14 @@
 // per cell and launch (f2 26 in, f3 26 and dF 24 out; f3 26 and dF 24 in, f2
 // 26 out), 1216 B, where the four launches it replaces move 248 values. The
 // state is written in the last two steps of a sequence (the residual compares
-// them) and where an instance fails. Same values bit for bit as the four
-// launches: the faces are the strip kernels' (March) and the pointwise stages
-// those of lbm_point.hpp. us per step, four launches -> two (the s12 launch
-// that begins a sequence left out): 64^2 Couette 43 -> 39, 256^2 shear wave
-// 60 -> 46, ensemble of 48 1697 -> 1561, 3072^2 Riemann 3943 -> 3287.
+// them) and where an instance fails: the failing step's state goes to the
+// buffer that does not hold the sequence's first state, so that the sequence
+// can be taken again up to the step before (lone_step). Same values bit for
+// bit as the four launches: the faces are the strip kernels' (March) and the
+// pointwise stages those of lbm_point.hpp. us per step, four launches -> two
+// (the s12 launch that begins a sequence left out): 64^2 Couette 43 -> 39,
+// 256^2 shear wave 60 -> 46, ensemble of 48 1697 -> 1561, 3072^2 Riemann
+// 3943 -> 3287.
 //
 // Bounds at 3072^2: the 5.7 GB a launch moves take 1.25 ms at the rate of a
 // large copy (4.6 TB/s); k_stage23 takes 1.74 ms, k_stage31 1.61. Without
@@ -49,6 +52,7 @@ namespace {
 constexpr int kQuadRows = 32;   // most rows of an item
 constexpr int kWriteState = 1;  // k_stage31: write the new state
 constexpr int kNextStages = 2;  // k_stage31: stages 1 and 2 of the next step
+constexpr int kStateBit = 2;    // k_stage31: the buffer of the new state (one bit)
 
 // The instance record through the constant address space: its fields (which no
 // launch of the step changes) come in scalar loads wherever they are used.
@@ -495,7 +499,7 @@ __device__ __forceinline__ void quad_rows(const InstDev& inst, const QuadItem& Q
     cc = fetch(y + 1 < end ? y + 1 : y);
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (STAGE31) {
-      if (what & kWriteState) put(q, Q.in->state[(Q.in->parity0 ^ step) & 1], oc, ro, o, rf, rh);
+      if (what & kWriteState) put(q, Q.in->state[(what >> kStateBit) & 1], oc, ro, o, rf, rh);
       if (!(what & kNextStages)) return;
     } else {
       const Buf dfl = make_buf(again(Q.dfl), 24u * Q.P8);
@@ -634,9 +638,13 @@ __device__ __forceinline__ void quad_launch(const InstDev* __restrict__ insts, c
   const InstDev& in = insts[sr.inst];
   // failures flagged while this launch runs are of its step or the next one:
   // every wavefront sees the same answers here
-  const int fail = *in.fail, now = in.step_base + step;
+  const int fail = __builtin_amdgcn_readfirstlane(*in.fail), now = in.step_base + step;
   if (fail < now) return;
-  if (fail == now) what |= kWriteState;  // the failing step's state stays
+  if constexpr (STAGE31) {
+    const bool stays = fail == now && (what & kNextStages);  // an inner step fails: its state stays
+    what |= ((in.parity0 ^ (stays ? 1 : step)) & 1) << kStateBit;
+    if (stays) what |= kWriteState;
+  }
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   for (int k = threadIdx.x; k < (sr.flags >> kStripRowsBit) + 2 * kH; k += 256)
     X.rows[k] = row_entry(*(InstC*)&in, sr.ty - kH + k);

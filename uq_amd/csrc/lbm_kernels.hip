@@ -1718,12 +1718,14 @@ int totals_scratch_doubles() { return 4 * kRedBlocks + 4; }
 // ---------------------------------------------------------------------------
 // Residual of the last step (reference runOne, cpuLBM.cpp:2322-2331): RMS
 // over all nx*ny cells of the change of T between the previous state (the
-// other state buffer, which a step leaves untouched) and the current one.
+// other state buffer) and the current one: a step of four launches leaves the
+// previous state untouched, and the fused step writes both in the last two
+// steps of a sequence (for one that fails before: lone_step).
 // Deterministic two-level FP64 reduction: one partial sum per grid row
 // (rows[y], wavefront shuffles within the row's block), then one block adds
 // the rows in a fixed order and writes sqrt(sum / (nx ny)) to *out. Launched
 // behind a sequence of `nsteps` steps, with the record it began with: where
-// the instance failed inside the sequence, the last step is the failing one.
+// the instance failed in the sequence, the last step is the failing one.
 // ---------------------------------------------------------------------------
 template <typename TS>
 __device__ __forceinline__ double cell_T(const InstDev& in, int k, long long o) {

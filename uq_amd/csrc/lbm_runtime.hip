@@ -1140,7 +1140,8 @@ int uqlbm::run_group(const std::vector<Solver*>& members, InstDev* table_dev, co
     Solver* s = members[k];
     if (fail_step[k] != INT_MAX) {
       const int taken = std::max(0, fail_step[k] - s->step);
-      s->cur ^= taken & 1;
+      // the fused step leaves the state of a failing inner step beside the sequence's first state
+      s->cur ^= fused && taken < n ? taken > 0 : taken & 1;
       s->step += taken;
       s->failed = true;
       status = LBM_FAILED;
@@ -1150,6 +1151,30 @@ int uqlbm::run_group(const std::vector<Solver*>& members, InstDev* table_dev, co
     }
   }
   return status;
+}
+
+// n steps of a lone solver, as run_group. A residual compares the states of the
+// last two steps taken; where the fused step fails at an inner step of the
+// sequence, the state before that step was never written, and the sequence,
+// whose first state is still there, is taken again with its end there: up to
+// the step before (which the last steps of a sequence write), then the failing
+// step alone. The same values either way, so only a failing call pays for it.
+static int lone_step(Solver& s, const StepLaunch& L, int n, GraphCache* graphs, bool timed, bool resid,
+                     StepResult* result, double* rows) {
+  const std::vector<Solver*> one{&s};
+  const int cur = s.cur, step = s.step;
+  if (!resid) rows = nullptr;
+  const int st = run_group(one, s.inst_dev, L, s.precision, s.stream, n, graphs, s.fails_dev, timed, result, rows);
+  const int taken = s.step - step;
+  if (st != LBM_FAILED || !resid || !L.fused || taken <= 1 || taken >= n) return st;
+  static const int none = INT_MAX;
+  HIP_TRY(hipMemcpyAsync(s.fail, &none, sizeof(int), hipMemcpyHostToDevice, s.stream));
+  s.cur = cur;
+  s.step = step;
+  s.failed = false;
+  const int before = run_group(one, s.inst_dev, L, s.precision, s.stream, taken - 1, graphs, s.fails_dev, false, result);
+  if (before != LBM_OK) return before;
+  return run_group(one, s.inst_dev, L, s.precision, s.stream, 1, graphs, s.fails_dev, false, result, rows);
 }
 
 // Residual of the solver's last step on the device (cpuLBM.cpp:2322-2331),
@@ -1182,9 +1207,7 @@ extern "C" int lbm_step(lbm_solver* h, int32_t nsteps, int32_t want_residual, do
     (void)hipGetLastError();
   }
   if (resid && !s.resid_dev) HIP_TRY(solver_alloc(s, (void**)&s.resid_dev, ((size_t)s.ny + 1) * sizeof(double)));
-  std::vector<Solver*> one{&s};
-  const int st = run_group(one, s.inst_dev, L, s.precision, s.stream, nsteps, s.graphs.get(), s.fails_dev, true,
-                           s.result, resid ? s.resid_dev : nullptr);
+  const int st = lone_step(s, L, nsteps, s.graphs.get(), true, resid, s.result, s.resid_dev);
   const int st2 = upload_inst(s);
   if (st < 0) return st;
   if (st2 != LBM_OK) return st2;
@@ -1251,8 +1274,7 @@ extern "C" int lbm_step_noalloc(lbm_solver* h, int32_t nsteps, int32_t want_resi
   launch_strips_of(L, s.strips_dev, s.nstrips, s.nmstrips, s.fused, s.strip_blocks, 0, s.ntiles);
   L.eq_kinds = s.precision == LBM_PREC_FP64 ? 1 : (s.eq32 ? 2 : 1);
   prepare_launch(s.precision == LBM_PREC_FP64);
-  std::vector<Solver*> one{&s};
-  const int st = run_group(one, s.inst_dev, L, s.precision, s.stream, nsteps, nullptr, s.fails_dev, false);
+  const int st = lone_step(s, L, nsteps, nullptr, false, want_residual && residual_out, nullptr, nullptr);
   const int st2 = upload_inst(s);
   if (st < 0) return st;
   if (st2 != LBM_OK) return st2;
