@@ -1,0 +1,23 @@
+"""The FP64 face reconstruction across jumps, and the reciprocal of the FP64
+kernels, on the host against long double: tests/weno_check.cpp, built against
+the header the kernels include."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+
+
+def test_reconstruction_across_jumps(tmp_path):
+    if not os.path.exists(HIPCC):
+        pytest.skip("hipcc not available")
+    exe = tmp_path / "weno_check"
+    build = subprocess.run([HIPCC, "-std=c++17", "-O2", "--offload-arch=gfx950", "-I", os.path.join(ROOT, "include"),
+                            os.path.join(ROOT, "tests", "weno_check.cpp"), "-o", str(exe)],
+                           capture_output=True, text=True, timeout=600)
+    assert build.returncode == 0, build.stderr[-2000:]
+    run = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
+    print(run.stdout)
+    assert run.returncode == 0, run.stdout

@@ -18,20 +18,6 @@ __host__ __device__ constexpr int quad_x(int w) { return w == 0 ? 1 : w == 1 ? 3
 __host__ __device__ constexpr int quad_y(int w) { return w == 0 ? 2 : w == 1 ? 10 : w == 2 ? 4 : 12; }
 __host__ __device__ constexpr int quad_d(int w) { return 5 + w; }
 
-// 1/x of a normal number away from the range limits (densities, one plus a
-// relaxation ratio): the hardware reciprocal with two Newton-Raphson steps,
-// within one rounding of the quotient in five operations (a division takes
-// eleven, for the range scaling that is not needed here).
-__host__ __device__ __forceinline__ double recip(double x) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  double r = __builtin_amdgcn_rcp(x);
-  r = fused(fused(-x, r, 1.0), r, r);
-  return fused(fused(-x, r, 1.0), r, r);
-#else
-  return 1.0 / x;
-#endif
-}
-
 // Mass, x and y momentum (in units of c) and energy.
 struct Sums {
   double m, px, py, e;
