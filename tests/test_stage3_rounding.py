@@ -1,0 +1,22 @@
+"""Rounding of stage 3 of FP64 storage, on the host: no larger than that of the
+reference's formulas evaluated from the state, tests/stage3_check.cpp."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+
+
+def test_no_further_from_the_stages_than_from_the_state(tmp_path):
+    if not os.path.exists(HIPCC):
+        pytest.skip("hipcc not available")
+    exe = tmp_path / "stage3_check"
+    build = subprocess.run([HIPCC, "-std=c++17", "-O2", "--offload-arch=gfx950", "-I", os.path.join(ROOT, "include"),
+                            os.path.join(ROOT, "tests", "stage3_check.cpp"), "-o", str(exe)],
+                           capture_output=True, text=True, timeout=600)
+    assert build.returncode == 0, build.stderr[-2000:]
+    run = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
+    print(run.stdout)
+    assert run.returncode == 0, run.stdout
