@@ -22,7 +22,7 @@ namespace uqlbm {
 
 constexpr int kQ = 13;
 constexpr int kPlanes = 26;
-constexpr int kPointConsts = 18;  // InstDev::kq
+constexpr int kPointConsts = 3;  // InstDev::kq
 
 // Boundary flag bits (reference cpuLBM.h:47-49).
 enum : int {
@@ -69,9 +69,9 @@ struct InstDev {
   double mu, Pr;
   // reciprocals and differences formed once on the host so that the
   // per-cell arithmetic multiplies instead of divides
-  double isRTc, iTc, ibR;  // 1/sqrt(R*Tc), 1/Tc, 1/(b*R)
+  double isRTc, iTc, ibR, iRTc;  // 1/sqrt(R*Tc), 1/Tc, 1/(b*R), 1/(R*Tc)
   double imu, Pr_m1;       // 1/mu, Pr - 1
-  double kq[kPointConsts];  // coefficients of the nested equilibria (point_consts)
+  double kq[kPointConsts];  // constants of the gas (point_consts)
   // viscosity law: 0 constant mu; 1 VHS mu_ref (T/T_ref)^vexp; 2 Sutherland
   // mu_ref (T/T_ref)^1.5 (T_ref + vS)/(T + vS)
   int visc_model;

@@ -162,17 +162,15 @@ __device__ __forceinline__ Quad make_quad(int w) {
 }
 
 // Equilibria of a wavefront's x and y direction (eq_point's arguments).
-template <typename KQ>
-__device__ __forceinline__ void quad_eq_x(const Quad& q, const KQ& kq, const PointEq& e, double& fe, double& he) {
+__device__ __forceinline__ void quad_eq_x(const Quad& q, const PointEq& e, double& fe, double& he) {
   const double a = q.sx * e.u;
-  if (q.w < 2) eq_axis(kq, e, a, e.u2, e.v2, fe, he);
-  else eq_axis2(kq, e, a, e.u2, e.v2, fe, he);
+  if (q.w < 2) eq_axis(e, a, e.v, fe, he);
+  else eq_axis2(e, a, fe, he);
 }
-template <typename KQ>
-__device__ __forceinline__ void quad_eq_y(const Quad& q, const KQ& kq, const PointEq& e, double& fe, double& he) {
+__device__ __forceinline__ void quad_eq_y(const Quad& q, const PointEq& e, double& fe, double& he) {
   const double b = q.sy * e.v;
-  if (q.w & 1) eq_axis2(kq, e, b, e.v2, e.u2, fe, he);
-  else eq_axis(kq, e, b, e.v2, e.u2, fe, he);
+  if (q.w & 1) eq_axis2(e, b, fe, he);
+  else eq_axis(e, b, e.u, fe, he);
 }
 
 // A work item: the instance's arrays, offsets and edge rules, and the lane's
@@ -539,20 +537,20 @@ __device__ __forceinline__ void quad_rows(const InstDev& inst, const QuadItem& Q
       const Relax12 R = make_relax12(k, m);
       __builtin_amdgcn_sched_barrier(0);
       double fe, he, f2, h2;
-      quad_eq_x(qe, k.kq, e, fe, he);
+      quad_eq_x(qe, e, fe, he);
       point_s12(R, e, q.exx, 0.0, o[0], o[1], fe, he, f2, h2);
       mass = fe;
       keep(q.Ix, f2, h2);
-      quad_eq_y(qe, k.kq, e, fe, he);
+      quad_eq_y(qe, e, fe, he);
       point_s12(R, e, 0.0, q.eyy, o[2], o[3], fe, he, f2, h2);
       mass = mass + fe;
       keep(q.Iy, f2, h2);
-      eq_diag(k.kq, e, q.sx * e.u, q.sy * e.v, e.u2, e.v2, fe, he);
+      eq_diag(e, q.sx * e.u, q.sy * e.v, fe, he);
       point_s12(R, e, q.sx, q.sy, o[4], o[5], fe, he, f2, h2);
       mass = mass + fe;
       keep(q.Id, f2, h2);
       if (w == 0) {
-        eq_rest(k.kq, e, fe, he);
+        eq_rest(e, fe, he);
         point_s12(R, e, 0.0, 0.0, rf, rh, fe, he, f2, h2);
         fm0 = fe;
         keep(0, f2, h2);
@@ -566,24 +564,24 @@ __device__ __forceinline__ void quad_rows(const InstDev& inst, const QuadItem& Q
       prho = m3.rho;
       __builtin_amdgcn_sched_barrier(0);
       double fe, he, fe3, he3, f3, h3;
-      quad_eq_x(qe, k.kq, e, fe, he);
-      quad_eq_x(qe, k.kq, e3, fe3, he3);
+      quad_eq_x(qe, e, fe, he);
+      quad_eq_x(qe, e3, fe3, he3);
       point_s3(R, e, e3, q.exx, 0.0, o[0], o[1], d[0], d[1], fe, he, fe3, he3, f3, h3);
       mass = fe3;
       keep(q.Ix, f3, h3);
-      quad_eq_y(qe, k.kq, e, fe, he);
-      quad_eq_y(qe, k.kq, e3, fe3, he3);
+      quad_eq_y(qe, e, fe, he);
+      quad_eq_y(qe, e3, fe3, he3);
       point_s3(R, e, e3, 0.0, q.eyy, o[2], o[3], d[2], d[3], fe, he, fe3, he3, f3, h3);
       mass = mass + fe3;
       keep(q.Iy, f3, h3);
-      eq_diag(k.kq, e, q.sx * e.u, q.sy * e.v, e.u2, e.v2, fe, he);
-      eq_diag(k.kq, e3, q.sx * e3.u, q.sy * e3.v, e3.u2, e3.v2, fe3, he3);
+      eq_diag(e, q.sx * e.u, q.sy * e.v, fe, he);
+      eq_diag(e3, q.sx * e3.u, q.sy * e3.v, fe3, he3);
       point_s3(R, e, e3, q.sx, q.sy, o[4], o[5], d[4], d[5], fe, he, fe3, he3, f3, h3);
       mass = mass + fe3;
       keep(q.Id, f3, h3);
       if (w == 0) {
-        eq_rest(k.kq, e, fe, he);
-        eq_rest(k.kq, e3, fe3, he3);
+        eq_rest(e, fe, he);
+        eq_rest(e3, fe3, he3);
         point_s3(R, e, e3, 0.0, 0.0, rf, rh, 0.0, 0.0, fe, he, fe3, he3, f3, h3);
         fm0 = fe3;
         keep(0, f3, h3);

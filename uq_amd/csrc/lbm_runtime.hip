@@ -519,6 +519,7 @@ static void fill_inst(const Solver& s, InstDev& d) {
   d.isRTc = 1.0 / d.sRTc;
   d.iTc = 1.0 / d.Tc;
   d.ibR = 1.0 / d.bR;
+  d.iRTc = 1.0 / d.RTc;
   d.imu = 1.0 / d.mu;
   d.Pr_m1 = d.Pr - 1.0;
   point_consts(s.K, d.kq);
