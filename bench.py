@@ -101,7 +101,8 @@ def batched_leg(members, precision: str, steps: int, warmup: int, timing_steps: 
     if tune_steps:
         shape, ms = b.autotune(tune_steps)
         tune = {"flux_tile_shape": shape, "tile_dims": list(lbm.flux_shape_dims(shape)),
-                "ms_per_step_by_shape": [round(m, 3) for m in ms]}
+                "ms_per_step_by_shape": [round(m, 3) for m in ms],
+                "tile_kernels": len(set(ms)) > 1}  # false: all members on strips, one time for every shape
     if warmup:
         b.step(warmup)
     t0 = time.perf_counter()

@@ -249,8 +249,11 @@ typedef struct lbm_timing {
  * as the default of solvers, batches and servers created afterwards with
  * the batch's precision, restores the members' states (tuning changes no
  * result) and reports the shape and each shape's milliseconds per step
- * (ms_per_step_out: LBM_FLUX_SHAPES entries, may be NULL). Results are the
- * same for every shape. No counterpart in the reference (its stencil loops
+ * (ms_per_step_out: LBM_FLUX_SHAPES entries, may be NULL). A batch that runs
+ * no tile kernel (lbm_set_strips) is timed once; it keeps its shape, the
+ * default stays, and every shape is given that time. Results are the
+ * same for every shape (within rounding where thin solids need the reference's
+ * physical addressing, which is taken tile by tile). No counterpart in the reference (its stencil loops
  * are per cell).
  */
 #define LBM_FLUX_SHAPES 5

@@ -1598,7 +1598,10 @@ extern "C" int lbm_flux_shape_dims(int32_t shape, int32_t* w, int32_t* h) {
 // the lowest-numbered shape within kTuneTie of the fastest (shapes that close
 // trade places from run to run on timing noise alone; the tie-break makes the
 // choice repeatable), and restores every member's state, step count and
-// failure flag, so tuning leaves the solution untouched.
+// failure flag, so tuning leaves the solution untouched. A batch whose members
+// are all on strips launches the same kernels whatever the shape: it is timed
+// once, and keeps its shape and the default (five timings of one sequence
+// would choose between them by noise).
 static constexpr double kTuneTie = 0.005;
 extern "C" int lbm_batch_autotune(lbm_batch* hb, int32_t steps, int32_t* shape_out, double* ms_per_step_out) {
   if (!hb || steps < 1) return fail_with(LBM_ERR_ARG, "bad autotune arguments");
@@ -1631,9 +1634,15 @@ extern "C" int lbm_batch_autotune(lbm_batch* hb, int32_t steps, int32_t* shape_o
     saved[k].failed = s.failed;
   }
   HIP_TRY(hipStreamSynchronize(b.stream));
+  const bool tiles = !strips_enabled() || b.tiles_rest > 0;
   double ms_of[kFluxShapes];
   for (int shape = 0; shape < kFluxShapes; shape++) {
-    int st = batch_set_shape(b, shape);
+    if (!tiles && shape > 0) {
+      ms_of[shape] = ms_of[0];
+      if (ms_per_step_out) ms_per_step_out[shape] = ms_of[0];
+      continue;
+    }
+    int st = tiles ? batch_set_shape(b, shape) : LBM_OK;
     if (st == LBM_OK) st = batch_step(b, 1);
     if (st == LBM_OK) st = batch_step(b, steps);
     if (st < 0) {
@@ -1648,6 +1657,7 @@ extern "C" int lbm_batch_autotune(lbm_batch* hb, int32_t steps, int32_t* shape_o
   for (int shape = 1; shape < kFluxShapes; shape++) fastest = std::min(fastest, ms_of[shape]);
   int best_shape = 0;
   while (ms_of[best_shape] > fastest * (1.0 + kTuneTie)) best_shape++;
+  if (!tiles) best_shape = b.flux_shape;
   for (size_t k = 0; k < b.members.size(); k++) {
     Solver& s = *b.members[k];
     const size_t bytes = (size_t)s.pitch * s.ny * kPlanes * es;
@@ -1668,9 +1678,11 @@ extern "C" int lbm_batch_autotune(lbm_batch* hb, int32_t steps, int32_t* shape_o
   }
   HIP_TRY(hipStreamSynchronize(b.stream));
   release();
-  const int st = batch_set_shape(b, best_shape);
-  if (st != LBM_OK) return st;
-  g_flux_shape[b.precision == LBM_PREC_FP64 ? 0 : 1] = best_shape;
+  if (tiles) {
+    const int st = batch_set_shape(b, best_shape);
+    if (st != LBM_OK) return st;
+    g_flux_shape[b.precision == LBM_PREC_FP64 ? 0 : 1] = best_shape;
+  }
   if (shape_out) *shape_out = best_shape;
   return LBM_OK;
 }

@@ -250,7 +250,8 @@ class Batch:
 
     def autotune(self, steps: int = 5) -> tuple[int, list[float]]:
         """Pick the fastest flux tile shape for this batch (the lowest-numbered
-        shape within 0.5 % of the fastest; state unchanged);
+        shape within 0.5 % of the fastest; state unchanged). A batch that runs
+        no tile kernel is timed once and keeps its shape and the default;
         returns the shape and each shape's milliseconds per step."""
         shape = C.c_int32(0)
         ms = np.zeros(FLUX_SHAPES)
