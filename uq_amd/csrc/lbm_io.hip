@@ -6,9 +6,9 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <exception>
 #include <memory>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -210,7 +210,11 @@ struct SlotPool {
   std::vector<Slot> free;
 };
 SlotPool& slot_pool() {
-  static SlotPool* p = new SlotPool();  // never destroyed: outlives every solver
+  static SlotPool* p = [] {
+    SlotPool* q = new SlotPool();  // never destroyed: outlives every solver
+    q->free.reserve(kSlotsKept);   // ~SlotUse gives slots back without an allocation
+    return q;
+  }();
   return *p;
 }
 
@@ -337,7 +341,7 @@ hipError_t staged_copy(char* dev, const std::vector<HostSeg>& segs, bool out, hi
         (void)hipSetDevice(device);
         pieces(w, workers, true);
       });
-    } catch (const std::system_error&) {
+    } catch (const std::exception&) {  // std::system_error, std::bad_alloc
       here.push_back(w);
     }
   }
