@@ -16,24 +16,24 @@
 // can be taken again up to the step before (lone_step). Same values bit for
 // bit as the four launches: the faces are the strip kernels' (March) and the
 // pointwise stages those of lbm_point.hpp. us per step, four launches -> two
-// (the s12 launch that begins a sequence left out): 64^2 Couette 43 -> 39,
-// 256^2 shear wave 60 -> 46, ensemble of 48 1697 -> 1561, 3072^2 Riemann
-// 3943 -> 3287.
+// (with the s12 launch that begins a sequence): 64^2 Couette 41 -> 29, 256^2
+// shear wave 48 -> 40, 512^2 129 -> 98, ensemble of 48 1855 -> 1550, 3072^2
+// Riemann 3865 -> 3165.
 //
 // Bounds at 3072^2: the 5.7 GB a launch moves take 1.25 ms at the rate of a
-// large copy (4.6 TB/s); k_stage23 takes 1.74 ms, k_stage31 1.61. Without
-// their loads or without their stores they take 1.3 and 1.0 ms, and the FP64
-// units are busy for two thirds of it: neither alone bounds them, but the
-// three wavefronts per SIMD that the registers leave room for, which wait for
-// memory at the same places of a row.
+// large copy (4.6 TB/s); k_stage23 takes 1.70 ms, k_stage31 1.45. Without
+// their loads or without their stores they took 1.3 and 1.0 ms (of 1.74 and
+// 1.61 then), with the FP64 units busy for two thirds of it: neither alone
+// bounds them, but the three wavefronts per SIMD that the registers leave room
+// for, which wait for memory at the same places of a row.
 //
 // One workgroup per work item (a strip of kStripW columns by some rows); its
 // four wavefronts march the rows in step, each with one direction along x, one
 // along y and one diagonal (quad_x, quad_y, quad_d): four net faces for f and h
 // each, equal work, and a quarter of the cell's equilibria, so that the
 // stencil windows (three directions) and the pointwise temporaries fit the
-// registers of three wavefronts per SIMD (3072^2 with two: 3378 us, three:
-// 3266). Wavefronts whose x direction is negative take the columns in reverse
+// registers of three wavefronts per SIMD (3072^2, when first built: with two
+// 3378 us, three 3266). Wavefronts whose x direction is negative take the columns in reverse
 // lane order, in which the direction is positive: one x sign in the code. Per
 // row the wavefronts exchange their parts of the cell's sums through LDS (one
 // barrier; two buffers in turn, so that a part is overwritten only after every
@@ -136,10 +136,12 @@ __device__ __forceinline__ T again(T v) {
   return v;
 }
 
+// quad_x, quad_y of a wavefront, four bits each.
+constexpr int kDirX = quad_x(0) | quad_x(1) << 4 | quad_x(2) << 8 | quad_x(3) << 12;
+constexpr int kDirY = quad_y(0) | quad_y(1) << 4 | quad_y(2) << 8 | quad_y(3) << 12;
+__device__ __forceinline__ int dir_x(int w) { return (kDirX >> (4 * w)) & 15; }
+__device__ __forceinline__ int dir_y(int w) { return (kDirY >> (4 * w)) & 15; }
 // A wavefront's directions: signs and lattice velocities.
-// quad_x, quad_y of a wavefront (1, 3, 11, 9 and 2, 10, 4, 12)
-__device__ __forceinline__ int dir_x(int w) { return (0x9B31 >> (4 * w)) & 15; }
-__device__ __forceinline__ int dir_y(int w) { return (0xC4A2 >> (4 * w)) & 15; }
 struct Quad {
   int w, Ix, Iy, Id;
   double sx, sy;    // signs

@@ -667,21 +667,26 @@ bool uqlbm::far_fp64(int blocks) { return g_strips == 2 || blocks >= kFarMinBloc
 // (n + 1) * (rows + 2), with n the workgroups of the busiest CU, `blocks` of
 // them per item (three of k_strip's directions, one of four wavefronts). A
 // row of the march takes the longer the more workgroups share the CU, but a
-// lone one cannot fill it (stage23: 3.0, 4.5, 5.9 and 7.8 us per row with one
-// to four), and the window that an item fills costs about two rows. Whole
-// numbers of workgroups per CU matter as much as the length: 512^2 at 6 rows
-// has 774 items, four on some CUs, at 7 rows 666, three: 122 and 107 us.
-// us per step (FP64) or launch at 1 / 2 / 4 / 8 / 16 / 32 rows, and at the rule's:
-//   64^2 Couette, step           31 / 40 / 54 / 67 / 110 / 199       1: 31
-//   256^2 shear, step            47 / 46 / 53 / 64 / 108 / 197       3: 45
-//   512^2 shear, step            126 / 104 / 107 / 118 / 158 / 199   5: 107
-//   ensemble of 48, step         2283 / 1815 / 1549 / 1421 / 1431 / 1514   12: 1396 (1417 with the s12 launch)
+// lone one cannot fill it (stage23, items of 32 rows: 3.9, 6.3, 8.3 and 10.9 us
+// per row with one to four), and the window that an item fills costs about two
+// rows. Whole numbers of workgroups per CU matter as much as the length: 512^2 at
+// 6 rows has 774 items, four on some CUs, at 7 rows 666, three: 110 and 99 us.
+// us per step (FP64; its share of the launch that begins a sequence included) or
+// launch at 1 / 2 / 4 / 8 / 16 / 32 rows, and at the rule's:
+//   64^2 Couette, step           29 / 31 / 42 / 63 / 103 / 189       1: 29
+//   256^2 shear, step            39 / 39 / 48 / 56 / 97 / 182        3: 40
+//   512^2 shear, step            112 / 95 / 97 / 108 / 147 / 185     5: 98
+//   ensemble of 48, step         2305 / 1930 / 1678 / 1555 / 1554 / 1639   12: 1550
+//   3072^2 Riemann, step         4869 / 4084 / 3438 / 3174 / 3107 / 3165   32: 3165
 //   512^2, FP32 k_strip          62 / 44 / 36 / 33 / 35 / 49         8: 33
 //   1100^2, FP32 k_strip_mom     266 / 199 / 164 / 147 / 150 / 150   12: 141
-// (without the launch that begins an FP64 sequence).
+// so the rule is within 3 % of the best of these everywhere; where it is not the
+// best itself (512^2 at 2 rows, 3072^2 at 16) fewer rows do slightly better than
+// the cost of a window suggests.
 // Items near solids have half as many: their rows take about twice as long,
-// and the launch waits for the last of them (301^2 with a block, FP64 step 87
-// us with all rows, 67 with half, 67 with a third; FP32 storage 110, 94, 94).
+// and the launch waits for the last of them (301^2 with a block, FP64 step 79
+// us with all rows, 64 with half, 64 with a third; FP32 storage 110, 91, 93).
+// kCus: the compute units of an MI355X.
 static constexpr int kStripRows = 32, kCus = 256;
 static int solid_rows(int rows) { return (rows + 1) / 2; }
 static int strip_rows(const std::vector<Solver*>& members, int blocks) {
@@ -704,8 +709,8 @@ static int strip_rows(const std::vector<Solver*>& members, int blocks) {
 // The fused step takes FP64 RK3 groups whose members all have strips and
 // arrays within the 32-bit offsets of its buffer accesses (19 million cells);
 // the others keep four launches a step. Not a matter of size otherwise: it is
-// the faster one from 64^2 (39 against 43 us per step) over an ensemble of 48
-// (1561, 1697) to 3072^2 (3287, 3943).
+// the faster one from 64^2 (29 against 41 us per step) over an ensemble of 48
+// (1550, 1855) to 3072^2 (3165, 3865).
 static constexpr unsigned long long kFusedMaxBytes = 0xF0000000ull;
 static bool fused_instance(const Solver& s) {
   return s.precision == LBM_PREC_FP64 && s.p.rk_method == 1 && s.strip_cols > 0 &&

@@ -39,7 +39,6 @@ struct PropRow {
   int type;
 };
 
-// One solver instance: the deck, its derived constants and its device state.
 // What a step call returns to the host, written by the last kernels of its
 // sequence into pinned memory.
 struct StepResult {
@@ -48,6 +47,7 @@ struct StepResult {
   int fail;              // as InstDev::fail
 };
 
+// One solver instance: the deck, its derived constants and its device state.
 struct Solver {
   lbm_params p{};
   int nx = 0, ny = 0, pitch = 0;
@@ -203,10 +203,11 @@ hipError_t solver_alloc(Solver& s, void** p, size_t bytes);
 bool strips_enabled();
 bool far_fp64(int blocks);
 // Strip items of a launch group (member k's with instance index k): `items`
-// holds those of k_strip and then (FP32 storage) those of k_strip_mom.
+// holds those of k_strip and then those of four wavefronts each (k_strip_mom of
+// FP32 storage, the fused step of FP64).
 struct StripLists {
   std::vector<TileRef> items;
-  int n = 0, nmom = 0;  // items of k_strip, of k_strip_mom
+  int n = 0, nmom = 0;  // items of the two kinds
   int blocks = 0;       // the group's 32-row strip items
   int tiles_rest = 0;   // flux tiles of shape `shape` of the members not on strips
   bool fused = false;   // the members take the fused step

@@ -2,6 +2,7 @@
 // kernel of the D2Q13 thermal FD-LBM, with their launchers.
 #include <type_traits>
 
+#include "lbm_point.hpp"
 #include "lbm_stencil.hpp"
 
 namespace uqlbm {

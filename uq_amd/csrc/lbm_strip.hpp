@@ -590,7 +590,10 @@ struct MomRows {
 
 // Wavefront w: directions c_mom_dir[w] (x, y, diagonal), all of x sign
 // (w == 0 || w == 3) and y sign (w < 2).
-static __constant__ int c_mom_dir[4][3] = {{1, 2, 5}, {3, 10, 6}, {11, 4, 7}, {9, 12, 8}};
+static __constant__ int c_mom_dir[4][3] = {{quad_x(0), quad_y(0), quad_d(0)},
+                                           {quad_x(1), quad_y(1), quad_d(1)},
+                                           {quad_x(2), quad_y(2), quad_d(2)},
+                                           {quad_x(3), quad_y(3), quad_d(3)}};
 
 // Moment k (0 mass, 1 and 2 x and y momentum, 3 energy) of a row's net fluxes.
 template <typename TC>
