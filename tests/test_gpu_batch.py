@@ -3,9 +3,10 @@
 Per-instance arithmetic does not depend on the batch: every member of a
 batch, and every request served in a mix, must equal the same solve run
 alone bit for bit — also when the group runs its flux stages on the strip
-kernels and the lone run on the tile kernels (lbm_set_strips 2 and 0; the
-default rule gives these small groups tiles), a group that mixes strip
-instances with tile instances (the plate needs the physical path).
+kernels and the lone run on the tile kernels (lbm_set_strips 2 and 0).
+(Groups that mix strip instances with tile instances, which need the
+reference's physical addressing: tests/test_gpu_geometry.py,
+tests/test_gpu_tile_shapes.py.)
 """
 import numpy as np
 import pytest

@@ -1,7 +1,9 @@
 """Flux tile shapes and the autotuner. Every face flux and net flux is the
 same arithmetic whatever the tiling, so all shapes give bitwise identical
 states (and match the oracle); the autotuner leaves the solution untouched
-and the tuned batch continues exactly as an untuned one."""
+and the tuned batch continues exactly as an untuned one. (These decks run on
+strips by default, whatever the shape; with the tile kernels:
+tests/test_gpu_tile_shapes.py.)"""
 import numpy as np
 import pytest
 

@@ -1,9 +1,10 @@
 """Work items of the strip flux kernels: one wavefront per item and direction,
-the rows per item (2 to 32) chosen by the size of the launch group. The item
+the rows per item (1 to 32) chosen by the size of the launch group. The item
 edges (rows per item, the last partial strip and item, items of one row next
 to a solid, grids of fewer items than XCDs) must not show: strips (the
 default) equal the tile kernels bit for bit, and a member of a large batch,
-whose items are longer, equals its lone run."""
+whose items are longer, equals its lone run. (Items of up to 32 rows:
+tests/test_gpu_long_items.py.)"""
 import numpy as np
 import pytest
 
@@ -37,8 +38,8 @@ def _run(lbm, case, prec, mode):
         lbm.set_strips(1)
 
 
-# sides: below, at and beyond one strip (58 columns), one item (2 rows at the
-# smallest), the window (7 rows) and the 64 lanes; rows not a multiple of any item
+# sides: below, at and beyond one strip (58 columns), one item (one row at
+# the smallest), the window (7 rows) and the 64 lanes; rows not a multiple of any item
 SIDES = [(5, 6), (58, 9), (59, 33), (64, 64), (117, 65), (175, 130)]
 
 
@@ -58,7 +59,7 @@ def test_items_equal_tiles(gpu_lib, kind, flux, rk, prec):
 
 @pytest.mark.parametrize("prec", ["fp64", "mixed"])
 def test_member_of_a_large_batch_equals_alone(gpu_lib, prec):
-    """The batch's items have 32 rows, the lone solver's two."""
+    """The batch's items have some ten rows, the lone solver's one or two."""
     small = [cases.couette(41, nx=61, steps=8), cases.shear_wave(66, u0=0.1, steps=8)]
     alone = []
     for c in small:

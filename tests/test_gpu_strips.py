@@ -1,7 +1,6 @@
 """Strip flux kernels (one wavefront per 58-column strip of up to 32 rows,
 marched row by row; lbm_set_strips) against the flux tile kernels they
-replace (strips forced on: lbm_set_strips mode 2, since these decks are
-smaller than the launch groups the strips take by default), on decks
+replace (strips in lbm_set_strips mode 2), on decks
 covering every boundary treatment the strips take over:
 doubly periodic (shear wave), periodic with solid walls (Couette, WENO5 and
 NND), clamped edges (Riemann), a north/south mirror with a clamp opposite
@@ -11,8 +10,8 @@ whose sides are no multiple of the strip width or height (taller than one
 row block: the items of a strip column alternate between ascending and
 descending row order, so both orders are compared), instances
 narrower than one strip and shorter than one row block, and mixed
-precision (FP32 storage: the stage-2 flux runs on strips, the
-moment-summing stage-3 flux stays on tiles).
+precision (FP32 storage: k_strip for the stage-2 flux, k_strip_mom for the
+moment-summing stage-3 flux).
 
 The two paths compute every face with the same arithmetic (WENO5, NND,
 solid extrapolation, wall closure) and form the net fluxes and the stage-3
